@@ -14,9 +14,10 @@
  *     every scale, score, coefficient and gradient scalar is fp32;
  *   - per-source arrays (src_v, src_r, ...) are HOST arrays of n device addresses, copied into the kernel
  *     arguments (no device pointer table, no host-to-device copy); n <= LDR_MAX_SOURCES;
- *   - except for the *_any entry points at the end, which take what the others reject: any width d >= 1, rows
- *     aligned to their element size only, up to LDR_ANY_MAX_SOURCES sources, whose addresses come as DEVICE arrays
- *     (n uint64 in device memory, read by the kernels; the caller keeps them until the launch has run);
+ *   - except for the entry points at the end, which take what the others reject, rows aligned to their element size
+ *     only: the *_rows ones any width 8 <= d <= LDR_MAX_WIDTH, and the *_any ones any width d >= 1 and up to
+ *     LDR_ANY_MAX_SOURCES sources, whose addresses come as DEVICE arrays (n uint64 in device memory, read by the
+ *     kernels; the caller keeps them until the launch has run);
  *   - stream is a hipStream_t; nothing synchronizes with the host, nothing allocates device memory;
  *   - the return value is 0, a negative LDR_E_* code (rejected before any launch), or a positive hipError_t
  *     from the launch; ldr_strerror() names it.
@@ -49,7 +50,7 @@ extern "C" {
 
 /* Version of this ABI; bumped on any signature change or change of what an entry point accepts. A caller compares
  * ldr_abi_version() of the library it loaded with the LDR_ABI_VERSION of the header it was compiled with. */
-#define LDR_ABI_VERSION 16
+#define LDR_ABI_VERSION 17
 int ldr_abi_version(void);
 
 /* Human-readable text for a return code of any entry point (static storage). */
@@ -215,8 +216,8 @@ int ldr_blend_sum(const uint64_t* g, int64_t m, float beta, int per_read, void* 
 /* ---- any-shape entry points ----------------------------------------------------------------------------------
  * The same computations for the shapes the entry points above reject -- the reference's kernels mask any width
  * and any source count (BLOCK_D = next_pow2(d), BLOCK_N = next_pow2(n): fused_dattn.py:60-63, 191-194) -- with
- * per-source addresses in device arrays (see the conventions at the top). One wave per token row; they are the
- * general path, not the fast one (the module routes to them only for such shapes). */
+ * per-source addresses in device arrays (see the conventions at the top). They are the general path (the module
+ * routes to them, or to the *_rows ones below, only for such shapes). */
 
 /* ldr_read_fwd (q == NULL: dots holds the stored raw scores) and ldr_read_fwd_online (q != NULL: the scores are
  * formed and stored into dots) for any shape: the same outputs and formulas; a zero query with cbar == c0 gives
@@ -255,6 +256,45 @@ int ldr_read_bwd2_list_any(const uint64_t* dv, int64_t n, int accum, const void*
  * reference leaves these adds to autograd, looped_transformer.py:380-381). */
 int ldr_blend_sum_any(const uint64_t* g, int64_t m, float beta, int per_read, void* out, int64_t n_tok, int64_t d,
                       int dtype, void* stream);
+
+/* ---- unaligned rows ------------------------------------------------------------------------------------------
+ * The *_any computations for up to LDR_MAX_SOURCES sources of any width 8 <= d <= LDR_MAX_WIDTH at element alignment,
+ * with the per-source addresses in HOST arrays, copied into the kernel arguments: no device table, no copy. Other
+ * shapes return LDR_E_SHAPE. Each gives the bits of its *_any counterpart on the same addresses. */
+
+/* The write without scores at any width d >= 1: v_out = round(h - x), r_out its scale, in ldr_rstd_fwd's order for
+ * such rows (the same bits). Replaces _write_stk_kernel (fused_dattn.py:561-585) at the shapes ldr_write_dots does not
+ * take. */
+int ldr_write_rows(const void* h, const void* x, void* v_out, float* r_out, int64_t n_tok, int64_t d, float eps,
+                   int dtype, void* stream);
+
+/* ldr_read_fwd_any with host arrays. */
+int ldr_read_fwd_rows(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const float* q, float* dots,
+                      int64_t dots_stride, const void* base, const void* h0, float beta, const float* cbar,
+                      int64_t cbar_cols, const float* c0, int64_t c0_cols, float lam, float inv_sqrt_d, void* out,
+                      float* tc, float* p, float* next_prior, int64_t n_tok, int64_t d, int dtype, void* stream);
+
+/* The number of partial rows that suits ldr_read_bwd1_rows for (n_tok, d): enough workgroups to fill the GPU with few
+ * tokens, at most ldr_read_bwd1's (0 for a width it does not take or no tokens). */
+int64_t ldr_read_bwd1_rows_parts(int64_t n_tok, int64_t d);
+
+/* ldr_read_bwd1_any with host arrays: the caller chooses the number of partial rows, every one of which is written.
+ * Rows that ldr_read_bwd1 takes run on its kernel, with tiles of as many tokens as dq_parts workgroups need. */
+int ldr_read_bwd1_rows(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const void* g, const float* gt,
+                       const float* p, const float* dots, int64_t dots_stride, const float* tc, const float* cbar,
+                       int64_t cbar_cols, const float* c0, int64_t c0_cols, float lam, float inv_sqrt_d, float* dcbar,
+                       int64_t dcbar_cols, const uint64_t* dr, int dr_accum, float* wz, int64_t wz_stride,
+                       float* dq_part, int64_t dq_parts, int64_t dq_part_stride, void* g_prop, void* g_h0, float beta,
+                       int64_t n_tok, int64_t d, int dtype, void* stream);
+
+/* ldr_dv_assemble_any, ldr_read_bwd2_list_any and ldr_blend_sum_any with host arrays. */
+int ldr_dv_assemble_rows(const uint64_t* g, const uint64_t* wz, const uint64_t* q, int64_t m, const void* v,
+                         const float* r, const float* gr, const void* add, float add_beta, int per_read, void* dv,
+                         void* dv_neg, int64_t n_tok, int64_t d, int dtype, void* stream);
+int ldr_read_bwd2_list_rows(const uint64_t* dv, int64_t n, int accum, const void* g, const float* q, const float* wz,
+                            int64_t wz_stride, int64_t n_tok, int64_t d, int dtype, void* stream);
+int ldr_blend_sum_rows(const uint64_t* g, int64_t m, float beta, int per_read, void* out, int64_t n_tok, int64_t d,
+                       int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -12,7 +12,7 @@ import torch  # noqa: F401  -- first: the library must bind to the HIP runtime t
 
 from . import build as _build
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 F32, BF16, F16 = 0, 1, 2
 MAX_SOURCES = 64
 MAX_WIDTH = 8192
@@ -70,6 +70,21 @@ SIGNATURES = {
     "ldr_read_bwd2_list_any": (_i32, [_c_void_p, _i64, _i32, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i32,
                                       _c_void_p]),
     "ldr_blend_sum_any": (_i32, [_c_void_p, _i64, _f32, _i32, _c_void_p, _i64, _i64, _i32, _c_void_p]),
+    # the unaligned-row entry points: the same with host address arrays
+    "ldr_write_rows": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _f32, _i32, _c_void_p]),
+    "ldr_read_fwd_rows": (_i32, [_u64p, _u64p, _i64, _c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p, _f32,
+                                 _c_void_p, _i64, _c_void_p, _i64, _f32, _f32, _c_void_p, _c_void_p, _c_void_p,
+                                 _c_void_p, _i64, _i64, _i32, _c_void_p]),
+    "ldr_read_bwd1_rows_parts": (_i64, [_i64, _i64]),
+    "ldr_read_bwd1_rows": (_i32, [_u64p, _u64p, _i64, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _c_void_p,
+                                  _c_void_p, _i64, _c_void_p, _i64, _f32, _f32, _c_void_p, _i64, _u64p, _i32,
+                                  _c_void_p, _i64, _c_void_p, _i64, _i64, _c_void_p, _c_void_p, _f32, _i64, _i64,
+                                  _i32, _c_void_p]),
+    "ldr_dv_assemble_rows": (_i32, [_u64p, _u64p, _u64p, _i64, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _f32, _i32,
+                                    _c_void_p, _c_void_p, _i64, _i64, _i32, _c_void_p]),
+    "ldr_read_bwd2_list_rows": (_i32, [_u64p, _i64, _i32, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i32,
+                                       _c_void_p]),
+    "ldr_blend_sum_rows": (_i32, [_u64p, _i64, _f32, _i32, _c_void_p, _i64, _i64, _i32, _c_void_p]),
 }
 
 
@@ -114,3 +129,7 @@ def row_layout(d: int) -> tuple[int, int]:
 
 def bwd1_parts(n_tok: int, d: int) -> int:
     return int(LIB.ldr_read_bwd1_parts(n_tok, d))
+
+
+def bwd1_rows_parts(n_tok: int, d: int) -> int:
+    return int(LIB.ldr_read_bwd1_rows_parts(n_tok, d))

@@ -647,9 +647,7 @@ __global__ __launch_bounds__(WG) void k_rstd_bwd(const T* __restrict__ x, const 
   }
 }
 
-// Rows of any width and alignment (those the vector layout does not take: d not a multiple of 8, above the widest
-// row, or not 16-byte aligned): one wave per row, its lanes striding the row with scalar loads (64 consecutive
-// elements per step, coalesced), the sum reduced in registers.
+// one element at element alignment
 __device__ __forceinline__ float ld1(const bf16_t* p) { return __uint_as_float((uint32_t)*p << 16); }
 __device__ __forceinline__ float ld1(const float* p) { return *p; }
 __device__ __forceinline__ float ld1(const _Float16* p) { return (float)*p; }
@@ -657,18 +655,184 @@ __device__ __forceinline__ void st1(bf16_t* p, float v) { *p = __builtin_bit_cas
 __device__ __forceinline__ void st1(float* p, float v) { *p = v; }
 __device__ __forceinline__ void st1(_Float16* p, float v) { *p = to_f16(v); }
 
+// wave_lds_sync: the lanes of one wave meet around LDS (no barrier: the wave's LDS operations are in order)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// unaligned-row kernels (the *_rows entry points, and *_any at 8 <= d <= LDR_MAX_WIDTH): rows of any width at element
+// alignment, any source count. They compute what the row-layout kernels compute, with two differences in the rows:
+//   * a row of d elements is ceil(d/8) eight-element vectors loaded at element alignment (global loads take any
+//     alignment; one that crosses a cache line costs a second line, not a second instruction); the last vector is
+//     moved back to end with the row, so nothing past a row is read, and its first `skip` elements, which the vector
+//     before it holds too, are masked to zero where they are summed and not stored;
+//   * the per-source scalars of a row sit in dynamic LDS, sized by n, so the count is bounded by LDS alone.
+// What bounds them is the HBM stream of the rows. Before, one lane held one column (2-byte loads, 64 columns per
+// instruction) and backward pass 1 ran one wave on each of n_tok / 64 partial rows. A 12-step training pass of 2049
+// tokens at d = 1001 in bf16: 31.8 -> 2.06 ms (the host's launch rate; 1.04 ms of kernels), per launch backward
+// pass 1 2690 -> 22.6 us (7 sources on average), the read 70-79 -> 23-26, the update gradient 44.6 -> 24.1. A read of
+// 65-72 sources of 4096 x 768 bf16: 746 -> 138 us (3.1 TB/s; two waves per SIMD, a row's online softmax between loads).
+// ---------------------------------------------------------------------------------------------------------------
+typedef unsigned int u32x4_u16 __attribute__((ext_vector_type(4), aligned(2), may_alias));
+typedef unsigned int u32x4_u32 __attribute__((ext_vector_type(4), aligned(4), may_alias));
+
+template <typename T> struct UIO {   // 16-bit elements: one 16-byte vector at 2-byte alignment
+  typedef typename IO<T>::Raw Raw;
+  struct Mask { uint4 m; };
+  static __device__ __forceinline__ Raw put(u32x4 v) { Raw r; r.u = make_uint4(v.x, v.y, v.z, v.w); return r; }
+  static __device__ __forceinline__ Raw raw(const T* p) { return put(*reinterpret_cast<const u32x4_u16*>(p)); }
+  static __device__ __forceinline__ Raw raw_nt(const T* p) {
+    return put(__builtin_nontemporal_load(reinterpret_cast<const u32x4_u16*>(p)));
+  }
+  static __device__ __forceinline__ Mask mask(int skip) {   // zero for the first `skip` elements
+    auto word = [&](int w) -> unsigned {
+      return (2 * w >= skip ? 0xffffu : 0u) | (2 * w + 1 >= skip ? 0xffff0000u : 0u);
+    };
+    return Mask{make_uint4(word(0), word(1), word(2), word(3))};
+  }
+  static __device__ __forceinline__ Raw masked(Raw r, const Mask& m) {
+    r.u.x &= m.m.x; r.u.y &= m.m.y; r.u.z &= m.m.z; r.u.w &= m.m.w;
+    return r;
+  }
+  static __device__ __forceinline__ void store(T* p, const float (&o)[8]) {
+    typedef typename std::conditional<std::is_same<T, bf16_t>::value, Bf16Cvt, F16Cvt>::type Cvt;
+    *reinterpret_cast<u32x4_u16*>(p) = u32x4{Cvt::pack2(o[0], o[1]), Cvt::pack2(o[2], o[3]), Cvt::pack2(o[4], o[5]),
+                                             Cvt::pack2(o[6], o[7])};
+  }
+};
+
+template <> struct UIO<float> {      // fp32 elements: two 16-byte vectors at 4-byte alignment
+  typedef IO<float>::Raw Raw;
+  struct Mask { uint4 a, b; };
+  static __device__ __forceinline__ Raw put(u32x4 a, u32x4 b) {
+    Raw r;
+    r.a = make_float4(__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w));
+    r.b = make_float4(__uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w));
+    return r;
+  }
+  static __device__ __forceinline__ Raw raw(const float* p) {
+    const u32x4_u32* q = reinterpret_cast<const u32x4_u32*>(p);
+    return put(q[0], q[1]);
+  }
+  static __device__ __forceinline__ Raw raw_nt(const float* p) {
+    const u32x4_u32* q = reinterpret_cast<const u32x4_u32*>(p);
+    return put(__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1));
+  }
+  static __device__ __forceinline__ Mask mask(int skip) {
+    auto word = [&](int k) -> unsigned { return k >= skip ? 0xffffffffu : 0u; };
+    return Mask{make_uint4(word(0), word(1), word(2), word(3)), make_uint4(word(4), word(5), word(6), word(7))};
+  }
+  static __device__ __forceinline__ float and_f(float x, unsigned m) { return __uint_as_float(__float_as_uint(x) & m); }
+  static __device__ __forceinline__ Raw masked(Raw r, const Mask& m) {
+    r.a = make_float4(and_f(r.a.x, m.a.x), and_f(r.a.y, m.a.y), and_f(r.a.z, m.a.z), and_f(r.a.w, m.a.w));
+    r.b = make_float4(and_f(r.b.x, m.b.x), and_f(r.b.y, m.b.y), and_f(r.b.z, m.b.z), and_f(r.b.w, m.b.w));
+    return r;
+  }
+  static __device__ __forceinline__ void store(float* p, const float (&o)[8]) {
+    u32x4_u32* q = reinterpret_cast<u32x4_u32*>(p);
+    q[0] = u32x4{__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]), __float_as_uint(o[3])};
+    q[1] = u32x4{__float_as_uint(o[4]), __float_as_uint(o[5]), __float_as_uint(o[6]), __float_as_uint(o[7])};
+  }
+};
+
+// Row geometry at any width d >= 8: vector c of a row covers elements [8c, 8c + 8), the last one [d - 8, d).
+struct URows {
+  int d, d8, tpr, rpw, rs, lr;
+  __device__ __forceinline__ URows(int d_, int tpr_)
+      : d(d_), d8((d_ + 7) >> 3), tpr(tpr_), rpw(WG / tpr_), rs((int)threadIdx.x / tpr_),
+        lr((int)threadIdx.x % tpr_) {}
+  __device__ __forceinline__ int c8(int v) const { return lr + v * tpr; }
+  __device__ __forceinline__ bool act(int v) const { return c8(v) < d8; }
+  __device__ __forceinline__ int off(int v) const { return min(c8(v) * 8, d - 8); }
+  __device__ __forceinline__ int skip(int v) const { return min(c8(v) * 8 - off(v), 8); }   // 8: no vector here
+  template <typename T> __device__ __forceinline__ void store(T* row, int v, const float (&o)[8]) const {
+    const int s = skip(v);
+    if (s == 0) UIO<T>::store(row + off(v), o);
+    else
+#pragma unroll
+      for (int k = 1; k < 8; ++k)
+        if (k >= s) st1(row + off(v) + k, o[k]);
+  }
+  // what the lanes of a row wrote to LDS is read by its other lanes after this (a row of more than 64 lanes spans
+  // waves: then every lane of the workgroup is here)
+  __device__ __forceinline__ void sync() const {
+    if (tpr > 64) __syncthreads();
+    else wave_lds_sync();
+  }
+};
+
+// The scale and the write of rows the vector row layout does not take, one wave per row. row_sumsq is the one
+// summation order of both, so a stacked write and rstd() store the same bits: lane l sums vectors l, l + 64, ... in
+// order (fused multiply-adds), the lanes meet in lanes_reduce. get(off, skip, e) fills the 8 elements of the vector
+// that starts at off, the first `skip` of them zero. Rows shorter than a vector take one element per lane.
+template <typename Get> __device__ __forceinline__ float row_sumsq(int64_t d, int lane, Get get) {
+  float ss = 0.f;
+  for (int64_t c = lane; c < (d + 7) / 8; c += 64) {
+    const int64_t off = min(8 * c, d - 8);
+    float e[8];
+    get(off, (int)(8 * c - off), e);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ss = __builtin_fmaf(e[k], e[k], ss);
+  }
+  return ss;
+}
+
 template <typename T>
 __global__ __launch_bounds__(WG) void k_rstd_fwd_any(const T* __restrict__ x, float* __restrict__ r, int64_t n_tok,
                                                      int64_t d, float eps) {
   const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
   for (int64_t tok = (int64_t)blockIdx.x * (WG / 64) + w; tok < n_tok; tok += (int64_t)gridDim.x * (WG / 64)) {
     const T* row = x + tok * d;
-    float ss = 0.f;
-    for (int64_t k = lane; k < d; k += 64) {
-      const float e = ld1(row + k);
-      ss += e * e;
+    float ss;
+    if (d >= 8) {
+      ss = row_sumsq(d, lane, [&](int64_t off, int skip, float (&e)[8]) {
+        IO<T>::unpack(UIO<T>::masked(UIO<T>::raw(row + off), UIO<T>::mask(skip)), e);
+      });
+    } else {
+      const float e = lane < d ? ld1(row + lane) : 0.f;
+      ss = e * e;
     }
     ss = lanes_reduce(ss, 64, AddOp());   // every lane of the wave is here: the row loop is wave-uniform
+    if (lane == 0) r[tok] = rsqrtf(ss / (float)d + eps);
+  }
+}
+
+// v = round(h - x) and the scale of the rounded row, in one pass (2049 rows of 1001 bf16: 5.3 us; a subtraction and
+// the scale kernel before, 5.0 + 6.6 us)
+template <typename T>
+__global__ __launch_bounds__(WG) void k_write_any(const T* __restrict__ h, const T* __restrict__ x,
+                                                  T* __restrict__ v, float* __restrict__ r, int64_t n_tok, int64_t d,
+                                                  float eps) {
+  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  for (int64_t tok = (int64_t)blockIdx.x * (WG / 64) + w; tok < n_tok; tok += (int64_t)gridDim.x * (WG / 64)) {
+    const int64_t roff = tok * d;
+    float ss;
+    if (d >= 8) {
+      ss = row_sumsq(d, lane, [&](int64_t off, int skip, float (&e)[8]) {
+        float a[8], b[8];
+        IO<T>::unpack(UIO<T>::raw_nt(h + roff + off), a);
+        IO<T>::unpack(UIO<T>::raw(x + roff + off), b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = IO<T>::round(a[k] - b[k]);
+        if (skip == 0) UIO<T>::store(v + roff + off, e);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if (k < skip) e[k] = 0.f;
+          else if (skip > 0) st1(v + roff + off + k, e[k]);
+        }
+      });
+    } else {
+      float e = 0.f;
+      if (lane < d) {
+        e = IO<T>::round(ld1(h + roff + lane) - ld1(x + roff + lane));
+        st1(v + roff + lane, e);
+      }
+      ss = e * e;
+    }
+    ss = lanes_reduce(ss, 64, AddOp());
     if (lane == 0) r[tok] = rsqrtf(ss / (float)d + eps);
   }
 }
@@ -681,7 +845,25 @@ __global__ __launch_bounds__(WG) void k_rstd_bwd_any(const T* __restrict__ x, co
   for (int64_t tok = (int64_t)blockIdx.x * (WG / 64) + w; tok < n_tok; tok += (int64_t)gridDim.x * (WG / 64)) {
     const float rv = r[tok];
     const float c = gr[tok] * (-rv * rv * rv) / (float)d;
-    for (int64_t k = lane; k < d; k += 64) st1(gx + tok * d + k, c * ld1(x + tok * d + k));
+    const T* row = x + tok * d;
+    T* o = gx + tok * d;
+    if (d >= 8) {
+      for (int64_t j = lane; j < (d + 7) / 8; j += 64) {
+        const int64_t off = min(8 * j, d - 8);
+        const int skip = (int)(8 * j - off);
+        float e[8];
+        IO<T>::unpack(UIO<T>::raw(row + off), e);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = c * e[k];
+        if (skip == 0) UIO<T>::store(o + off, e);
+        else
+#pragma unroll
+          for (int k = 1; k < 8; ++k)
+            if (k >= skip) st1(o + off + k, e[k]);
+      }
+    } else if (lane < d) {
+      st1(o + lane, c * ld1(row + lane));
+    }
   }
 }
 
@@ -807,14 +989,6 @@ __global__ __launch_bounds__(WG) void k_write_dots(const T* __restrict__ h, cons
     }
   }
 }
-
-// LDS written by some lanes of a wave and read by others of the same wave: complete the writes, keep the order
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // write step on the matrix cores (bf16 updates): the scores are a (tokens x d) . (d x queries) product. Each fp32
 // query row is held as three bf16 parts q = hi + mid + lo (the split is exact to ~2^-24 relative); the update is
@@ -2604,12 +2778,12 @@ __global__ __launch_bounds__(WG) void k_dv_assemble(AsmTab tab, int m, const T* 
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// any-shape kernels (the *_any entry points): rows of any width d >= 1 at element alignment and up to
+// scalar kernels of the any-shape entry points (*_any): rows narrower than one eight-element vector or wider than a
+// workgroup's lanes hold (d < 8, d > LDR_MAX_WIDTH), which the unaligned-row kernels below do not take. Up to
 // LDR_ANY_MAX_SOURCES sources, whose addresses come from DEVICE arrays. One wave per token row, the row's columns
 // strided over its 64 lanes (each load instruction covers consecutive elements), row sums by the lane reduction
 // above; per-source scalars of the row in LDS. They compute what the row-layout kernels compute (the same formulas,
-// and for the elementwise ones the same order of every rounding), for the shapes those do not take: d not a
-// multiple of 8 or above LDR_MAX_WIDTH, more than LDR_MAX_SOURCES sources, rows not 16-byte aligned.
+// and for the elementwise ones the same order of every rounding).
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int ANY_MAXS = LDR_ANY_MAX_SOURCES;
 constexpr int ANY_WAVES = WG / 64;
@@ -2866,16 +3040,610 @@ __global__ __launch_bounds__(WG) void k_any_bwd2_list(const uint64_t* __restrict
   }
 }
 
-// out = round(sum_j round(beta * g_j)) in table order, or with per_read each addition rounded (k_blend_sum)
-template <typename T>
-__global__ __launch_bounds__(WG) void k_any_blend_sum(const uint64_t* __restrict__ tg, int m, float beta, int per_read,
-                                                      T* __restrict__ out, int64_t n_tok, int64_t d) {
+// Where a kernel finds its per-source addresses: by value in its arguments (up to MAXS), or in device arrays.
+struct ValSrc {
+  SrcTab t;
+  PtrTab d;
+  __device__ __forceinline__ const void* v(int i) const { return t.v[i]; }
+  __device__ __forceinline__ const float* r(int i) const { return t.r[i]; }
+  __device__ __forceinline__ float* dr(int i) const { return static_cast<float*>(d.p[i]); }
+};
+struct DevSrc {
+  const uint64_t *tv, *tr, *td;
+  __device__ __forceinline__ const void* v(int i) const { return reinterpret_cast<const void*>(tv[i]); }
+  __device__ __forceinline__ const float* r(int i) const { return reinterpret_cast<const float*>(tr[i]); }
+  __device__ __forceinline__ float* dr(int i) const { return reinterpret_cast<float*>(td[i]); }
+};
+struct ValAsm {
+  AsmTab t;
+  __device__ __forceinline__ const void* g(int j) const { return t.g[j]; }
+  __device__ __forceinline__ const float* wz(int j) const { return t.wz[j]; }
+  __device__ __forceinline__ const float* q(int j) const { return t.q[j]; }
+};
+struct DevAsm {
+  const uint64_t *tg, *tw, *tq;
+  __device__ __forceinline__ const void* g(int j) const { return reinterpret_cast<const void*>(tg[j]); }
+  __device__ __forceinline__ const float* wz(int j) const { return reinterpret_cast<const float*>(tw[j]); }
+  __device__ __forceinline__ const float* q(int j) const { return reinterpret_cast<const float*>(tq[j]); }
+};
+struct ValPtr {
+  PtrTab t;
+  __device__ __forceinline__ void* p(int i) const { return t.p[i]; }
+};
+struct DevPtr {
+  const uint64_t* tp;
+  __device__ __forceinline__ void* p(int i) const { return reinterpret_cast<void*>(tp[i]); }
+};
+
+// softmax of a row's a[0..n) in LDS, in place, by the row's lanes (its first wave when it spans several; the caller
+// syncs the row around it): p = exp(l - max) / sum. One order for every row and the prior, so equal logits give
+// equal bits.
+__device__ __forceinline__ void row_softmax(float* a, int n, const URows& R) {
+  const int w = R.tpr < 64 ? R.tpr : 64;
+  if (R.lr >= 64) return;   // wave-uniform
+  float mx = -INFINITY;
+  for (int i = R.lr; i < n; i += w) mx = fmaxf(mx, a[i]);
+  mx = lanes_reduce(mx, w, MaxOp());
+  float s = 0.f;
+  for (int i = R.lr; i < n; i += w) {
+    const float e = (a[i] == -INFINITY) ? 0.f : expf(a[i] - mx);
+    a[i] = e;
+    s += e;
+  }
+  s = lanes_reduce(s, w, AddOp());
+  for (int i = R.lr; i < n; i += w) a[i] = a[i] / s;
+}
+
+// sources of a row in flight in the read's ring: 64 bytes per lane or more, within two waves' registers
+template <typename T, int VPT> struct URing {
+  static constexpr int PD = std::is_same<T, float>::value ? (VPT == 1 ? 4 : VPT == 2 ? 2 : 1) : (VPT <= 2 ? 4 : 2);
+};
+
+// The read (k_read_fwd without stored scores q == NULL, k_read_online with): its formulas and summation orders.
+// Dynamic LDS: c0, lc, p0 [n], then per row of the workgroup its logits, fixed weights and scales [n].
+template <typename T, int VPT, bool BLEND, typename TAB>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_rows_read(TAB src, int n, const float* __restrict__ q,
+                                                  float* __restrict__ dots, int64_t dots_stride,
+                                                  const T* __restrict__ base, const T* __restrict__ h0, float beta,
+                                                  Coef cf, float inv, T* __restrict__ out, float* __restrict__ tc,
+                                                  float* __restrict__ prob, float* __restrict__ next_prior,
+                                                  int64_t n_tok, int d, int tpr) {
+  extern __shared__ float dyn[];
+  __shared__ float s_M, red[4];
+  __shared__ int s_qnz;
+  using Raw = typename IO<T>::Raw;
+  constexpr int PD = URing<T, VPT>::PD;
+  const URows R(d, tpr);
+  const int tid = (int)threadIdx.x;
+  float *s_c0 = dyn, *s_lc = dyn + n, *s_p0 = dyn + 2 * n;
+  float *lg = dyn + 3 * n + R.rs * 3 * n, *wt = lg + n, *rsc = wt + n;
+  if (tid == 0) s_qnz = 0;
+  for (int i = tid; i < n; i += WG) {
+#pragma clang fp contract(off)   // the product rounded on its own, as the caller's scaling is
+    const float v = i < cf.c0_cols ? cf.lam * cf.c0[i] : cf.lam;
+    s_c0[i] = v;
+    s_lc[i] = logf(fmaxf(v, 1e-8f));
+    s_p0[i] = s_lc[i];
+    if (next_prior && blockIdx.x == 0) next_prior[i] = v;
+  }
+  __syncthreads();
+  if (tid < 64) row_softmax(s_p0, R.rs == 0 ? n : 0, R);   // by row 0's lanes, in the rows' own order
+  if (tid == WG - 1) {
+    float m = 0.f;
+    for (int i = 0; i < n; ++i) m += s_c0[i];
+    s_M = m;
+  }
+  float qv[VPT][8];
+  typename UIO<T>::Mask mk[VPT];
+  bool nz = false;
+#pragma unroll
+  for (int v = 0; v < VPT; ++v) {
+    mk[v] = UIO<T>::mask(R.skip(v));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float x = q ? q[R.off(v) + k] : 0.f;
+      qv[v][k] = k >= R.skip(v) ? x : 0.f;
+      nz |= qv[v][k] != 0.f;
+    }
+  }
+  if (nz) s_qnz = 1;   // every writer stores the same value
+  __syncthreads();
+  const float M = s_M;
+  const bool qz = s_qnz == 0, online = q != nullptr;   // workgroup-uniform
+  const int64_t groups = (n_tok + R.rpw - 1) / R.rpw;
+  for (int64_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+    const int64_t tok = gi * R.rpw + R.rs;
+    const bool valid = tok < n_tok;
+    const int64_t tk = valid ? tok : n_tok - 1;   // rows past the end recompute the last token, store nothing
+    const int64_t roff = tk * (int64_t)d;
+    auto load_src = [&](int i, Raw (&rw)[VPT]) {
+      const T* p = static_cast<const T*>(src.v(i)) + roff;
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) rw[v] = UIO<T>::raw_nt(p + R.off(v));
+    };
+    Raw buf[PD][VPT];   // a ring of PD sources in flight: source i lives in buf[i % PD]
+#pragma unroll
+    for (int j = 0; j < PD; ++j)
+      if (j < n) load_src(j, buf[j]);
+    float acc[VPT][8];
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) IO<T>::unpack(UIO<T>::raw(base + roff + R.off(v)), acc[v]);
+    for (int i = R.lr; i < n; i += tpr) {   // the row's per-source scalars, spread over its lanes
+      const float cb = coef_cbar(cf, tk, i), rv = src.r(i)[tk];
+      if (online) {
+        wt[i] = qz ? s_c0[i] - cb : (s_c0[i] - cb) - M * s_p0[i];
+        rsc[i] = rv;
+      } else {
+        wt[i] = cb;
+        lg[i] = dots[(int64_t)i * dots_stride + tk] * rv * inv + s_lc[i];
+      }
+    }
+    R.sync();
+    if (!online) {   // stored scores: the softmax first, then one fixed weight per source
+      row_softmax(lg, n, R);
+      R.sync();
+      for (int i = R.lr; i < n; i += tpr) {
+        const float tcv = s_c0[i] + M * (lg[i] - s_p0[i]);
+        if (valid) {
+          tc[tok * n + i] = tcv;
+          if (prob) prob[tok * n + i] = lg[i];
+        }
+        wt[i] = tcv - wt[i];
+      }
+      R.sync();
+    }
+    if (BLEND) {   // iteration end: base = proposal + beta (h0 - proposal), each step rounded as the caller's ops
 #pragma clang fp contract(off)
-  const int64_t total = n_tok * d;
-  for (int64_t e = (int64_t)blockIdx.x * WG + threadIdx.x; e < total; e += (int64_t)gridDim.x * WG) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) {
+        float hv[8];
+        IO<T>::unpack(UIO<T>::raw(h0 + roff + R.off(v)), hv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          acc[v][k] = IO<T>::round(acc[v][k] + IO<T>::round(beta * IO<T>::round(hv[k] - acc[v][k])));
+      }
+    }
+    float P[VPT][8];
+#pragma unroll
+    for (int v = 0; v < VPT; ++v)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) P[v][k] = 0.f;
+    float S = 0.f, mref = -INFINITY;
+    auto one = [&](int i, Raw (&rw)[VPT]) {   // source i, then its slot refilled with source i + PD
+      float e[VPT][8];
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) IO<T>::unpack(UIO<T>::masked(rw[v], mk[v]), e[v]);
+      if (i + PD < n) load_src(i + PD, rw);
+      if (online) {
+        float pd[1] = {0.f};
+#pragma unroll
+        for (int v = 0; v < VPT; ++v)
+#pragma unroll
+          for (int k = 0; k < 8; ++k) pd[0] += qv[v][k] * e[v][k];
+        row_sum<1>(pd, tpr, red);
+        const float l = pd[0] * rsc[i] * inv + s_lc[i];
+        if (R.lr == 0) {
+          lg[i] = l;
+          if (valid) dots[(int64_t)i * dots_stride + tok] = pd[0];
+        }
+        if (!qz) {
+          if (l > mref + RF_LAZY) {   // the reference maximum moves: the running sums rescaled (k_read_online)
+            const float a = expf(mref - l);
+            S *= a;
+#pragma unroll
+            for (int v = 0; v < VPT; ++v)
+#pragma unroll
+              for (int k = 0; k < 8; ++k) P[v][k] *= a;
+            mref = l;
+          }
+          const float ex = expf(l - mref);
+          S += ex;
+#pragma unroll
+          for (int v = 0; v < VPT; ++v)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) P[v][k] += ex * e[v][k];
+        }
+      }
+      const float w = wt[i];
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[v][k] += w * e[v][k];
+    };
+    int i0 = 0;
+    for (; i0 + PD <= n; i0 += PD) {
+#pragma unroll
+      for (int j = 0; j < PD; ++j) one(i0 + j, buf[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < PD; ++j)
+      if (i0 + j < n) one(i0 + j, buf[j]);
+    if (online && !qz) {
+      const float f = M / S;
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[v][k] += f * P[v][k];
+    }
+    if (valid) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+        if (R.act(v)) R.store(out + roff, v, acc[v]);
+    }
+    R.sync();
+    if (online) {
+      row_softmax(lg, n, R);
+      R.sync();
+      if (valid) {
+        for (int i = R.lr; i < n; i += tpr) {
+          tc[tok * n + i] = s_c0[i] + M * (lg[i] - s_p0[i]);
+          if (prob) prob[tok * n + i] = lg[i];   // for the backward only
+        }
+      }
+      R.sync();   // this row's scalars are read before the next row overwrites them
+    }
+  }
+}
+
+// Backward pass 1 (k_bwd1), its formulas and summation orders (fp32 updates: g . v in fp64). Dynamic LDS: per row of
+// the workgroup p, p r and the upstream tc gradient (then g . v) [n]; at the end the workgroup's dq [d].
+template <typename T, int VPT, typename TAB>
+__global__ __launch_bounds__(WG) void k_rows_bwd1(TAB src, int n, const T* __restrict__ g,
+                                                  const float* __restrict__ gt, const float* __restrict__ prob,
+                                                  const float* __restrict__ dots, int64_t dots_stride,
+                                                  const float* __restrict__ tcp, Coef cf, float inv,
+                                                  float* __restrict__ dcbar, int dcbar_cols, int dr_accum,
+                                                  float* __restrict__ wz, int64_t wz_stride,
+                                                  float* __restrict__ dq_part, int64_t dq_stride,
+                                                  T* __restrict__ g_prop, T* __restrict__ g_h0, float beta,
+                                                  int64_t n_tok, int d, int tpr) {
+  constexpr bool GD64 = LDR_B1_GD64 && std::is_same<T, float>::value;
+  typedef typename std::conditional<GD64, double, float>::type Acc;
+  constexpr int C = VPT == 1 ? 4 : VPT == 2 ? 2 : 1;   // sources per row reduction
+  using Raw = typename IO<T>::Raw;
+  extern __shared__ float dyn[];
+  __shared__ float s_M;
+  __shared__ Acc red[4 * C];
+  const URows R(d, tpr);
+  const int tid = (int)threadIdx.x;
+  for (int i = tid; i < n; i += WG) {
+#pragma clang fp contract(off)
+    dyn[i] = i < cf.c0_cols ? cf.lam * cf.c0[i] : cf.lam;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    float m = 0.f;
+    for (int i = 0; i < n; ++i) m += dyn[i];
+    s_M = m;
+  }
+  __syncthreads();
+  const float M = s_M;
+  float *s_p = dyn + R.rs * 3 * n, *s_pr = s_p + n, *s_x = s_pr + n;
+  typename UIO<T>::Mask mk[VPT];
+  float dqa[VPT][8];
+#pragma unroll
+  for (int v = 0; v < VPT; ++v) {
+    mk[v] = UIO<T>::mask(R.skip(v));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) dqa[v][k] = 0.f;
+  }
+  const int64_t groups = (n_tok + R.rpw - 1) / R.rpw;
+  for (int64_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+    const int64_t tok = gi * R.rpw + R.rs;
+    const bool valid = tok < n_tok;
+    const int64_t tk = valid ? tok : n_tok - 1;
+    const int64_t roff = tk * (int64_t)d;
+    Raw cur[C][VPT], gq[VPT];
+    auto load_chunk = [&](int i0, Raw (&rw)[C][VPT]) {   // sources past the last: the last one again, not used
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const T* p = static_cast<const T*>(src.v(min(i0 + c, n - 1))) + roff;
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) rw[c][v] = UIO<T>::raw_nt(p + R.off(v));
+      }
+    };
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) gq[v] = UIO<T>::raw(g + roff + R.off(v));
+    load_chunk(0, cur);
+    for (int i = R.lr; i < n; i += tpr) {
+      const float p = prob[tk * n + i];
+      s_p[i] = p;
+      s_pr[i] = p * src.r(i)[tk];
+      s_x[i] = gt ? gt[tk * n + i] : 0.f;
+    }
+    R.sync();
+    float gv[VPT][8], a[VPT][8], b[VPT][8];
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+      IO<T>::unpack(UIO<T>::masked(gq[v], mk[v]), gv[v]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[v][k] = b[v][k] = 0.f;
+    }
+    if ((g_prop || g_h0) && valid) {   // the blend's gradients: beta g to h0, g - beta g to the proposal
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) {
+        if (!R.act(v)) continue;
+        float gb[8], gpv[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          gb[k] = IO<T>::round(beta * gv[v][k]);
+          gpv[k] = gv[v][k] - gb[k];
+        }
+        if (g_h0) R.store(g_h0 + roff, v, gb);
+        if (g_prop) R.store(g_prop + roff, v, gpv);
+      }
+    }
+    Acc sacc = 0;
+    for (int i0 = 0; i0 < n; i0 += C) {   // the next chunk's loads in flight while this one is reduced
+      Raw nxt[C][VPT];
+      if (i0 + C < n) load_chunk(i0 + C, nxt);
+      Acc pd[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        pd[c] = 0;
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) {
+          float e[8];
+          IO<T>::unpack(UIO<T>::masked(cur[c][v], mk[v]), e);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) pd[c] += (Acc)(gv[v][k] * e[k]);
+        }
+      }
+      if constexpr (GD64) row_sum_d(pd, tpr, red);
+      else row_sum(pd, tpr, red);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        if (i0 + c < n) {   // uniform
+          const int i = i0 + c;
+          const float pr = s_pr[i];
+          const Acc gp = (Acc)M * (pd[c] + (Acc)s_x[i]);
+          sacc += (Acc)s_p[i] * gp;
+          const float alpha = (float)((Acc)pr * gp);
+#pragma unroll
+          for (int v = 0; v < VPT; ++v) {
+            float e[8];
+            IO<T>::unpack(cur[c][v], e);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              a[v][k] += alpha * e[k];
+              b[v][k] += pr * e[k];
+            }
+          }
+        }
+      }
+      R.sync();   // every lane has read this chunk's upstream gradients before their slots take g . v
+      if (R.lr == 0) {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          if (i0 + c < n) s_x[i0 + c] = (float)pd[c];
+      }
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) cur[c][v] = nxt[c][v];
+    }
+    const float sf = (float)sacc;
+    if (valid) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) dqa[v][k] += a[v][k] - sf * b[v][k];
+    }
+    R.sync();
+    if (valid) {
+      for (int i = R.lr; i < n; i += tpr) {
+        const float gd = s_x[i];
+        const float gp = M * (gd + (gt ? gt[tok * n + i] : 0.f));
+        const float dz = s_p[i] * (gp - sf);
+        if (i < dcbar_cols) dcbar[tok * dcbar_cols + i] = -(cf.lam * gd);
+        float* dri = src.dr(i);
+        const float drv = dz * dots[(int64_t)i * dots_stride + tok] * inv;
+        dri[tok] = dr_accum ? dri[tok] + drv : drv;
+        *reinterpret_cast<float2*>(wz + 2 * ((int64_t)i * wz_stride + tok)) =
+            make_float2(tcp[tok * n + i] - coef_cbar(cf, tok, i), dz * src.r(i)[tok] * inv);
+      }
+    }
+    R.sync();   // the row's scalars are read before the next row overwrites them
+  }
+  // the workgroup's dq: row slots add their columns in a fixed order
+  __syncthreads();
+  for (int k = 0; k < R.rpw; ++k) {
+    if (R.rs == k) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) {
+        const int s = R.skip(v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (e >= s) {
+            float* o = dyn + R.off(v) + e;
+            const float val = dqa[v][e] * inv;
+            *o = k == 0 ? val : *o + val;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int c = tid; c < d; c += WG) dq_part[(int64_t)blockIdx.x * dq_stride + c] = dyn[c];
+}
+
+// token rows per lane of the update gradient, within two waves' registers
+template <typename T> constexpr int rows_rb(int vpt) {
+  return std::is_same<T, float>::value ? (vpt == 1 ? 4 : 2) : (vpt <= 2 ? 4 : 2);
+}
+
+// The update gradient (k_dv_assemble): the same roundings in the same order, so the same bits for the same table.
+// RB token rows per lane share each query load.
+template <typename T, int VPT, bool PER_READ, typename TAB>
+__global__ __launch_bounds__(WG) void k_rows_dv_assemble(TAB tab, int m, const T* __restrict__ vsrc,
+                                                         const float* __restrict__ r, const float* __restrict__ gr,
+                                                         const T* __restrict__ add, float add_beta,
+                                                         T* __restrict__ dv, T* __restrict__ dv_neg, int64_t n_tok,
+                                                         int d, int tpr) {
+  constexpr int RB = rows_rb<T>(VPT);
+  const URows R(d, tpr);
+  const int64_t per = (int64_t)R.rpw * RB, tiles = (n_tok + per - 1) / per;
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    int64_t tok[RB], tk[RB];
+    float acc[RB][VPT][8];
+#pragma unroll
+    for (int k = 0; k < RB; ++k) {
+      tok[k] = tile * per + R.rs + (int64_t)k * R.rpw;
+      tk[k] = min(tok[k], n_tok - 1);
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int x = 0; x < 8; ++x) acc[k][v][x] = 0.f;
+    }
+    for (int j = 0; j < m; ++j) {
+      const T* gj = static_cast<const T*>(tab.g(j));
+      const float *wj = tab.wz(j), *qj = tab.q(j);
+      typename IO<T>::Raw raw[RB][VPT];
+      float2 sc[RB];
+      float qv[VPT][8];
+#pragma unroll
+      for (int k = 0; k < RB; ++k)
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) raw[k][v] = UIO<T>::raw_nt(gj + tk[k] * (int64_t)d + R.off(v));
+#pragma unroll
+      for (int k = 0; k < RB; ++k) sc[k] = *reinterpret_cast<const float2*>(wj + 2 * tk[k]);
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) IO<float>::unpack(UIO<float>::raw(qj + R.off(v)), qv[v]);
+#pragma unroll
+      for (int k = 0; k < RB; ++k)
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) {
+          float e[8];
+          IO<T>::unpack(raw[k][v], e);
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            if (PER_READ) {
+              const float t = IO<T>::round(bwd2_term(sc[k].x, e[x], sc[k].y, qv[v][x]));
+              acc[k][v][x] = j == 0 ? t : IO<T>::round(acc[k][v][x] + t);
+            } else {
+              acc[k][v][x] = __builtin_fmaf(sc[k].y, qv[v][x], __builtin_fmaf(sc[k].x, e[x], acc[k][v][x]));
+            }
+          }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < RB; ++k) {
+      const int64_t roff = tk[k] * (int64_t)d;
+      const float rv = r[tk[k]];
+      const float c = gr ? gr[tk[k]] * (-rv * rv * rv) / (float)d : 0.f;
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) {
+        float e[8], a[8], o[8];
+        IO<T>::unpack(UIO<T>::raw(vsrc + roff + R.off(v)), e);
+        if (add) {   // a gradient of the write's h from elsewhere, added as autograd would add it
+          IO<T>::unpack(UIO<T>::raw(add + roff + R.off(v)), a);
+          if (add_beta != 0.f) {   // the proposal's share of an iteration-end blend's output gradient
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int x = 0; x < 8; ++x) a[x] = IO<T>::round(a[x] - IO<T>::round(add_beta * a[x]));
+          }
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          if (PER_READ) {
+#pragma clang fp contract(off)
+            o[x] = acc[k][v][x];
+            if (gr) {
+              const float gx = IO<T>::round(c * e[x]);
+              o[x] = m == 0 ? gx : IO<T>::round(o[x] + gx);
+            }
+          } else {
+            o[x] = __builtin_fmaf(c, e[x], acc[k][v][x]);
+          }
+        }
+        if (tok[k] < n_tok && R.act(v)) {
+          if (dv_neg) {
+            float ng[8];
+#pragma unroll
+            for (int x = 0; x < 8; ++x) ng[x] = -o[x];
+            R.store(dv_neg + roff, v, ng);
+          }
+          if (add) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) o[x] = IO<T>::round(o[x]) + a[x];
+          }
+          R.store(dv + roff, v, o);
+        }
+      }
+    }
+  }
+}
+
+// Backward pass 2, list layout (k_bwd2_list): dv_i (=|+=) w_i g + dzr_i q, the accumulation rounded as autograd's
+template <typename T, int VPT, typename TAB>
+__global__ __launch_bounds__(WG) void k_rows_bwd2_list(TAB tab, int n, int accum, const T* __restrict__ g,
+                                                       const float* __restrict__ q, const float* __restrict__ wz,
+                                                       int64_t wz_stride, int64_t n_tok, int d, int tpr) {
+  const URows R(d, tpr);
+  float qv[VPT][8];
+#pragma unroll
+  for (int v = 0; v < VPT; ++v) IO<float>::unpack(UIO<float>::raw(q + R.off(v)), qv[v]);
+  const int64_t groups = (n_tok + R.rpw - 1) / R.rpw;
+  for (int64_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+    const int64_t tok = gi * R.rpw + R.rs;
+    if (tok >= n_tok) continue;
+    const int64_t roff = tok * (int64_t)d;
+    float gv[VPT][8];
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) IO<T>::unpack(UIO<T>::raw(g + roff + R.off(v)), gv[v]);
+    for (int i = 0; i < n; ++i) {
+      const float2 s = *reinterpret_cast<const float2*>(wz + 2 * ((int64_t)i * wz_stride + tok));
+      T* dvi = static_cast<T*>(tab.p(i)) + roff;
+      typename IO<T>::Raw prev[VPT];
+      if (accum) {
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) prev[v] = UIO<T>::raw(dvi + R.off(v));
+      }
+#pragma unroll
+      for (int v = 0; v < VPT; ++v) {
+        float o[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o[k] = bwd2_term(s.x, gv[v][k], s.y, qv[v][k]);
+        if (accum) {
+          float pv[8];
+          IO<T>::unpack(prev[v], pv);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) o[k] = pv[k] + IO<T>::round(o[k]);
+        }
+        if (R.act(v)) R.store(dvi, v, o);
+      }
+    }
+  }
+}
+
+// out = round(sum_j round(beta * g_j)) in table order, or with per_read each addition rounded (k_blend_sum); the
+// tensors taken as flat runs of elements, eight per lane, the last total mod 8 one per lane
+template <typename T, typename TAB>
+__global__ __launch_bounds__(WG) void k_flat_blend_sum(TAB tab, int m, float beta, int per_read, T* __restrict__ out,
+                                                       int64_t total) {
+#pragma clang fp contract(off)
+  const int64_t nv = total >> 3, step = (int64_t)gridDim.x * WG;
+  for (int64_t c = (int64_t)blockIdx.x * WG + threadIdx.x; c < nv; c += step) {
+    float acc[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) acc[x] = 0.f;
+    for (int j = 0; j < m; ++j) {
+      float e[8];
+      IO<T>::unpack(UIO<T>::raw_nt(static_cast<const T*>(tab.p(j)) + 8 * c), e);
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        const float t = IO<T>::round(beta * e[x]);
+        acc[x] = !per_read ? acc[x] + t : (j == 0 ? t : IO<T>::round(acc[x] + t));
+      }
+    }
+    UIO<T>::store(out + 8 * c, acc);
+  }
+  if (blockIdx.x == 0 && (int)threadIdx.x < (int)(total & 7)) {
+    const int64_t e = 8 * nv + threadIdx.x;
     float acc = 0.f;
     for (int j = 0; j < m; ++j) {
-      const float t = IO<T>::round(beta * ld1(reinterpret_cast<const T*>(tg[j]) + e));
+      const float t = IO<T>::round(beta * ld1(static_cast<const T*>(tab.p(j)) + e));
       acc = !per_read ? acc + t : (j == 0 ? t : IO<T>::round(acc + t));
     }
     st1(out + e, acc);
@@ -3019,6 +3787,132 @@ int scratch_on(hipStream_t st, float** out) {
 // a vector of fp32 zeros, by a kernel (no memset node in a captured graph)
 __global__ __launch_bounds__(WG) void k_zero(float* __restrict__ p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) p[i] = 0.f;
+}
+
+// unaligned rows: vectors per lane (1, 2 or 4) and lanes per row for width d, the fewest idle lanes first, then rows
+// inside one wave, then fewer vectors per lane; with many sources fewer rows per workgroup (their per-source scalars
+// take 3 n floats of LDS each: at most 48 KiB)
+int rows_layout(int64_t d, int64_t n, int* vpt, int* tpr) {
+  if (d < 8 || d > LDR_MAX_WIDTH) return LDR_E_SHAPE;
+  const int64_t d8 = (d + 7) >> 3;
+  int64_t best = INT64_MAX;
+  for (int v = 1; v <= 4; v <<= 1) {
+    for (int t = 8; t <= WG; t <<= 1) {
+      if ((int64_t)v * t < d8 || (WG / t) * n > 4096) continue;
+      const int64_t key = ((int64_t)v * t - d8) * 16 + (t > 64 ? 8 : 0) + v;
+      if (key < best) { best = key; *vpt = v; *tpr = t; }
+    }
+  }
+  return best == INT64_MAX ? LDR_E_SHAPE : LDR_OK;
+}
+
+inline bool rows_width(int64_t d) { return d >= 8 && d <= LDR_MAX_WIDTH; }
+
+#define LDR_VPT124_SWITCH(VPT_RT, ...)                           \
+  switch (VPT_RT) {                                              \
+    case 1: { constexpr int VPT = 1; __VA_ARGS__; } break;       \
+    case 2: { constexpr int VPT = 2; __VA_ARGS__; } break;       \
+    default: { constexpr int VPT = 4; __VA_ARGS__; } break;      \
+  }
+
+template <typename TAB>
+int rows_read(const TAB& src, int64_t n, const float* q, float* dots, int64_t dots_stride, const void* base,
+              const void* h0, float beta, const Coef& cf, float inv, void* out, float* tc, float* p,
+              float* next_prior, int64_t n_tok, int64_t d, int dtype, hipStream_t st) {
+  int vpt, tpr, e = rows_layout(d, n, &vpt, &tpr);
+  if (e) return e;
+  const size_t lds = sizeof(float) * (size_t)(3 * n * (1 + WG / tpr));
+  const unsigned grid = grid_of(cdiv(n_tok, WG / tpr), 2048);   // no tokens: one workgroup writes next_prior
+#define LDR_ROWS_READ(BL)                                                                                            \
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_read<T, VPT, BL, TAB>), dim3(grid),        \
+      dim3(WG), lds, st, src, (int)n, q, dots, dots_stride, static_cast<const T*>(base), static_cast<const T*>(h0),    \
+      beta, cf, inv, static_cast<T*>(out), tc, p, next_prior, n_tok, (int)d, tpr)))
+  if (h0) {
+    LDR_ROWS_READ(true)
+  } else {
+    LDR_ROWS_READ(false)
+  }
+#undef LDR_ROWS_READ
+  return launched();
+}
+
+template <typename TAB>
+int rows_bwd1(const TAB& src, int64_t n, const void* g, const float* gt, const float* p, const float* dots,
+              int64_t dots_stride, const float* tc, const Coef& cf, float inv, float* dcbar, int64_t dcbar_cols,
+              int dr_accum, float* wz, int64_t wz_stride, float* dq_part, int64_t dq_parts, int64_t dq_part_stride,
+              void* g_prop, void* g_h0, float beta, int64_t n_tok, int64_t d, int dtype, hipStream_t st) {
+  int vpt, tpr, e = rows_layout(d, n, &vpt, &tpr);
+  if (e) return e;
+  const int64_t planes = 3 * n * (WG / tpr);
+  const size_t lds = sizeof(float) * (size_t)(planes > d ? planes : d);
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd1<T, VPT, TAB>),
+      dim3((unsigned)dq_parts), dim3(WG), lds, st, src, (int)n, static_cast<const T*>(g), gt, p, dots, dots_stride, tc,
+      cf, inv, dcbar, (int)dcbar_cols, dr_accum, wz, wz_stride, dq_part, dq_part_stride, static_cast<T*>(g_prop),
+      static_cast<T*>(g_h0), beta, n_tok, (int)d, tpr)))
+  return launched();
+}
+
+template <typename TAB>
+int rows_dv_assemble(const TAB& tab, int64_t m, const void* v, const float* r, const float* gr, const void* add,
+                     float add_beta, int per_read, void* dv, void* dv_neg, int64_t n_tok, int64_t d, int dtype,
+                     hipStream_t st) {
+  int vpt, tpr, e = rows_layout(d, 1, &vpt, &tpr);
+  if (e) return e;
+  const int rb = dtype == LDR_F32 ? rows_rb<float>(vpt) : rows_rb<bf16_t>(vpt);
+  const unsigned grid = grid_of(cdiv(n_tok, (WG / tpr) * rb), 65535);
+#define LDR_ROWS_AS(PR)                                                                                              \
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_dv_assemble<T, VPT, PR, TAB>), dim3(grid), \
+      dim3(WG), 0, st, tab, (int)m, static_cast<const T*>(v), r, gr, static_cast<const T*>(add), add_beta,             \
+      static_cast<T*>(dv), static_cast<T*>(dv_neg), n_tok, (int)d, tpr)))
+  if (per_read) {
+    LDR_ROWS_AS(true)
+  } else {
+    LDR_ROWS_AS(false)
+  }
+#undef LDR_ROWS_AS
+  return launched();
+}
+
+template <typename TAB>
+int rows_bwd2_list(const TAB& dv, int64_t n, int accum, const void* g, const float* q, const float* wz,
+                   int64_t wz_stride, int64_t n_tok, int64_t d, int dtype, hipStream_t st) {
+  int vpt, tpr, e = rows_layout(d, 1, &vpt, &tpr);
+  if (e) return e;
+  const unsigned grid = grid_of(cdiv(n_tok, WG / tpr), 8192);
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd2_list<T, VPT, TAB>), dim3(grid),
+      dim3(WG), 0, st, dv, (int)n, accum, static_cast<const T*>(g), q, wz, wz_stride, n_tok, (int)d, tpr)))
+  return launched();
+}
+
+template <typename TAB>
+int flat_blend_sum(const TAB& g, int64_t m, float beta, int per_read, void* out, int64_t total, int dtype,
+                   hipStream_t st) {
+  LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_flat_blend_sum<T, TAB>), dim3(grid_of(cdiv(total, 8 * WG), 8192)),
+                                             dim3(WG), 0, st, g, (int)m, beta, per_read, static_cast<T*>(out), total))
+  return launched();
+}
+
+// host address arrays into kernel arguments, every row pointer element-aligned
+inline bool al_elt(const void* p, int dtype) {
+  return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(elt_bytes(dtype) - 1)) == 0;
+}
+
+int fill_rows(SrcTab& s, const uint64_t* v, const uint64_t* r, int64_t n, int64_t n_tok, int dtype) {
+  for (int64_t i = 0; i < MAXS; ++i) {
+    s.v[i] = i < n ? reinterpret_cast<const void*>(v[i]) : nullptr;
+    s.r[i] = i < n ? reinterpret_cast<const float*>(r[i]) : nullptr;
+    if (i < n && (!tok_ptr(s.v[i], n_tok) || !tok_ptr(s.r[i], n_tok))) return LDR_E_ARG;
+    if (i < n && !al_elt(s.v[i], dtype)) return LDR_E_ALIGN;
+  }
+  return LDR_OK;
+}
+
+// backward pass 1 with dq_parts workgroups on the row layout: the smallest power-of-two tile that covers the tokens
+// in one round (at least a row per row slot, at most a tile's LDS planes)
+inline int b1_tile_for(int64_t n_tok, int64_t dq_parts, int tpr) {
+  int t = WG / tpr;
+  while (t < TT_MAX && (int64_t)t * dq_parts < n_tok) t <<= 1;
+  return t;
 }
 
 }  // namespace
@@ -3481,11 +4375,9 @@ int ldr_dv_assemble(const uint64_t* g, const uint64_t* wz, const uint64_t* q, in
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// any-shape entry points: per-source addresses in device arrays, rows of any width at element alignment
+// any-shape entry points: rows of any width at element alignment, the per-source addresses by value (*_rows) or in
+// device arrays (*_any)
 // ---------------------------------------------------------------------------------------------------------------
-static inline bool al_elt(const void* p, int dtype) {
-  return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(elt_bytes(dtype) - 1)) == 0;
-}
 static inline unsigned any_row_grid(int64_t n_tok, int64_t cap) { return grid_of(cdiv(n_tok, ANY_WAVES), cap); }
 
 int ldr_read_fwd_any(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const float* q, float* dots,
@@ -3501,9 +4393,12 @@ int ldr_read_fwd_any(const uint64_t* src_v, const uint64_t* src_r, int64_t n, co
   if (!al_elt(base, dtype) || !al_elt(out, dtype) || (h0 && !al_elt(h0, dtype))) return LDR_E_ALIGN;
   if (n_tok == 0 && !next_prior) return LDR_OK;
   const Coef cf{cbar, (int)cbar_cols, c0, (int)c0_cols, lam};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rows_width(d))
+    return rows_read(DevSrc{src_v, src_r, nullptr}, n, q, dots, dots_stride, base, h0, beta, cf, inv_sqrt_d, out, tc, p,
+                     next_prior, n_tok, d, dtype, st);
   const size_t lds = sizeof(float) * (size_t)((3 + ANY_WAVES) * n + 4);
   const unsigned grid = any_row_grid(n_tok, 4096);   // no tokens: one workgroup writes next_prior
-  hipStream_t st = static_cast<hipStream_t>(stream);
 #define LDR_ANY_READ(BL)                                                                                          \
   LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_any_read<T, BL>), dim3(grid), dim3(WG), lds, st, src_v, src_r,    \
                                              (int)n, q, dots, dots_stride, static_cast<const T*>(base),           \
@@ -3538,8 +4433,12 @@ int ldr_read_bwd1_any(const uint64_t* src_v, const uint64_t* src_r, int64_t n, c
       (reinterpret_cast<uintptr_t>(wz) & 7u))
     return LDR_E_ALIGN;
   const Coef cf{cbar, (int)cbar_cols, c0, (int)c0_cols, lam};
-  const size_t lds = sizeof(float) * (size_t)(4 * n);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rows_width(d))
+    return rows_bwd1(DevSrc{src_v, src_r, dr}, n, g, gt, p, dots, dots_stride, tc, cf, inv_sqrt_d, dcbar, dcbar_cols,
+                     dr_accum, wz, wz_stride, dq_part, dq_parts, dq_part_stride, g_prop, g_h0, beta, n_tok, d, dtype,
+                     st);
+  const size_t lds = sizeof(float) * (size_t)(4 * n);
   // every partial row is written (zeros for a workgroup without tokens), so the caller sums dq_parts rows
   LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_any_bwd1<T>), dim3((unsigned)dq_parts), dim3(64), lds, st, src_v,
                                              src_r, (int)n, static_cast<const T*>(g), gt, p, dots, dots_stride, tc,
@@ -3561,6 +4460,8 @@ int ldr_dv_assemble_any(const uint64_t* g, const uint64_t* wz, const uint64_t* q
     return LDR_E_ALIGN;
   if (n_tok == 0) return LDR_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rows_width(d))
+    return rows_dv_assemble(DevAsm{g, wz, q}, m, v, r, gr, add, add_beta, per_read, dv, dv_neg, n_tok, d, dtype, st);
 #define LDR_ANY_AS(PR)                                                                                            \
   LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_any_dv_assemble<T, PR>), dim3(any_row_grid(n_tok, 8192)), dim3(WG), 0, \
                                              st, g, wz, q, (int)m, static_cast<const T*>(v), r, gr,                 \
@@ -3585,6 +4486,8 @@ int ldr_read_bwd2_list_any(const uint64_t* dv, int64_t n, int accum, const void*
   if (!al_elt(g, dtype) || (reinterpret_cast<uintptr_t>(wz) & 7u)) return LDR_E_ALIGN;
   if (n_tok == 0) return LDR_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rows_width(d))
+    return rows_bwd2_list(DevPtr{dv}, n, accum, g, q, wz, wz_stride, n_tok, d, dtype, st);
   LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_any_bwd2_list<T>), dim3(any_row_grid(n_tok, 8192)), dim3(WG), 0, st,
                                              dv, (int)n, accum, static_cast<const T*>(g), q, wz, wz_stride, n_tok, d))
   return launched();
@@ -3598,10 +4501,157 @@ int ldr_blend_sum_any(const uint64_t* g, int64_t m, float beta, int per_read, vo
   if (!g || !tok_ptr(out, n_tok) || n_tok < 0) return LDR_E_ARG;
   if (!al_elt(out, dtype)) return LDR_E_ALIGN;
   if (n_tok == 0) return LDR_OK;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_any_blend_sum<T>), dim3(grid_of(cdiv(n_tok * d, WG), 8192)), dim3(WG),
-                                             0, st, g, (int)m, beta, per_read, static_cast<T*>(out), n_tok, d))
+  return flat_blend_sum(DevPtr{g}, m, beta, per_read, out, n_tok * d, dtype, static_cast<hipStream_t>(stream));
+}
+
+// the *_rows entry points: rows of any width 8 <= d <= LDR_MAX_WIDTH at element alignment, host address arrays
+int ldr_write_rows(const void* h, const void* x, void* v_out, float* r_out, int64_t n_tok, int64_t d, float eps,
+                   int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (n_tok < 0 || !tok_ptr(h, n_tok) || !tok_ptr(x, n_tok) || !tok_ptr(v_out, n_tok) || !tok_ptr(r_out, n_tok))
+    return LDR_E_ARG;
+  if (d < 1) return LDR_E_SHAPE;
+  if (!al_elt(h, dtype) || !al_elt(x, dtype) || !al_elt(v_out, dtype)) return LDR_E_ALIGN;
+  if (n_tok == 0) return LDR_OK;
+  LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_write_any<T>), dim3(any_row_grid(n_tok, 8192)), dim3(WG), 0,
+                                             static_cast<hipStream_t>(stream), static_cast<const T*>(h),
+                                             static_cast<const T*>(x), static_cast<T*>(v_out), r_out, n_tok, d, eps))
   return launched();
+}
+
+int ldr_read_fwd_rows(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const float* q, float* dots,
+                      int64_t dots_stride, const void* base, const void* h0, float beta, const float* cbar,
+                      int64_t cbar_cols, const float* c0, int64_t c0_cols, float lam, float inv_sqrt_d, void* out,
+                      float* tc, float* p, float* next_prior, int64_t n_tok, int64_t d, int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (n < 1 || n > MAXS || !rows_width(d)) return LDR_E_SHAPE;
+  if (!src_v || !src_r || n_tok < 0 || !tok_ptr(dots, n_tok) || dots_stride < n_tok || !tok_ptr(base, n_tok) ||
+      !tok_ptr(cbar, n_tok) || !c0 || !tok_ptr(out, n_tok) || !tok_ptr(tc, n_tok))
+    return LDR_E_ARG;
+  if ((cbar_cols != n && cbar_cols != n - 1) || (c0_cols != n && c0_cols != n - 1)) return LDR_E_ARG;
+  if (!al_elt(base, dtype) || !al_elt(out, dtype) || (h0 && !al_elt(h0, dtype))) return LDR_E_ALIGN;
+  ValSrc s{};
+  const int e = fill_rows(s.t, src_v, src_r, n, n_tok, dtype);
+  if (e) return e;
+  if (n_tok == 0 && !next_prior) return LDR_OK;
+  return rows_read(s, n, q, dots, dots_stride, base, h0, beta, Coef{cbar, (int)cbar_cols, c0, (int)c0_cols, lam},
+                   inv_sqrt_d, out, tc, p, next_prior, n_tok, d, dtype, static_cast<hipStream_t>(stream));
+}
+
+int64_t ldr_read_bwd1_rows_parts(int64_t n_tok, int64_t d) {
+  int vpt, tpr;
+  if (n_tok < 1) return 0;
+  if (row_layout(d, &vpt, &tpr, B1_MAX_VPT, LDR_B1_WAVE_ROWS, LDR_B1_VPT, true) != LDR_OK &&
+      rows_layout(d, 1, &vpt, &tpr) != LDR_OK)
+    return 0;
+  // a workgroup on every CU first (256), then two rows per row slot before a second one: each part is a row of d
+  // floats to write and reduce
+  const int rpw = WG / tpr;
+  const int64_t one = grid_of(cdiv(n_tok, rpw), 256), two = grid_of(cdiv(n_tok, 2 * rpw), B1_GRID);
+  return one > two ? one : two;
+}
+
+int ldr_read_bwd1_rows(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const void* g, const float* gt,
+                       const float* p, const float* dots, int64_t dots_stride, const float* tc, const float* cbar,
+                       int64_t cbar_cols, const float* c0, int64_t c0_cols, float lam, float inv_sqrt_d, float* dcbar,
+                       int64_t dcbar_cols, const uint64_t* dr, int dr_accum, float* wz, int64_t wz_stride,
+                       float* dq_part, int64_t dq_parts, int64_t dq_part_stride, void* g_prop, void* g_h0, float beta,
+                       int64_t n_tok, int64_t d, int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (n < 1 || n > MAXS || !rows_width(d)) return LDR_E_SHAPE;
+  if (!src_v || !src_r || n_tok < 0 || !tok_ptr(g, n_tok) || !tok_ptr(p, n_tok) || !tok_ptr(dots, n_tok) ||
+      dots_stride < n_tok || !tok_ptr(tc, n_tok) || !tok_ptr(cbar, n_tok) || !c0 || !tok_ptr(dcbar, n_tok) || !dr ||
+      !tok_ptr(wz, n_tok) || !dq_part || wz_stride < n_tok || dq_part_stride < d || dq_parts < 1 ||
+      dq_parts > 65535 || (dr_accum != 0 && dr_accum != 1))
+    return LDR_E_ARG;
+  if ((cbar_cols != n && cbar_cols != n - 1) || (c0_cols != n && c0_cols != n - 1) || dcbar_cols < 0 ||
+      dcbar_cols > n)
+    return LDR_E_ARG;
+  if (!al_elt(g, dtype) || (g_prop && !al_elt(g_prop, dtype)) || (g_h0 && !al_elt(g_h0, dtype)) ||
+      (reinterpret_cast<uintptr_t>(wz) & 7u))
+    return LDR_E_ALIGN;
+  ValSrc s{};
+  const int e = fill_rows(s.t, src_v, src_r, n, n_tok, dtype);
+  if (e) return e;
+  bool vec = al16(g) && al16(g_prop) && al16(g_h0);
+  for (int64_t i = 0; i < n; ++i) {
+    s.d.p[i] = reinterpret_cast<void*>(dr[i]);
+    if (!tok_ptr(s.d.p[i], n_tok)) return LDR_E_ARG;
+    vec = vec && al16(s.t.v[i]);
+  }
+  const Coef cf{cbar, (int)cbar_cols, c0, (int)c0_cols, lam};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int vpt, tpr;
+  if (vec && n_tok > 0 && row_layout(d, &vpt, &tpr, B1_MAX_VPT, LDR_B1_WAVE_ROWS, LDR_B1_VPT, true) == LDR_OK) {
+    const int tt = b1_tile_for(n_tok, dq_parts, tpr);
+    LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_bwd1<T, VPT, B1Chunk<VPT>::C>),
+        dim3((unsigned)dq_parts), dim3(WG), 0, st, s.t, (int)n, static_cast<const T*>(g), gt, p, dots, dots_stride, tc,
+        cf, inv_sqrt_d, dcbar, (int)dcbar_cols, s.d, dr_accum, wz, wz_stride, dq_part, dq_part_stride,
+        static_cast<T*>(g_prop), static_cast<T*>(g_h0), beta, n_tok, (int)d, tpr, tt)))
+    return launched();
+  }
+  return rows_bwd1(s, n, g, gt, p, dots, dots_stride, tc, cf, inv_sqrt_d, dcbar, dcbar_cols, dr_accum, wz, wz_stride,
+                   dq_part, dq_parts, dq_part_stride, g_prop, g_h0, beta, n_tok, d, dtype, st);
+}
+
+int ldr_dv_assemble_rows(const uint64_t* g, const uint64_t* wz, const uint64_t* q, int64_t m, const void* v,
+                         const float* r, const float* gr, const void* add, float add_beta, int per_read, void* dv,
+                         void* dv_neg, int64_t n_tok, int64_t d, int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (per_read != 0 && per_read != 1) return LDR_E_ARG;
+  if (m < 0 || m > MAXS || !rows_width(d)) return LDR_E_SHAPE;
+  if ((m > 0 && (!g || !wz || !q)) || !tok_ptr(v, n_tok) || !tok_ptr(r, n_tok) || !tok_ptr(dv, n_tok) || n_tok < 0)
+    return LDR_E_ARG;
+  if (!al_elt(v, dtype) || !al_elt(dv, dtype) || (dv_neg && !al_elt(dv_neg, dtype)) || (add && !al_elt(add, dtype)))
+    return LDR_E_ALIGN;
+  ValAsm t{};
+  for (int64_t j = 0; j < m; ++j) {
+    t.t.g[j] = reinterpret_cast<const void*>(g[j]);
+    t.t.wz[j] = reinterpret_cast<const float*>(wz[j]);
+    t.t.q[j] = reinterpret_cast<const float*>(q[j]);
+    if (!tok_ptr(t.t.g[j], n_tok) || !tok_ptr(t.t.wz[j], n_tok) || !t.t.q[j]) return LDR_E_ARG;
+    if (!al_elt(t.t.g[j], dtype) || (reinterpret_cast<uintptr_t>(t.t.wz[j]) & 7u) ||
+        (reinterpret_cast<uintptr_t>(t.t.q[j]) & 3u))
+      return LDR_E_ALIGN;
+  }
+  if (n_tok == 0) return LDR_OK;
+  return rows_dv_assemble(t, m, v, r, gr, add, add_beta, per_read, dv, dv_neg, n_tok, d, dtype,
+                          static_cast<hipStream_t>(stream));
+}
+
+int ldr_read_bwd2_list_rows(const uint64_t* dv, int64_t n, int accum, const void* g, const float* q, const float* wz,
+                            int64_t wz_stride, int64_t n_tok, int64_t d, int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (n < 1 || n > MAXS || !rows_width(d)) return LDR_E_SHAPE;
+  if (!dv || !tok_ptr(g, n_tok) || !q || !tok_ptr(wz, n_tok) || wz_stride < n_tok || n_tok < 0 ||
+      (accum != 0 && accum != 1))
+    return LDR_E_ARG;
+  if (!al_elt(g, dtype) || (reinterpret_cast<uintptr_t>(wz) & 7u)) return LDR_E_ALIGN;
+  ValPtr t{};
+  for (int64_t i = 0; i < n; ++i) {
+    t.t.p[i] = reinterpret_cast<void*>(dv[i]);
+    if (!tok_ptr(t.t.p[i], n_tok)) return LDR_E_ARG;
+    if (!al_elt(t.t.p[i], dtype)) return LDR_E_ALIGN;
+  }
+  if (n_tok == 0) return LDR_OK;
+  return rows_bwd2_list(t, n, accum, g, q, wz, wz_stride, n_tok, d, dtype, static_cast<hipStream_t>(stream));
+}
+
+int ldr_blend_sum_rows(const uint64_t* g, int64_t m, float beta, int per_read, void* out, int64_t n_tok, int64_t d,
+                       int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return LDR_E_DTYPE;
+  if (per_read != 0 && per_read != 1) return LDR_E_ARG;
+  if (m < 1 || m > MAXS || !rows_width(d)) return LDR_E_SHAPE;
+  if (!g || !tok_ptr(out, n_tok) || n_tok < 0) return LDR_E_ARG;
+  if (!al_elt(out, dtype)) return LDR_E_ALIGN;
+  ValPtr t{};
+  for (int64_t j = 0; j < m; ++j) {
+    t.t.p[j] = reinterpret_cast<void*>(g[j]);
+    if (!tok_ptr(t.t.p[j], n_tok)) return LDR_E_ARG;
+    if (!al_elt(t.t.p[j], dtype)) return LDR_E_ALIGN;
+  }
+  if (n_tok == 0) return LDR_OK;
+  return flat_blend_sum(t, m, beta, per_read, out, n_tok * d, dtype, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

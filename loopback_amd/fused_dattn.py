@@ -113,8 +113,8 @@ def grad_rounding() -> str:
 
 def _fast(d: int, n: int, *rows) -> bool:
     """Whether the row-layout entry points take a call: width d a multiple of 8 up to MAX_WIDTH, at most
-    MAX_SOURCES sources, every row tensor 16-byte aligned. Other calls go to the any-shape entry points (rows of any
-    width at element alignment, up to ANY_MAX_SOURCES sources, per-source addresses in device arrays)."""
+    MAX_SOURCES sources, every row tensor 16-byte aligned. Other calls go to the unaligned-row entry points (_rows), or
+    to the any-shape ones (any width, up to ANY_MAX_SOURCES sources, per-source addresses in device arrays)."""
     if d % 8 or d > L.MAX_WIDTH or n > MAX_SOURCES:
         return False
     for t in rows:
@@ -123,56 +123,72 @@ def _fast(d: int, n: int, *rows) -> bool:
     return True
 
 
-def _dev_addrs(addrs, dev: torch.device) -> torch.Tensor:
-    """A device array of addresses for an any-shape entry point, copied on the current stream from pinned host
-    memory (torch keeps the host buffer until the copy has run; the device array is freed in stream order). Not
-    under HIP graph capture: a replay would copy from a host buffer torch may since have reused."""
+def _rows(d: int, n: int) -> bool:
+    """Whether the unaligned-row entry points (*_rows: element alignment, host address tables) take a call the
+    row-layout ones do not; the rest goes to the *_any ones (device address arrays)."""
+    return 8 <= d <= L.MAX_WIDTH and n <= MAX_SOURCES
+
+
+def _refuse_capture() -> None:
+    """Shapes outside the row layout are not captured in a HIP graph: a replay of the any-shape path would copy its
+    address arrays from a host buffer torch may since have reused."""
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("delta_attnres HIP read: shapes the row-layout kernels do not take (d not a multiple of 8 "
                            "or above 8192, more than 64 sources, unaligned rows) cannot be captured in a HIP graph")
+
+
+def _dev_addrs(addrs, dev: torch.device) -> torch.Tensor:
+    """A device array of addresses for an any-shape entry point, copied on the current stream from pinned host
+    memory (torch keeps the host buffer until the copy has run; the device array is freed in stream order)."""
+    _refuse_capture()
     host = torch.tensor(list(addrs), dtype=torch.int64).pin_memory()
     return host.to(dev, non_blocking=True)
 
 
 def _b1_parts(n_tok: int, d: int) -> int:
     """Rows of backward pass 1's query-gradient partials: the row-layout kernel's workgroups (which the any-shape
-    kernel then also uses), or for widths that layout does not take one per 64 tokens, up to 512."""
+    kernels then also use), or for widths that layout does not take as many as fill the GPU (one workgroup per four
+    tokens on the scalar kernels)."""
     p = L.bwd1_parts(n_tok, d)
-    return p if p > 0 else max(1, min(512, -(-n_tok // 64)))
+    return p if p > 0 else L.bwd1_rows_parts(n_tok, d) or max(1, min(512, -(-n_tok // 4)))
 
 
 class _Src:
     """The sources of one read: host address arrays (v, r; dr for the scale gradients) for the row-layout entry
-    points when `fast`, else device address arrays for the any-shape ones."""
-    __slots__ = ("fast", "v", "r", "dr")
+    points when `fast` and for the unaligned-row ones when `rows`, else device address arrays for the any-shape
+    ones."""
+    __slots__ = ("fast", "rows", "v", "r", "dr")
 
-    def __init__(self, fast: bool, v, r, dr=None):
-        self.fast, self.v, self.r, self.dr = fast, v, r, dr
+    def __init__(self, fast: bool, rows: bool, v, r, dr=None):
+        self.fast, self.rows, self.v, self.r, self.dr = fast, rows, v, r, dr
 
     @staticmethod
-    def of(fast: bool, values, rstds, dev, drs=None):
-        addrs = (lambda ts: L.u64_array(t.data_ptr() for t in ts)) if fast else \
+    def of(fast: bool, rows: bool, values, rstds, dev, drs=None):
+        addrs = (lambda ts: L.u64_array(t.data_ptr() for t in ts)) if fast or rows else \
                 (lambda ts: _dev_addrs((t.data_ptr() for t in ts), dev))
-        return _Src(fast, addrs(values), addrs(rstds), None if drs is None else addrs(drs))
+        if not fast:
+            _refuse_capture()
+        return _Src(fast, rows, addrs(values), addrs(rstds), None if drs is None else addrs(drs))
 
     def ptrs(self):
         """(v, r) as entry-point arguments: host arrays, or the device arrays' addresses."""
-        return (self.v, self.r) if self.fast else (self.v.data_ptr(), self.r.data_ptr())
+        return (self.v, self.r) if self.fast or self.rows else (self.v.data_ptr(), self.r.data_ptr())
 
     def dr_ptr(self):
-        return self.dr if self.fast else self.dr.data_ptr()
+        return self.dr if self.fast or self.rows else self.dr.data_ptr()
 
 
 def _read(src: _Src, n: int, q, dots, stored: bool, base, h0, beta: float, cbar, cols: int, c0, lam: float, out, tc,
           prob, next_prior, n_tok: int, d: int, dt: int, st) -> None:
     """One read forward from stored raw scores (stored: dots[i, tok]) or with the scores formed from the fp32 query q
-    and kept in dots: the row-layout kernels when src.fast, else the any-shape kernel. cols: n (cbar, c0 as the read
+    and kept in dots: the row-layout kernels when src.fast, else the unaligned-row or any-shape ones. cols: n (cbar, c0 as the read
     takes them) or n - 1 (the previous read's coefficients and prior, scaled by lam, the newest entry implied)."""
     v, r = src.ptrs()
     tail = (_p(base), _p(h0), float(beta), _p(cbar), cols, _p(c0), cols, float(lam), _inv_sqrt(d), _p(out), _p(tc),
             _p(prob), _p(next_prior), n_tok, d, dt, st)
     if not src.fast:
-        _run("read_fwd_any", v, r, n, None if stored else _p(q), _p(dots), n_tok, *tail)
+        _run("read_fwd_rows" if src.rows else "read_fwd_any", v, r, n, None if stored else _p(q), _p(dots), n_tok,
+             *tail)
     elif stored:
         _run("read_fwd", v, r, n, _p(dots), n_tok, *tail)
     else:
@@ -295,7 +311,7 @@ def _forward_impl(ctx, q, base, cbar, c0, srcs):
     grad = any(ctx.needs_input_grad)      # else no backward: the probabilities are not stored
     prob = torch.empty((n_tok, n), device=dev, dtype=torch.float32) if grad else None
     dots = torch.empty((n, n_tok), device=dev, dtype=torch.float32)
-    src = _Src.of(_fast(d, n, base_c, qc, *values), values, rstds, dev)
+    src = _Src.of(_fast(d, n, base_c, qc, *values), _rows(d, n), values, rstds, dev)
     _read(src, n, qc, dots, False, base_c, None, 0.0, cbar_c, n, c0c, 1.0, out, tc, prob, None, n_tok, d, dt, st)
     if grad:
         ctx.save_for_backward(qc, cbar_c, c0c, prob, dots, tc, *values, *rstds)
@@ -329,7 +345,7 @@ def _bwd1(src: _Src, n, g, gt, prob, dots, tc, cbar_c, c0c, dr_accum, wz, wz_str
             raise RuntimeError("delta_attnres HIP read: host source tables with rows the row-layout kernels refuse")
         _run("read_bwd1", *head, dq_part.stride(0), *tail)
     else:
-        _run("read_bwd1_any", *head, parts, dq_part.stride(0), *tail)
+        _run("read_bwd1_rows" if src.rows else "read_bwd1_any", *head, parts, dq_part.stride(0), *tail)
     if part is not None:
         return None, dcbar
     dq = torch.empty(d, device=dev, dtype=torch.float32) if dq is None else dq
@@ -354,13 +370,16 @@ def _backward_impl(ctx, g, gt, dv, accum):
     dr = torch.empty((n, n_tok), device=dev, dtype=torch.float32)
     wz = torch.empty((n, n_tok, 2), device=dev, dtype=torch.float32)
     fast = _fast(d, n, g, qc, *values, *dv)
-    src = _Src.of(fast, values, rstds, dev, drs=[dr[i] for i in range(n)])
+    src = _Src.of(fast, _rows(d, n), values, rstds, dev, drs=[dr[i] for i in range(n)])
     dq, dcbar = _bwd1(src, n, g, gt, prob, dots, tc, cbar_c, c0c, False, wz, n_tok, n_tok, d, dt, dev)
     for t in dv:
         if t.dtype != v0.dtype or not t.is_contiguous() or t.numel() != v0.numel():
             raise RuntimeError("delta_attnres HIP read: gradient buffers must match the sources")
     if fast:
         _run("read_bwd2_list", L.u64_array(t.data_ptr() for t in dv), n, int(bool(accum)), _p(g), _p(qc), _p(wz),
+             n_tok, n_tok, d, dt, _stream(dev))
+    elif src.rows:
+        _run("read_bwd2_list_rows", L.u64_array(t.data_ptr() for t in dv), n, int(bool(accum)), _p(g), _p(qc), _p(wz),
              n_tok, n_tok, d, dt, _stream(dev))
     else:
         dvt = _dev_addrs((t.data_ptr() for t in dv), dev)
@@ -530,14 +549,18 @@ class DattnStack:
     def src(self, n: int, *rows) -> _Src:
         """The stack's sources for a read of n of them (with the scale gradients' addresses once the backward state
         exists): the host tables for the row-layout kernels when they take the read (n <= MAX_SOURCES, the other
-        rows 16-byte aligned), else device arrays of the same addresses, made on first use."""
+        rows 16-byte aligned) and for the unaligned-row ones, else device arrays of the same addresses, made on first
+        use."""
         if self.fast_d and _fast(self.d, n, *rows):
             if self.src_fast is None or (self.src_fast.dr is None and self.drptr is not None):
-                self.src_fast = _Src(True, self.vptr, self.rptr, self.drptr)
+                self.src_fast = _Src(True, False, self.vptr, self.rptr, self.drptr)
             return self.src_fast
+        _refuse_capture()
+        if _rows(self.d, n):
+            return _Src(False, True, self.vptr, self.rptr, self.drptr)
         if self.src_any is None or (self.src_any.dr is None and self.dR is not None):
             dev = self.V.device
-            self.src_any = _Src(False, _dev_addrs(self.vptr, dev), _dev_addrs(self.rptr, dev),
+            self.src_any = _Src(False, False, _dev_addrs(self.vptr, dev), _dev_addrs(self.rptr, dev),
                                 None if self.dR is None else _dev_addrs(self.drptr, dev))
         return self.src_any
 
@@ -597,6 +620,9 @@ def _assemble(stack: DattnStack, s: int, gr):
             _dtype_code(v.dtype), _stream(v.device))
     if fast:
         _run("dv_assemble", *([L.u64_array(t) for t in tables] if tables else [None] * 3), *args)
+    elif _rows(stack.d, len(reads)):
+        _refuse_capture()
+        _run("dv_assemble_rows", *([L.u64_array(t) for t in tables] if tables else [None] * 3), *args)
     else:
         dev_tabs = [_dev_addrs(t, v.device) for t in tables] if tables else None
         _run("dv_assemble_any", *([t.data_ptr() for t in dev_tabs] if dev_tabs else [None] * 3), *args)
@@ -624,9 +650,9 @@ class _WriteDelta(torch.autograd.Function):
         out = _alias(stack.V, s)
         r = _alias(stack.R, s)
         V = stack.V
-        if (stack.fast_d and h.is_cuda and h.is_contiguous() and x.is_contiguous() and h.dtype == V.dtype == x.dtype
-                and h.numel() == x.numel() == stack.n_tok * stack.d and h.shape[-1] == stack.d
-                and _aligned(h) and _aligned(x)):
+        whole = (h.is_cuda and x.is_cuda and h.is_contiguous() and x.is_contiguous() and h.dtype == V.dtype == x.dtype
+                 and h.numel() == x.numel() == stack.n_tok * stack.d and h.shape[-1] == stack.d)
+        if whole and stack.fast_d and _aligned(h) and _aligned(x):
             nq, j_lo, dptr, jstride = 0, 0, None, stack.n_steps * stack.n_tok
             if stack.DOTS is not None:
                 nq = stack.Q.shape[0]
@@ -636,6 +662,10 @@ class _WriteDelta(torch.autograd.Function):
             _run("write_dots", _p(h), _p(x), _p(out), _p(r), _p(stack.Q), _p(stack.QB), nq, j_lo, _p(dptr),
                  stack.n_tok, stack.d, jstride, stack.eps, _dtype_code(V.dtype), _stream(V.device))
             stack.r_done[s] = True
+        elif whole and not stack.fast_d and h.shape == x.shape == V.shape[1:] and h.device == x.device == V.device:
+            _run("write_rows", _p(h), _p(x), _p(out), _p(r), stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype),
+                 _stream(V.device))
+            stack.r_done[s] = False           # the update has no scores (the reads form them online)
         else:
             torch.sub(h, x, out=out)
             _run("rstd_fwd", _p(out), _p(r), stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype), _stream(V.device))
@@ -892,6 +922,9 @@ class FusedCombineStk(torch.autograd.Function):
                         _stream(dev))
                 if stack.fast_d and _fast(d, len(gs), dh0, *gs):
                     _run("blend_sum", L.u64_array(x.data_ptr() for x in gs), *tail)
+                elif _rows(d, len(gs)):
+                    _refuse_capture()
+                    _run("blend_sum_rows", L.u64_array(x.data_ptr() for x in gs), *tail)
                 else:
                     gt_ = _dev_addrs((x.data_ptr() for x in gs), dev)
                     _run("blend_sum_any", gt_.data_ptr(), *tail)

@@ -1,0 +1,49 @@
+"""The unaligned-row kernels (8 <= d <= 8192, any width and alignment) at the edges of their layouts: the narrowest
+row, one element past and short of a vector, of a wave's 512 and 2048 elements, of the widest row, several waves per
+row; two and 64 sources (addresses by value), 65 and 300 (device arrays, with fewer rows per workgroup)."""
+import pytest
+import torch
+
+from gpu_helpers import DEV, err_rms, make
+from test_gpu_read import compare, run_hip, run_oracle
+from test_gpu_stack import check_chain, hip_chain
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,t,d,n", [(1, 70, 8, 3), (1, 70, 9, 2), (3, 11, 63, 64), (2, 9, 511, 5), (2, 9, 513, 6),
+                                     (1, 13, 2047, 4), (1, 13, 2049, 7), (1, 3, 8191, 5), (1, 6, 40, 300),
+                                     (1, 5, 1001, 65), (1, 2, 4097, 65)])
+def test_list_read_at_layout_edges(b, t, d, n):
+    """Forward and every gradient within 1e-5 x RMS of the exact read, the bar of every fp32 read."""
+    args = make(b, t, d, n, torch.float32, seed=7 * n + d)
+    print(f"case unaligned rows b{b} t{t} d{d} n{n}", flush=True)
+    e64 = compare(run_hip(d, n, args, True), run_oracle(d, n, args, True, dtype=torch.float64), err_rms)
+    assert max(e64.values()) <= 1e-5, e64
+
+
+@pytest.mark.parametrize("d", [9, 1001, 4099])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_chain_at_layout_edges(d, dtype):
+    """A stacked chain (the write, the update gradients, the blends' sum) to the chain bars."""
+    from loopback_amd.chain import ChainConfig
+    cfg = ChainConfig(f"rows-d{d}", d, 2, 3, 1, 67, dtype, True, q_std=0.5)
+    print(f"case unaligned chain d{d} {dtype}", flush=True)
+    h, g = hip_chain(cfg, "scores")
+    check_chain(h, g, cfg)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [3, 9, 130, 1001])
+def test_write_stores_the_scale_of_rstd(dtype, d):
+    """V = h - x as torch subtracts, R bitwise the scale kernel's (one summation order for both)."""
+    from loopback_amd import fused_dattn as FD
+    g = torch.Generator().manual_seed(d)
+    h, x = (torch.randn(1, 37, d, generator=g).to(dtype).to(DEV) for _ in range(2))
+    stack = FD.DattnStack(2, (1, 37, d), dtype, DEV)
+    print(f"case unaligned write d{d} {dtype}", flush=True)
+    with torch.no_grad():
+        v = stack.write(0, h, x)
+        r = FD.rstd(v, stack.eps)
+    torch.cuda.synchronize()
+    assert torch.equal(v, h - x) and torch.equal(stack.R[0], r.view_as(stack.R[0]))

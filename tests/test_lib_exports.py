@@ -191,3 +191,27 @@ def test_any_shape_argument_checks_before_launch(lib):
     assert L.ldr_blend_sum_any(p, 2, 0.5, 0, odd, 16, 100, 1, null) == -3
     assert L.ldr_blend_sum_any(p, 2, 0.5, 1, p, 0, 100, 1, null) == 0
     assert L.ldr_blend_sum_any(p, 2, 0.5, 5, p, 0, 100, 1, null) == -1
+
+
+def test_unaligned_row_argument_checks_before_launch(lib):
+    """The *_rows entry points take 8 <= d <= LDR_MAX_WIDTH and up to LDR_MAX_SOURCES sources from host tables at
+    element alignment, and refuse the rest before any launch."""
+    L, p, null = lib.LIB, 4096, None
+    tab = lambda n, a=4098: lib.u64_array([a] * n)
+    rd = lambda n, d, base=4098, n_tok=16, cols=None, a=4098: L.ldr_read_fwd_rows(
+        tab(n, a), tab(n, 4096), n, p, p, 16, base, null, 0.0, p, n if cols is None else cols, p,
+        n if cols is None else cols, 1.0, 0.1, 4098, p, p, null, n_tok, d, 1, null)
+    assert rd(0, 64) == -2 and rd(65, 64) == -2 and rd(2, 7) == -2 and rd(2, 8193) == -2
+    assert rd(2, 65, cols=4) == -1 and rd(2, 65, a=0) == -1
+    assert rd(2, 65, base=4097) == -3 and rd(2, 65, a=4097) == -3
+    assert rd(64, 1001, n_tok=0) == 0
+    dv = lambda m, d=100, v=4098, a=4098: L.ldr_dv_assemble_rows(tab(m, a), tab(m, 4096), tab(m, 4096), m, v, p, null,
+                                                                 null, 0.0, 0, 4098, null, 16, d, 1, null)
+    assert dv(65) == -2 and dv(2, d=7) == -2 and dv(2, v=4097) == -3 and dv(2, a=4097) == -3
+    assert L.ldr_read_bwd2_list_rows(tab(2, 4097), 2, 0, 4098, p, p, 16, 16, 100, 1, null) == -3
+    assert L.ldr_blend_sum_rows(tab(2), 2, 0.5, 0, 4098, 16, 4, 1, null) == -2
+    assert L.ldr_write_rows(4097, p, p, p, 16, 100, 1e-6, 1, null) == -3
+    # partial rows: a workgroup per CU before two rows per row slot, at most ldr_read_bwd1's
+    parts = lib.bwd1_rows_parts
+    assert parts(0, 2048) == 0 and parts(16, 8193) == 0 and parts(16, 7) == 0
+    assert [parts(t, 2048) for t in (1, 65, 1024, 2048, 4096, 16384)] == [1, 17, 256, 256, 512, 512]
