@@ -1067,40 +1067,42 @@ struct QTile {
   int nq;     // queries in the table
 };
 
-template <typename T, int NB>   // 16-bit updates; NB 16-query blocks scored (from block qt.b0); NB = 0: no scores
+// 16-bit updates; NB 16-query blocks scored (from block qt.b0; NB = 0: no scores), MB 16-token blocks per workgroup
+template <typename T, int NB, int MB>
 __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, const T* __restrict__ x,
                                                    T* __restrict__ v, float* __restrict__ r, QTile qt,
                                                    float* __restrict__ dots, int64_t n_tok, int d,
                                                    int64_t dots_jstride, float eps) {
   using AP = MfmaA<T>;
   constexpr int NBA = NB > 0 ? NB : 1;   // array extents
-  __shared__ f32x4_t s_part[4][WM_MB][NBA][64];
-  __shared__ float s_ss[4][WM_MB][16];
-  __shared__ uint4 s_v[4][WM_TT][WM_KC / 8 + 1];   // each wave's V tile of a chunk (a 16-byte pad per row)
+  constexpr int TT = 16 * MB;            // tokens per workgroup
+  __shared__ f32x4_t s_part[4][MB][NBA][64];
+  __shared__ float s_ss[4][MB][16];
+  __shared__ uint4 s_v[4][TT][WM_KC / 8 + 1];   // each wave's V tile of a chunk (a 16-byte pad per row)
   const int tid = (int)threadIdx.x, w = tid >> 6, l = tid & 63, row = l & 15, quad = l >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * WM_TT;
-  f32x4_t acc[WM_MB][NBA];
+  const int64_t t0 = (int64_t)blockIdx.x * TT;
+  f32x4_t acc[MB][NBA];
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[mb][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ss[WM_MB];
+  float ss[MB];
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb) ss[mb] = 0.f;
-  int64_t roff[WM_MB];
-  bool tok_ok[WM_MB];
+  for (int mb = 0; mb < MB; ++mb) ss[mb] = 0.f;
+  int64_t roff[MB];
+  bool tok_ok[MB];
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     const int64_t tok = t0 + 16 * mb + row;
     tok_ok[mb] = tok < n_tok;
     roff[mb] = (tok_ok[mb] ? tok : n_tok - 1) * (int64_t)d;
   }
   const int nchunks = (d + WM_KC - 1) / WM_KC;
   // a chunk's h and x rows: every 16-token block, the lane's two 8-column k-groups (clamped in bounds)
-  auto load_hx = [&](int c, uint4 (&hr)[WM_MB][2], uint4 (&xr)[WM_MB][2]) {
+  auto load_hx = [&](int c, uint4 (&hr)[MB][2], uint4 (&xr)[MB][2]) {
     const int col = c * WM_KC + quad * WM_QS;
 #pragma unroll
-    for (int mb = 0; mb < WM_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const int cc = col + WM_HS * hf < d ? col + WM_HS * hf : 0;
@@ -1108,7 +1110,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
         xr[mb][hf] = *reinterpret_cast<const uint4*>(x + roff[mb] + cc);
       }
   };
-  uint4 hr[WM_MB][2], xr[WM_MB][2];
+  uint4 hr[MB][2], xr[MB][2];
   if (w < nchunks) load_hx(w, hr, xr);
   for (int c = w; c < nchunks; c += 4) {   // wave-uniform trip count
     const int col = c * WM_KC + quad * WM_QS;
@@ -1129,15 +1131,15 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
         for (int hf = 0; hf < 2; ++hf)
           qv[p][b][hf] = qt.qt[((((int64_t)c * qt.nbq + qt.b0 + b) * 3 + p) * 2 + hf) * 64 + l];
 
-    uint4 hc[WM_MB][2], xc[WM_MB][2];   // this chunk's rows; the next chunk's are requested now
+    uint4 hc[MB][2], xc[MB][2];   // this chunk's rows; the next chunk's are requested now
 #pragma unroll
-    for (int mb = 0; mb < WM_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) { hc[mb][hf] = hr[mb][hf]; xc[mb][hf] = xr[mb][hf]; }
     if (c + 4 < nchunks) load_hx(c + 4, hr, xr);   // uniform branch
-    uint4 va[WM_MB][2][AP::NP];
+    uint4 va[MB][2][AP::NP];
 #pragma unroll
-    for (int mb = 0; mb < WM_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         float hv[8], xv[8], vv[8];
@@ -1158,7 +1160,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
       }
     wave_lds_sync();
 #pragma unroll
-    for (int k = 0; k < WM_TT * 8 / 64; ++k) {   // 8 lanes per token row
+    for (int k = 0; k < TT * 8 / 64; ++k) {   // 8 lanes per token row
       const int e = l + 64 * k, t = e >> 3, u8 = e & 7;
       const int64_t tok = t0 + t;
       const int col8 = c * WM_KC + 8 * u8;
@@ -1176,7 +1178,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
 #pragma unroll
-          for (int mb = 0; mb < WM_MB; ++mb)   // (columns past d: zero operands on both sides)
+          for (int mb = 0; mb < MB; ++mb)   // (columns past d: zero operands on both sides)
 #pragma unroll
             for (int a = 0; a < AP::NP; ++a)
               acc[mb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(va[mb][hf][a]), as_bf16x8(qv[p][b][hf]),
@@ -1184,7 +1186,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
         }
   }
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     ss[mb] += __shfl_xor(ss[mb], 16, 64);
     ss[mb] += __shfl_xor(ss[mb], 32, 64);
     if (quad == 0) s_ss[w][mb][row] = ss[mb];
@@ -1192,14 +1194,14 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
     for (int b = 0; b < NB; ++b) s_part[w][mb][b][l] = acc[mb][b];
   }
   __syncthreads();
-  if (tid < 16 * WM_MB) {
+  if (tid < 16 * MB) {
     const int mb = tid >> 4, rr = tid & 15;
     const float tot = ((s_ss[0][mb][rr] + s_ss[1][mb][rr]) + s_ss[2][mb][rr]) + s_ss[3][mb][rr];
     const int64_t tok = t0 + tid;
     if (tok < n_tok) r[tok] = rsqrtf(tot / (float)d + eps);
   }
   if constexpr (NB > 0) {   // the scores (NB = 0 writes none)
-    for (int e = tid; e < WM_MB * NB * 64; e += WG) {
+    for (int e = tid; e < MB * NB * 64; e += WG) {
       const int mb = e / (NB * 64), rem = e - mb * NB * 64, b = rem >> 6, ll = rem & 63;
       const f32x4_t sum = ((s_part[0][mb][b][ll] + s_part[1][mb][b][ll]) + s_part[2][mb][b][ll]) + s_part[3][mb][b][ll];
       const int jj = 16 * (qt.b0 + b) + (ll & 15);   // the query; dots points at query j_lo's slice
@@ -1217,50 +1219,51 @@ __global__ __launch_bounds__(WG) void k_write_mfma(const T* __restrict__ h, cons
 // 512-byte row segments (32 lanes per row), stores V row-major and puts it in an LDS tile; then each wave runs the
 // matrix-core product of its 64-column quarter (chunk 4 step + w, as k_write_mfma's chunks) on the tile. The chunk
 // order per wave, the operands and the order of every sum are k_write_mfma's: V, R and the scores are its bits.
-template <typename T, int NB>
+template <typename T, int NB, int MB>
 __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, const T* __restrict__ x,
                                                    T* __restrict__ v, float* __restrict__ r, QTile qt,
                                                    float* __restrict__ dots, int64_t n_tok, int d,
                                                    int64_t dots_jstride, float eps) {
-  static_assert(WM_MB == 4, "k_write_rows: its 4 waves x 16 rows are the workgroup's 64 tokens");
   using AP = MfmaA<T>;
   constexpr int NBA = NB > 0 ? NB : 1;
   constexpr int KS = 4 * WM_KC;   // columns per step
-  __shared__ f32x4_t s_part[4][WM_MB][NBA][64];
-  __shared__ float s_ss[4][WM_MB][16];
+  constexpr int TT = 16 * MB, RI = 2 * MB;   // tokens per workgroup, row loads per lane
+  constexpr int DEPTH = MB == 4 ? WM_DEPTH : 3;   // steps of rows in flight (small tiles: registers for three)
+  __shared__ f32x4_t s_part[4][MB][NBA][64];
+  __shared__ float s_ss[4][MB][16];
   // the step's V tile (a 16-byte pad per row); with WM_DBUF two tiles alternate between steps, so a step needs one
   // barrier (its tile is written, then read; the next step writes the other tile)
-  __shared__ uint4 s_a[WM_DBUF ? 2 : 1][WM_TT][KS / 8 + 1];
+  __shared__ uint4 s_a[WM_DBUF ? 2 : 1][TT][KS / 8 + 1];
   const int tid = (int)threadIdx.x, w = tid >> 6, l = tid & 63, row = l & 15, quad = l >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * WM_TT;
-  f32x4_t acc[WM_MB][NBA];
+  const int64_t t0 = (int64_t)blockIdx.x * TT;
+  f32x4_t acc[MB][NBA];
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[mb][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ss[WM_MB];
+  float ss[MB];
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb) ss[mb] = 0.f;
-  // this lane's rows in the streaming layout: 16 w + 2 i + (l / 32), i < 8, vector column l % 32 of the step
+  for (int mb = 0; mb < MB; ++mb) ss[mb] = 0.f;
+  // this lane's rows in the streaming layout: 4 MB w + 2 i + (l / 32), i < RI, vector column l % 32 of the step
   const int lr = l & 31, lh = l >> 5;
-  int64_t rof[8];
-  bool rok[8];
+  int64_t rof[RI];
+  bool rok[RI];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int64_t tok = t0 + 16 * w + 2 * i + lh;
+  for (int i = 0; i < RI; ++i) {
+    const int64_t tok = t0 + 4 * MB * w + 2 * i + lh;
     rok[i] = tok < n_tok;
     rof[i] = (rok[i] ? tok : n_tok - 1) * (int64_t)d;
   }
-  auto load_rows = [&](int st, uint4 (&hr)[8], uint4 (&xr)[8]) {
+  auto load_rows = [&](int st, uint4 (&hr)[RI], uint4 (&xr)[RI]) {
     const int col = st * KS + lr * 8;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < RI; ++i) {
       hr[i] = ld_nt16(h + rof[i] + col);   // non-temporal: see ld_nt16
       xr[i] = *reinterpret_cast<const uint4*>(x + rof[i] + col);
     }
   };
   const int nsteps = d / KS;
-  // one 256-column step; its rows arrive in (hb, xb), which then take the rows of step st + WM_DEPTH: WM_DEPTH steps
+  // one 256-column step; its rows arrive in (hb, xb), which then take the rows of step st + DEPTH: DEPTH steps
   // of rows are in flight while a step is worked on
   // the query parts of this wave's chunk of step st (cache-resident)
   auto load_q = [&](int st, uint4 (&qv)[3][NBA][2]) {
@@ -1275,19 +1278,19 @@ __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, cons
   };
   uint4 qcur[3][NBA][2], qnext[3][NBA][2];   // WM_QPF: the next step's parts are requested a step ahead
   if (WM_QPF && NB > 0) load_q(0, qcur);
-  auto step = [&](int st, uint4 (&hb)[8], uint4 (&xb)[8]) {
+  auto step = [&](int st, uint4 (&hb)[RI], uint4 (&xb)[RI]) {
     uint4 (&qv)[3][NBA][2] = qcur;
     if (NB > 0) {
       if (!WM_QPF) load_q(st, qcur);
       else if (st + 1 < nsteps) load_q(st + 1, qnext);
     }
     auto& tile = s_a[WM_DBUF ? (st & 1) : 0];
-    uint4 hc[8], xc[8];   // this step's rows; the buffer now takes the rows WM_DEPTH steps ahead
+    uint4 hc[RI], xc[RI];   // this step's rows; the buffer now takes the rows DEPTH steps ahead
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { hc[i] = hb[i]; xc[i] = xb[i]; }
-    if (st + WM_DEPTH < nsteps) load_rows(st + WM_DEPTH, hb, xb);   // uniform branch
+    for (int i = 0; i < RI; ++i) { hc[i] = hb[i]; xc[i] = xb[i]; }
+    if (st + DEPTH < nsteps) load_rows(st + DEPTH, hb, xb);   // uniform branch
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < RI; ++i) {
       float hv[8], xv[8], vv[8];
       IO<T>::unpack(typename IO<T>::Raw{hc[i]}, hv);
       IO<T>::unpack(typename IO<T>::Raw{xc[i]}, xv);
@@ -1299,12 +1302,12 @@ __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, cons
       const u32x4 u{ru.x, ru.y, ru.z, ru.w};
       // non-temporal: the read that follows streams V[s] with its other sources
       if (rok[i]) __builtin_nontemporal_store(u, reinterpret_cast<u32x4*>(v + rof[i] + st * KS + lr * 8));
-      tile[16 * w + 2 * i + lh][lr] = make_uint4(u.x, u.y, u.z, u.w);
+      tile[4 * MB * w + 2 * i + lh][lr] = make_uint4(u.x, u.y, u.z, u.w);
     }
     __syncthreads();
-    uint4 va[WM_MB][2][AP::NP];
+    uint4 va[MB][2][AP::NP];
 #pragma unroll
-    for (int mb = 0; mb < WM_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const uint4 u = tile[16 * mb + row][w * (WM_KC / 8) + quad + 4 * hf];
@@ -1322,7 +1325,7 @@ __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, cons
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
 #pragma unroll
-          for (int mb = 0; mb < WM_MB; ++mb)
+          for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int a = 0; a < AP::NP; ++a)
               acc[mb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(va[mb][hf][a]), as_bf16x8(qv[p][b][hf]),
@@ -1337,17 +1340,17 @@ __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, cons
           for (int hf = 0; hf < 2; ++hf) qcur[p][b][hf] = qnext[p][b][hf];
     }
   };
-  uint4 hr[WM_DEPTH][8], xr[WM_DEPTH][8];
+  uint4 hr[DEPTH][RI], xr[DEPTH][RI];
 #pragma unroll
-  for (int k = 0; k < WM_DEPTH; ++k)
+  for (int k = 0; k < DEPTH; ++k)
     if (k < nsteps) load_rows(k, hr[k], xr[k]);
-  for (int st = 0; st < nsteps; st += WM_DEPTH) {
+  for (int st = 0; st < nsteps; st += DEPTH) {
 #pragma unroll
-    for (int k = 0; k < WM_DEPTH; ++k)
+    for (int k = 0; k < DEPTH; ++k)
       if (st + k < nsteps) step(st + k, hr[k], xr[k]);   // uniform branch; the buffer index is static
   }
 #pragma unroll
-  for (int mb = 0; mb < WM_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     ss[mb] += __shfl_xor(ss[mb], 16, 64);
     ss[mb] += __shfl_xor(ss[mb], 32, 64);
     if (quad == 0) s_ss[w][mb][row] = ss[mb];
@@ -1355,14 +1358,14 @@ __global__ __launch_bounds__(WG) void k_write_rows(const T* __restrict__ h, cons
     for (int b = 0; b < NB; ++b) s_part[w][mb][b][l] = acc[mb][b];
   }
   __syncthreads();
-  if (tid < 16 * WM_MB) {
+  if (tid < 16 * MB) {
     const int mb = tid >> 4, rr = tid & 15;
     const float tot = ((s_ss[0][mb][rr] + s_ss[1][mb][rr]) + s_ss[2][mb][rr]) + s_ss[3][mb][rr];
     const int64_t tok = t0 + tid;
     if (tok < n_tok) r[tok] = rsqrtf(tot / (float)d + eps);
   }
   if constexpr (NB > 0) {   // the scores (NB = 0 writes none)
-    for (int e = tid; e < WM_MB * NB * 64; e += WG) {
+    for (int e = tid; e < MB * NB * 64; e += WG) {
       const int mb = e / (NB * 64), rem = e - mb * NB * 64, b = rem >> 6, ll = rem & 63;
       const f32x4_t sum = ((s_part[0][mb][b][ll] + s_part[1][mb][b][ll]) + s_part[2][mb][b][ll]) + s_part[3][mb][b][ll];
       const int jj = 16 * (qt.b0 + b) + (ll & 15);   // the query; dots points at query j_lo's slice
@@ -1401,40 +1404,41 @@ __device__ __forceinline__ void split3(const float (&e)[8], uint4 (&a)[3]) {
   }
 }
 
-template <int NB>   // NB 16-query blocks scored (from block qt.b0); NB = 0: no scores
+template <int NB, int MB>   // as k_write_mfma
 __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h, const float* __restrict__ x,
                                                      float* __restrict__ v, float* __restrict__ r, QTile qt,
                                                      float* __restrict__ dots, int64_t n_tok, int d,
                                                      int64_t dots_jstride, float eps) {
   constexpr int NBA = NB > 0 ? NB : 1;
-  __shared__ f32x4_t s_part[4][W32_MB][NBA][64];
-  __shared__ float s_ss[4][W32_MB][16];
-  __shared__ float4 s_v[4][W32_TT][WM_KC / 4 + 1];   // each wave's V tile of a chunk (a 16-byte pad per row)
+  constexpr int TT = 16 * MB;
+  __shared__ f32x4_t s_part[4][MB][NBA][64];
+  __shared__ float s_ss[4][MB][16];
+  __shared__ float4 s_v[4][TT][WM_KC / 4 + 1];   // each wave's V tile of a chunk (a 16-byte pad per row)
   const int tid = (int)threadIdx.x, w = tid >> 6, l = tid & 63, row = l & 15, quad = l >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * W32_TT;
-  f32x4_t acc[W32_MB][NBA];
+  const int64_t t0 = (int64_t)blockIdx.x * TT;
+  f32x4_t acc[MB][NBA];
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[mb][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ss[W32_MB];
+  float ss[MB];
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb) ss[mb] = 0.f;
-  int64_t roff[W32_MB];
-  bool tok_ok[W32_MB];
+  for (int mb = 0; mb < MB; ++mb) ss[mb] = 0.f;
+  int64_t roff[MB];
+  bool tok_ok[MB];
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     const int64_t tok = t0 + 16 * mb + row;
     tok_ok[mb] = tok < n_tok;
     roff[mb] = (tok_ok[mb] ? tok : n_tok - 1) * (int64_t)d;
   }
   const int nchunks = (d + WM_KC - 1) / WM_KC;
   using Raw = IO<float>::Raw;
-  Raw hr[W32_MB][2], xr[W32_MB][2];
+  Raw hr[MB][2], xr[MB][2];
   auto load_hx = [&](int c) {   // a chunk's h and x rows: every 16-token block, the lane's two k-groups
     const int col = c * WM_KC + quad * WM_QS;
 #pragma unroll
-    for (int mb = 0; mb < W32_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const int cc = col + WM_HS * hf < d ? col + WM_HS * hf : 0;
@@ -1453,9 +1457,9 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf)
           qv[p][b][hf] = qt.qt[((((int64_t)c * qt.nbq + qt.b0 + b) * 3 + p) * 2 + hf) * 64 + l];
-    uint4 va[W32_MB][2][3];
+    uint4 va[MB][2][3];
 #pragma unroll
-    for (int mb = 0; mb < W32_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         float hv[8], xv[8], vv[8];
@@ -1474,7 +1478,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
     if (c + 4 < nchunks) load_hx(c + 4);   // uniform branch; the registers are free again
     wave_lds_sync();
 #pragma unroll
-    for (int k = 0; k < W32_TT * (WM_KC / 4) / 64; ++k) {   // 16 lanes per token row
+    for (int k = 0; k < TT * (WM_KC / 4) / 64; ++k) {   // 16 lanes per token row
       const int e = l + 64 * k, t = e >> 4, u = e & 15;
       const int64_t tok = t0 + t;
       const int col4 = c * WM_KC + 4 * u;
@@ -1491,7 +1495,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-        for (int mb = 0; mb < W32_MB; ++mb)   // a_i q_j, i + j <= 2 (columns past d: zero operands on both sides)
+        for (int mb = 0; mb < MB; ++mb)   // a_i q_j, i + j <= 2 (columns past d: zero operands on both sides)
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1500,7 +1504,7 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
                                                                    acc[mb][b], 0, 0, 0);
   }
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     ss[mb] += __shfl_xor(ss[mb], 16, 64);
     ss[mb] += __shfl_xor(ss[mb], 32, 64);
     if (quad == 0) s_ss[w][mb][row] = ss[mb];
@@ -1508,14 +1512,14 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
     for (int b = 0; b < NB; ++b) s_part[w][mb][b][l] = acc[mb][b];
   }
   __syncthreads();
-  if (tid < 16 * W32_MB) {
+  if (tid < 16 * MB) {
     const int mb = tid >> 4, rr = tid & 15;
     const float tot = ((s_ss[0][mb][rr] + s_ss[1][mb][rr]) + s_ss[2][mb][rr]) + s_ss[3][mb][rr];
     const int64_t tok = t0 + tid;
     if (tok < n_tok) r[tok] = rsqrtf(tot / (float)d + eps);
   }
   if constexpr (NB > 0) {   // the scores (NB = 0 writes none)
-    for (int e = tid; e < W32_MB * NB * 64; e += WG) {
+    for (int e = tid; e < MB * NB * 64; e += WG) {
       const int mb = e / (NB * 64), rem = e - mb * NB * 64, b = rem >> 6, ll = rem & 63;
       const f32x4_t sum = ((s_part[0][mb][b][ll] + s_part[1][mb][b][ll]) + s_part[2][mb][b][ll]) + s_part[3][mb][b][ll];
       const int jj = 16 * (qt.b0 + b) + (ll & 15);   // the query; dots points at query j_lo's slice
@@ -1534,34 +1538,35 @@ __global__ __launch_bounds__(WG) void k_write_mfma32(const float* __restrict__ h
 // two rows (k_write_mfma32's layout strides 32 bytes between lanes); V is stored row-major from there and put in an
 // LDS tile, from which each wave takes its 64-column chunk of the step in k_write_mfma32's layout. The chunks per
 // wave and the order of every sum are k_write_mfma32's, so V, R and the scores are its bits.
-template <int NB>   // NB 16-query blocks scored (from block qt.b0); NB = 0: no scores
+template <int NB, int MB>   // as k_write_mfma
 __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h, const float* __restrict__ x,
                                                      float* __restrict__ v, float* __restrict__ r, QTile qt,
                                                      float* __restrict__ dots, int64_t n_tok, int d,
                                                      int64_t dots_jstride, float eps) {
   constexpr int NBA = NB > 0 ? NB : 1;
+  constexpr int TT = 16 * MB;
   constexpr int KS = 4 * WM_KC;   // columns per step
-  __shared__ f32x4_t s_part[4][W32_MB][NBA][64];
-  __shared__ float s_ss[4][W32_MB][16];
-  __shared__ float4 s_a[W32_TT][KS / 4 + 1];   // the step's V tile (a 16-byte pad per row)
+  __shared__ f32x4_t s_part[4][MB][NBA][64];
+  __shared__ float s_ss[4][MB][16];
+  __shared__ float4 s_a[TT][KS / 4 + 1];   // the step's V tile (a 16-byte pad per row)
   const int tid = (int)threadIdx.x, w = tid >> 6, l = tid & 63, row = l & 15, quad = l >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * W32_TT;
-  f32x4_t acc[W32_MB][NBA];
+  const int64_t t0 = (int64_t)blockIdx.x * TT;
+  f32x4_t acc[MB][NBA];
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[mb][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ss[W32_MB];
+  float ss[MB];
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb) ss[mb] = 0.f;
-  // this lane's rows in the streaming layout: 8 w + 2 i + (l / 32), i < 4; float4 columns l % 32 and 32 + l % 32
-  constexpr int RI = W32_TT / 8;
+  for (int mb = 0; mb < MB; ++mb) ss[mb] = 0.f;
+  // this lane's rows in the streaming layout: 4 MB w + 2 i + (l / 32), i < RI; float4 columns l % 32 and 32 + l % 32
+  constexpr int RI = TT / 8;
   const int lr = l & 31, lh = l >> 5;
   int64_t rof[RI];
   bool rok[RI];
 #pragma unroll
   for (int i = 0; i < RI; ++i) {
-    const int64_t tok = t0 + 8 * w + 2 * i + lh;
+    const int64_t tok = t0 + 4 * MB * w + 2 * i + lh;
     rok[i] = tok < n_tok;
     rof[i] = (rok[i] ? tok : n_tok - 1) * (int64_t)d;
   }
@@ -1607,12 +1612,12 @@ __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h
           __builtin_nontemporal_store(u32x4{__float_as_uint(vv.x), __float_as_uint(vv.y), __float_as_uint(vv.z),
                                             __float_as_uint(vv.w)},
                                       reinterpret_cast<u32x4*>(v + rof[i] + st * KS + lr * 4 + 128 * hh));
-        s_a[8 * w + 2 * i + lh][lr + 32 * hh] = vv;
+        s_a[4 * MB * w + 2 * i + lh][lr + 32 * hh] = vv;
       }
     __syncthreads();
-    uint4 va[W32_MB][2][3];
+    uint4 va[MB][2][3];
 #pragma unroll
-    for (int mb = 0; mb < W32_MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const int u4 = 16 * w + 2 * quad + 8 * hf;   // k_write_mfma32's columns 8 quad + 32 hf of chunk c
@@ -1628,7 +1633,7 @@ __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-        for (int mb = 0; mb < W32_MB; ++mb)   // a_i q_j, i + j <= 2, in k_write_mfma32's order
+        for (int mb = 0; mb < MB; ++mb)   // a_i q_j, i + j <= 2, in k_write_mfma32's order
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1637,7 +1642,7 @@ __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h
                                                                    acc[mb][b], 0, 0, 0);
   }
 #pragma unroll
-  for (int mb = 0; mb < W32_MB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     ss[mb] += __shfl_xor(ss[mb], 16, 64);
     ss[mb] += __shfl_xor(ss[mb], 32, 64);
     if (quad == 0) s_ss[w][mb][row] = ss[mb];
@@ -1645,14 +1650,14 @@ __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h
     for (int b = 0; b < NB; ++b) s_part[w][mb][b][l] = acc[mb][b];
   }
   __syncthreads();
-  if (tid < 16 * W32_MB) {
+  if (tid < 16 * MB) {
     const int mb = tid >> 4, rr = tid & 15;
     const float tot = ((s_ss[0][mb][rr] + s_ss[1][mb][rr]) + s_ss[2][mb][rr]) + s_ss[3][mb][rr];
     const int64_t tok = t0 + tid;
     if (tok < n_tok) r[tok] = rsqrtf(tot / (float)d + eps);
   }
   if constexpr (NB > 0) {   // the scores (NB = 0 writes none)
-    for (int e = tid; e < W32_MB * NB * 64; e += WG) {
+    for (int e = tid; e < MB * NB * 64; e += WG) {
       const int mb = e / (NB * 64), rem = e - mb * NB * 64, b = rem >> 6, ll = rem & 63;
       const f32x4_t sum = ((s_part[0][mb][b][ll] + s_part[1][mb][b][ll]) + s_part[2][mb][b][ll]) + s_part[3][mb][b][ll];
       const int jj = 16 * (qt.b0 + b) + (ll & 15);   // the query; dots points at query j_lo's slice
@@ -1667,23 +1672,22 @@ __global__ __launch_bounds__(WG) void k_write_rows32(const float* __restrict__ h
 }
 
 // the fp32 write kernel: rows streamed whole when d is whole 256-column steps (LDR_W32_ROWS), else the matrix
-// cores' layout; both give the same bits
-template <int NB>
+// cores' layout; both, and every MB, give the same bits
+template <int NB, int MB>
 auto write32_kernel(bool rows) {
   if constexpr (LDR_W32_ROWS) {
-    if (rows) return &k_write_rows32<NB>;
+    if (rows) return &k_write_rows32<NB, MB>;
   }
-  return &k_write_mfma32<NB>;
+  return &k_write_mfma32<NB, MB>;
 }
 
-// the write kernel for bf16 updates: rows streamed whole when d is whole 256-column steps (and the build keeps
-// 64-token workgroups), else the matrix cores' layout; both give the same bits
-template <typename T, int NB>
+// the write kernel for 16-bit updates, the same way
+template <typename T, int NB, int MB>
 auto write_kernel(bool rows) {
   if constexpr (WM_ROWS) {
-    if (rows) return &k_write_rows<T, NB>;
+    if (rows) return &k_write_rows<T, NB, MB>;
   }
-  return &k_write_mfma<T, NB>;
+  return &k_write_mfma<T, NB, MB>;
 }
 
 // the three bf16 parts of fp32 query values, q = hi + mid + lo, into the operand table (QTile's layout)
@@ -1803,7 +1807,7 @@ __global__ __launch_bounds__(NTH) void k_read_fwd(SrcTab src, int n, const float
                                                  Coef cf, float inv, T* __restrict__ out, float* __restrict__ tc,
                                                  float* __restrict__ prob, float* __restrict__ next_prior,
                                                  int64_t n_tok, int d, int tpr,
-                                                 int tt) {
+                                                 int tt, int lpt) {   // lpt: lanes per token in the softmax
   // the logits [i][t] during a tile's prologue; with STAGE, then the tile's output rows, written out together at
   // its end (the launch picks STAGE when the tile's rows fit)
   constexpr int STAGE_BYTES = NTH > WG ? RF_BIG_STAGE : RF_STAGE_BYTES;
@@ -1855,7 +1859,6 @@ __global__ __launch_bounds__(NTH) void k_read_fwd(SrcTab src, int n, const float
   load_prior(cf, n, s_c0, s_lc, &s_M, src, s_rp, dots);
   const float M = s_M;
   if (next_prior && blockIdx.x == 0 && tid < n) next_prior[tid] = s_c0[tid];
-  const int lpt = NTH / tt;   // lanes per token in the softmax
   const int ns = (n + lpt - 1) / lpt;
   if (tid < lpt) {   // p0 = softmax(lc), a per-read constant: once, by the lanes of one token
     float p0[8];
@@ -1880,7 +1883,8 @@ __global__ __launch_bounds__(NTH) void k_read_fwd(SrcTab src, int n, const float
     }
     __syncthreads();
     {
-      const int t = tid / lpt, j = tid - t * lpt;
+      const int tl = tid / lpt, j = tid - tl * lpt;
+      const int t = min(tl, tt - 1);   // a tile of fewer tokens than lpt lanes each cover: the others idle along
       const int64_t tok = t0 + t;
       float ps[8];
 #pragma unroll
@@ -1892,7 +1896,7 @@ __global__ __launch_bounds__(NTH) void k_read_fwd(SrcTab src, int n, const float
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
         const int i = j + m * lpt;
-        if (i < n) {
+        if (i < n && tl < tt) {
           const float tcv = s_c0[i] + M * (ps[m] - s_p0[i]);
           s_w[t * SP + i] = tcv - s_w[t * SP + i];
           if (tok < n_tok) {
@@ -2602,13 +2606,16 @@ template <typename T> constexpr int as_jb() { return std::is_same<T, float>::val
 // to the running gradient in T, in table order, then the scale's term rounded and added -- the roundings of the list
 // layout, whose per-read gradients autograd adds in backward order (the host orders the table so) -- instead of one
 // fp32 sum rounded once.
-template <typename T, int VPT, bool ADD_LAST, bool PER_READ>
+// SMALL (few tokens: the launch is bound by the latency of its chain of reads, not by bandwidth): one row per lane and
+// the rows of four reads in flight together. Taken while the large tiles would not reach every CU: 512 rows of 2048
+// bf16 13.8 -> 10.7 us per launch (8 reads on average), 128 rows of 768 8.8 -> 6.6; level from there on.
+template <typename T, int VPT, bool ADD_LAST, bool PER_READ, bool SMALL>
 __global__ __launch_bounds__(WG) void k_dv_assemble(AsmTab tab, int m, const T* __restrict__ vsrc,
                                                     const float* __restrict__ r, const float* __restrict__ gr,
                                                     const T* __restrict__ add, float add_beta,
                                                     T* __restrict__ dv, T* __restrict__ dv_neg, int64_t n_tok, int d,
                                                     int tpr) {
-  constexpr int AS_RB = as_rb(VPT, std::is_same<T, float>::value);
+  constexpr int AS_RB = SMALL ? 1 : as_rb(VPT, std::is_same<T, float>::value);
   const Rows R(d, tpr);
   const int64_t rows_per_tile = (int64_t)R.rpw * AS_RB;
   const int64_t tiles = (n_tok + rows_per_tile - 1) / rows_per_tile;
@@ -2673,7 +2680,7 @@ __global__ __launch_bounds__(WG) void k_dv_assemble(AsmTab tab, int m, const T* 
     };
     const int mm = ADD_LAST ? m - 1 : m;
     int j = 0;
-    constexpr int JB = as_jb<T>();
+    constexpr int JB = SMALL ? 4 : as_jb<T>();
     for (; j + JB <= mm; j += JB) batch(j, std::integral_constant<int, JB>());
     for (; j < mm; ++j) batch(j, std::integral_constant<int, 1>());
     typename IO<T>::Raw last[AS_RB][VPT];   // ADD_LAST: the last read's rows, kept for the added gradient
@@ -3688,6 +3695,7 @@ inline int64_t elt_bytes(int dt) { return dt == LDR_F32 ? 4 : 2; }
 inline bool tok_ptr(const void* p, int64_t n_tok) { return p != nullptr || n_tok == 0; }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline unsigned grid_of(int64_t blocks, int64_t cap) { return (unsigned)(blocks < 1 ? 1 : (blocks < cap ? blocks : cap)); }
+constexpr int64_t CUS = 256;   // compute units of the GPU
 inline int launched() { return (int)hipGetLastError(); }
 
 // tokens per tile of the tiled kernels: at least one row per row slot
@@ -3994,6 +4002,13 @@ int ldr_rstd_bwd(const void* x, const float* r, const float* gr, void* gx, int64
   return launched();
 }
 
+// 16-token workgroups while the large ones would not reach every CU: a workgroup's steps are then bound by the latency
+// of its own loads, and idle CUs load nothing. Per launch scoring 16 queries: 4096 rows of 1024 bf16 12.4 us in 64
+// workgroups, 7.6 in 256; 512 rows of 2048 19.7 and 8.6; 128 rows of 768 8.9 and 4.9; 4096 rows of 1024 fp32 13.9 and
+// 13.0. Where the large ones reach every CU they stay: each query-part load serves their four (fp32: two) blocks, and
+// 32-token workgroups were 7 % slower there.
+static inline bool write_small(int64_t n_tok, int64_t tile) { return cdiv(n_tok, tile) < CUS; }
+
 int ldr_write_dots(const void* h, const void* x, void* v_out, float* r_out, const float* q, const void* qb,
                    int64_t nq, int64_t j_lo, float* dots, int64_t n_tok, int64_t d, int64_t dots_jstride, float eps,
                    int dtype, void* stream) {
@@ -4015,13 +4030,14 @@ int ldr_write_dots(const void* h, const void* x, void* v_out, float* r_out, cons
     const int nbq = (int)query_blocks(nq), b0 = (int)(j_lo / 16);
     const QTile qtl{static_cast<const uint4*>(qb), nbq, b0, (int)j_lo, (int)nq};
     const int nb = scores ? nbq - b0 : 0;
-    const unsigned grid = (unsigned)cdiv(n_tok, W32_TT);
+    const bool small = write_small(n_tok, W32_TT);
+    const unsigned grid = (unsigned)cdiv(n_tok, small ? 16 : W32_TT);
     const float* hf = static_cast<const float*>(h);
     const float* xf = static_cast<const float*>(x);
     float* vf = static_cast<float*>(v_out);
     const bool rows = d % (4 * WM_KC) == 0;   // rows streamed whole when d is whole steps
 #define LDR_W32_LAUNCH(NBV)                                                                                   \
-  hipLaunchKernelGGL((write32_kernel<NBV>(rows)), dim3(grid), dim3(WG), 0, st, hf, xf, vf, r_out, qtl, dots, n_tok, \
+  hipLaunchKernelGGL((small ? write32_kernel<NBV, 1>(rows) : write32_kernel<NBV, W32_MB>(rows)), dim3(grid), dim3(WG), 0, st, hf, xf, vf, r_out, qtl, dots, n_tok, \
                      (int)d, dots_jstride, eps)
     switch (nb) {
       case 0: LDR_W32_LAUNCH(0); break;
@@ -4032,18 +4048,19 @@ int ldr_write_dots(const void* h, const void* x, void* v_out, float* r_out, cons
     }
 #undef LDR_W32_LAUNCH
   } else if (!valu) {   // matrix-core scores from the operand table of the nq queries (bf16 and fp16 updates)
-    const unsigned grid = (unsigned)cdiv(n_tok, WM_TT);
+    const bool small = write_small(n_tok, WM_TT);
+    const unsigned grid = (unsigned)cdiv(n_tok, small ? 16 : WM_TT);
     const int nbq = (int)query_blocks(nq), b0 = (int)(j_lo / 16);
     const QTile qtl{static_cast<const uint4*>(qb), nbq, b0, (int)j_lo, (int)nq};
     const int nb = scores ? nbq - b0 : 0;
     const bool rows = d % (4 * WM_KC) == 0;   // rows streamed whole when d is whole steps
 #define LDR_WM_LAUNCH(NBV)                                                                                        \
   if (dtype == LDR_BF16)                                                                                          \
-    hipLaunchKernelGGL((write_kernel<bf16_t, NBV>(rows)), dim3(grid), dim3(WG), 0, st,                            \
+    hipLaunchKernelGGL((small ? write_kernel<bf16_t, NBV, 1>(rows) : write_kernel<bf16_t, NBV, WM_MB>(rows)), dim3(grid), dim3(WG), 0, st,                            \
                        static_cast<const bf16_t*>(h), static_cast<const bf16_t*>(x), static_cast<bf16_t*>(v_out), \
                        r_out, qtl, dots, n_tok, (int)d, dots_jstride, eps);                                       \
   else                                                                                                            \
-    hipLaunchKernelGGL((write_kernel<_Float16, NBV>(rows)), dim3(grid), dim3(WG), 0, st,                          \
+    hipLaunchKernelGGL((small ? write_kernel<_Float16, NBV, 1>(rows) : write_kernel<_Float16, NBV, WM_MB>(rows)), dim3(grid), dim3(WG), 0, st,                          \
                        static_cast<const _Float16*>(h), static_cast<const _Float16*>(x),                          \
                        static_cast<_Float16*>(v_out), r_out, qtl, dots, n_tok, (int)d, dots_jstride, eps)
     switch (nb) {
@@ -4126,14 +4143,21 @@ int ldr_read_fwd(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const 
   // pass); else 256-lane workgroups, 16-token tiles, 64 KiB bursts when they fit
   int big_tt = RF_BIG_TT;
   if (LDR_RF_HALF_TT && big_tt * row_bytes > RF_BIG_STAGE) big_tt /= 2;
-  const bool big = LDR_RF_BIG && (n + 2) * row_bytes >= LDR_RF_BIG_MIN_ROW_BYTES && RF_BIG_LANES / tpr <= big_tt &&
-                   big_tt * row_bytes <= RF_BIG_STAGE;
+  const bool big_fits = (n + 2) * row_bytes >= LDR_RF_BIG_MIN_ROW_BYTES && RF_BIG_LANES / tpr <= big_tt &&
+                        big_tt * row_bytes <= RF_BIG_STAGE;
+  const bool big = LDR_RF_BIG && big_fits && cdiv(n_tok, big_tt) >= CUS;
   int tt = big ? big_tt : rf_tile(tpr);
   // rows too long for a tile's output to fit the staging space (fp32 rows of 2048, bf16 rows of 3072 and more): half
   // the tokens per tile, while that still gives every row slot a row, so the output still goes out in bursts
   if (LDR_RF_HALF_TT && !big && RF_STAGE_BYTES > 0 && tt * row_bytes > RF_STAGE_BYTES &&
       (tt / 2) * row_bytes <= RF_STAGE_BYTES && tt / 2 >= WG / tpr)
     tt /= 2;
+  // lanes per token of the softmax: fixed by the row, not by the token count, so a token's bits do not depend on it
+  const int lpt = (big ? RF_BIG_LANES : WG) / tt;
+  // few tokens: smaller tiles, down to a row per row slot, until every workgroup slot of the GPU has one, and the
+  // 512-lane launch only where its tiles reach every CU. Per launch, 16- and 32-token tiles against these: 512 rows of
+  // 2048 bf16 37-41 -> 13.5 us (1..16 sources), 4096 rows of 1024 21-34 -> 21-22 us (fp32 55-62 -> 33-37)
+  while (!big && tt / 2 >= WG / tpr && cdiv(n_tok, tt) < LDR_RF_GRID) tt /= 2;
   const unsigned grid = big ? grid_of(cdiv(n_tok, tt), LDR_RF_BIG_GRID)
                             : grid_of(cdiv(n_tok, tt), LDR_RF_GRID);   // no tokens: one workgroup writes next_prior
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -4144,7 +4168,7 @@ int ldr_read_fwd(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const 
                                                                   static_cast<const T*>(base),                     \
                                                                   static_cast<const T*>(h0), beta, cf, inv_sqrt_d, \
                                                                   static_cast<T*>(out), tc, p, next_prior, n_tok,  \
-                                                                  (int)d, tpr, tt)))
+                                                                  (int)d, tpr, tt, lpt)))
   if (big && h0) {
     LDR_RF_LAUNCH(true, true, RF_BIG_LANES);
   } else if (big) {
@@ -4350,26 +4374,36 @@ int ldr_dv_assemble(const uint64_t* g, const uint64_t* wz, const uint64_t* q, in
   if (e == LDR_E_SHAPE && !LDR_AS_VPT) e = row_layout(d, &vpt, &tpr, 4, false, 0, true);   // rows past 3 x 256 x 8
   if (e) return e;
   if (n_tok == 0) return LDR_OK;
-  const unsigned grid = grid_of(cdiv(n_tok, (WG / tpr) * as_rb(vpt, dtype == LDR_F32)), LDR_AS_GRID);
+  const int rb = as_rb(vpt, dtype == LDR_F32);
+  const bool small = cdiv(n_tok, (WG / tpr) * rb) < CUS;
+  const unsigned grid = grid_of(cdiv(n_tok, (WG / tpr) * (small ? 1 : rb)), LDR_AS_GRID);
   hipStream_t st = static_cast<hipStream_t>(stream);
   // the added gradient is often the last read's output gradient itself (the proposal of that read is this write's
   // h): then its rows are read once
   const bool add_last = add && m > 0 && add == t.g[m - 1];
-#define LDR_AS_LAUNCH(AL, PR)                                                                                     \
-  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_dv_assemble<T, VPT, AL, PR>), dim3(grid), dim3(WG),\
-                                                                  0, st, t, (int)m, static_cast<const T*>(v), r, gr, \
+#define LDR_AS_LAUNCH(AL, PR, SM)                                                                                 \
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_dv_assemble<T, VPT, AL, PR, SM>), dim3(grid),  \
+                                                                  dim3(WG), 0, st, t, (int)m,                      \
+                                                                  static_cast<const T*>(v), r, gr,                 \
                                                                   static_cast<const T*>(add), add_beta,            \
                                                                   static_cast<T*>(dv), static_cast<T*>(dv_neg),    \
                                                                   n_tok, (int)d, tpr)))
-  if (add_last && per_read) {
-    LDR_AS_LAUNCH(true, true)
-  } else if (add_last) {
-    LDR_AS_LAUNCH(true, false)
-  } else if (per_read) {
-    LDR_AS_LAUNCH(false, true)
-  } else {
-    LDR_AS_LAUNCH(false, false)
+#define LDR_AS_PICK(SM)                                                                                           \
+  if (add_last && per_read) {                                                                                     \
+    LDR_AS_LAUNCH(true, true, SM)                                                                                 \
+  } else if (add_last) {                                                                                          \
+    LDR_AS_LAUNCH(true, false, SM)                                                                                \
+  } else if (per_read) {                                                                                          \
+    LDR_AS_LAUNCH(false, true, SM)                                                                                \
+  } else {                                                                                                        \
+    LDR_AS_LAUNCH(false, false, SM)                                                                               \
   }
+  if (small) {
+    LDR_AS_PICK(true)
+  } else {
+    LDR_AS_PICK(false)
+  }
+#undef LDR_AS_PICK
 #undef LDR_AS_LAUNCH
   return launched();
 }
@@ -4545,7 +4579,9 @@ int64_t ldr_read_bwd1_rows_parts(int64_t n_tok, int64_t d) {
       rows_layout(d, 1, &vpt, &tpr) != LDR_OK)
     return 0;
   // a workgroup on every CU first (256), then two rows per row slot before a second one: each part is a row of d
-  // floats to write and reduce
+  // floats to write and reduce. Per launch, one 32-token tile per workgroup against these: 512 rows of 2048 bf16
+  // 59.9 -> 15.0 us, 4096 rows of 1024 33.4 -> 22.6 (fp32 46.4 -> 33.8), 128 rows of 768 20.3 -> 11.4; from 16384
+  // rows on (two 32-token tiles' workgroups per CU) the same launch
   const int rpw = WG / tpr;
   const int64_t one = grid_of(cdiv(n_tok, rpw), 256), two = grid_of(cdiv(n_tok, 2 * rpw), B1_GRID);
   return one > two ? one : two;

@@ -146,11 +146,9 @@ def _dev_addrs(addrs, dev: torch.device) -> torch.Tensor:
 
 
 def _b1_parts(n_tok: int, d: int) -> int:
-    """Rows of backward pass 1's query-gradient partials: the row-layout kernel's workgroups (which the any-shape
-    kernels then also use), or for widths that layout does not take as many as fill the GPU (one workgroup per four
-    tokens on the scalar kernels)."""
-    p = L.bwd1_parts(n_tok, d)
-    return p if p > 0 else L.bwd1_rows_parts(n_tok, d) or max(1, min(512, -(-n_tok // 4)))
+    """Rows of backward pass 1's query-gradient partials, one per workgroup: as many as fill the GPU (for the scalar
+    kernels' widths one per four tokens)."""
+    return L.bwd1_rows_parts(n_tok, d) or max(1, min(512, -(-n_tok // 4)))
 
 
 class _Src:
@@ -203,13 +201,16 @@ _TIMER = None
 # the entry points, bound once (name without the ldr_ prefix -> ctypes function with its signature)
 _FN = {name[4:]: getattr(_LIB, name) for name in L.SIGNATURES}
 
+# the kernel family an entry point's launches are reported under, where it is not the entry point's own name
+_FAMILY = {"read_bwd1_rows": "read_bwd1"}
+
 
 def _run(name: str, *args) -> None:
     fn = _FN[name]
     if _TIMER is None:
         code = fn(*args)
     else:
-        with _TIMER(name):
+        with _TIMER(_FAMILY.get(name, name)):
             code = fn(*args)
     if code:
         L.check(code, name)
@@ -343,9 +344,7 @@ def _bwd1(src: _Src, n, g, gt, prob, dots, tc, cbar_c, c0c, dr_accum, wz, wz_str
     if src.fast:
         if not _fast(d, n, g, g_prop, g_h0):   # the caller chose src with g among its rows
             raise RuntimeError("delta_attnres HIP read: host source tables with rows the row-layout kernels refuse")
-        _run("read_bwd1", *head, dq_part.stride(0), *tail)
-    else:
-        _run("read_bwd1_rows" if src.rows else "read_bwd1_any", *head, parts, dq_part.stride(0), *tail)
+    _run("read_bwd1_rows" if src.fast or src.rows else "read_bwd1_any", *head, parts, dq_part.stride(0), *tail)
     if part is not None:
         return None, dcbar
     dq = torch.empty(d, device=dev, dtype=torch.float32) if dq is None else dq
