@@ -1,4 +1,5 @@
-"""Build libloopback_read.so (the read's kernels and C ABI) in-tree with hipcc for gfx950 (MI355X).
+"""Build libloopback_read.so (the read's kernels and C ABI) and libloopback_lm.so (the language model's) in-tree with
+hipcc for gfx950 (MI355X).
 
     python -m loopback_amd.build                          # compile, print the commands
     python -m loopback_amd.build -D LDR_RF_GRID=768 ...   # with launch settings other than the measured defaults
@@ -23,6 +24,8 @@ ROOT = os.path.dirname(HERE)
 SRC = os.path.join(HERE, "csrc", "loopback_read.hip")
 INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(HERE, "libloopback_read.so")
+LM_SRC = os.path.join(HERE, "csrc", "loopback_lm.hip")
+LM_LIB = os.path.join(HERE, "libloopback_lm.so")
 # A test fixture: the same source built with the alternative kernel shapes -- the write in the matrix cores' layout
 # for every width and dtype (LDR_WM_ROWS=0, LDR_W32_ROWS=0), the read forward in 256-lane workgroups for every read
 # (LDR_RF_BIG=0) -- so the
@@ -101,18 +104,19 @@ def build_abi_smoke(verbose: bool = True) -> str:
 
 
 def build(verbose: bool = True, defines=None, fixtures: bool = True) -> str:
-    """Compile the library (always; a stale build never survives a call) and, with `fixtures`, beside it the test
-    fixture TEST_LIB_ALT (the two compiles run in parallel) and then the C ABI test program; returns the library's
-    path. Every compile started is waited for before any error is raised. The library's failure raises; a test
+    """Compile the libraries (always; a stale build never survives a call) and, with `fixtures`, beside them the test
+    fixture TEST_LIB_ALT (the compiles run in parallel) and then the C ABI test program; returns the read library's
+    path. Every compile started is waited for before any error is raised. A library's failure raises; a test
     fixture's is reported on stderr and does not fail the library's build (the GPU tests that load the fixture then
     fail on its absence). defines: NAME=VALUE launch settings (see the module docstring)."""
-    jobs = [_start(SRC, LIB, verbose, defines)]
+    jobs = [_start(SRC, LIB, verbose, defines), _start(LM_SRC, LM_LIB, verbose, [])]
     if fixtures:
         jobs.append(_start(SRC, TEST_LIB_ALT, verbose, list(defines or []) + ALT_DEFINES))
     errors = [_wait(job) for job in jobs]
-    if errors[0] is not None:
-        raise RuntimeError(errors[0])
-    fixture_errors = [e for e in errors[1:] if e is not None]
+    for e in errors[:2]:
+        if e is not None:
+            raise RuntimeError(e)
+    fixture_errors = [e for e in errors[2:] if e is not None]
     if fixtures and not fixture_errors:
         try:
             build_abi_smoke(verbose)

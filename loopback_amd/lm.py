@@ -10,7 +10,8 @@ layout: each block update is written into the stack, the read combines them) or 
 Plain Loop). Init: every Linear and the embedding N(0, initializer_range), RMSNorm gains 1, the read query zero.
 
 MI355X choices (not the reference's parameterization): q, k, v come from one fused projection and the MLP's gate and
-up from another (one GEMM each instead of three / two); attention is torch's SDPA restricted to its flash and
+up from another (one GEMM each instead of three / two); in 16 bits the norms, SwiGLU and the loss run in this
+package's own kernels (lm_ops), the residual's add and its gradient inside the norms; attention is torch's SDPA restricted to its flash and
 memory-efficient kernels in 16-bit (never the math path's batched products in bf16).
 
     python -m loopback_amd.lm --steps 10 --warmup 3            # config 5: the Loopback LM step, tokens/s
@@ -30,6 +31,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import lm_ops as ops
 from .cell import LoopDeltaAttnRes
 
 
@@ -146,21 +148,47 @@ class SwiGLU(nn.Module):
         self.down = nn.Linear(cfg.intermediate, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        g, u = self.gate_up(x).chunk(2, dim=-1)
-        return self.down(F.silu(g) * u)
+        return self.down(ops.swiglu(self.gate_up(x)))
+
+
+class RMSNorm(nn.RMSNorm):
+    """nn.RMSNorm, on the HIP kernel where it takes the rows."""
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if ops.norm_native(x, self.weight):
+            return ops.add_rms_norm(x, None, self.weight, self.eps)[1]
+        return super().forward(x)
+
+
+def _hooked(m: nn.Module) -> bool:
+    """Whether calling m runs more than its forward (hooks of its own, or of every module)."""
+    g = nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks)
+
+
+def add_norm(norm: nn.Module, x: torch.Tensor, add: torch.Tensor | None = None):
+    """(x + add, norm(x + add)); add None: (x, norm(x)). The kernel takes both steps in one pass, and the gradient
+    that comes back along the first output joins the norm's in one, unless the norm's call is hooked."""
+    if type(norm) is RMSNorm and not _hooked(norm) and ops.norm_native(x, norm.weight, add):
+        return ops.add_rms_norm(x, add, norm.weight, norm.eps)
+    h = x if add is None else x + add
+    return h, norm(h)
 
 
 class Block(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
-        self.attn_norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.attn_norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.attn = Attention(cfg)
-        self.mlp_norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.mlp_norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.mlp = SwiGLU(cfg)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        x = x + self.attn(self.attn_norm(x))
-        return x + self.mlp(self.mlp_norm(x))
+        x, n = add_norm(self.attn_norm, x)
+        x, n = add_norm(self.mlp_norm, x, self.attn(n))
+        return x + self.mlp(n)
 
 
 class LoopbackLM(nn.Module):
@@ -174,7 +202,7 @@ class LoopbackLM(nn.Module):
         self.prelude = nn.ModuleList(Block(cfg) for _ in range(cfg.prelude))
         self.middle = nn.ModuleList(Block(cfg) for _ in range(cfg.loop_blocks))   # shared over the R iterations
         self.coda = nn.ModuleList(Block(cfg) for _ in range(cfg.coda))
-        self.norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
         self.read = (LoopDeltaAttnRes(cfg.hidden_size, cfg.loops, cfg.loop_blocks, beta=cfg.beta, eps=cfg.norm_eps)
                      if cfg.residual == "delta_attnres" else None)
@@ -224,9 +252,7 @@ class LoopbackLM(nn.Module):
         return self.norm(h)
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
-        logits = self.head(self.hidden(ids))
-        labels = torch.cat((ids[:, 1:], torch.full_like(ids[:, :1], -100)), dim=1)
-        return F.cross_entropy(logits.reshape(-1, logits.shape[-1]).float(), labels.reshape(-1), ignore_index=-100)
+        return ops.next_token_loss(self.head(self.hidden(ids)), ids)
 
     def num_params(self) -> int:
         seen = {id(p): p.numel() for p in self.parameters()}

@@ -1,0 +1,238 @@
+"""The language model's row operations on the HIP kernels of libloopback_lm.so (include/loopback_lm.h): RMSNorm with the
+residual's add before it and the residual's gradient folded into its backward, SwiGLU, and the next-token cross
+entropy on 16-bit logits.
+
+`native(...)` says whether the kernels take a call: plain 16-bit GPU tensors of one dtype on one device, no transform
+or tracer that has to see torch operations (torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else --
+the CPU, fp32, other shapes -- stays on torch in lm.py. A backward that is itself differentiated (create_graph) runs
+the torch form of the operation, so second derivatives are torch's.
+"""
+from __future__ import annotations
+
+import ctypes
+import os
+
+import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
+
+from . import build as _build
+
+ABI_VERSION = 1
+NORM_MAX_WIDTH = 2048
+_CODES = {torch.bfloat16: 1, torch.float16: 2}
+
+_p, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
+# name -> (restype, argtypes); one line per declaration of include/loopback_lm.h
+SIGNATURES = {
+    "llm_abi_version": (_i32, []),
+    "llm_rms_norm_fwd": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32, _p]),
+    "llm_rms_norm_parts": (_i64, [_i64]),
+    "llm_rms_norm_bwd": (_i32, [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _p]),
+    "llm_sum_rows": (_i32, [_p, _i64, _i64, _p, _i32, _p]),
+    "llm_swiglu_fwd": (_i32, [_p, _p, _i64, _i64, _i32, _p]),
+    "llm_swiglu_bwd": (_i32, [_p, _p, _p, _i64, _i64, _i32, _p]),
+    "llm_next_token_loss_fwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
+    "llm_next_token_loss_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
+}
+
+
+def _load() -> ctypes.CDLL:
+    path = _build.LM_LIB
+    if not os.path.exists(path):
+        raise ImportError(f"loopback_lm: {path} is not built (run `python -m loopback_amd.build`)")
+    lib = ctypes.CDLL(path)
+    for name, (res, args) in SIGNATURES.items():
+        fn = getattr(lib, name)          # AttributeError -> the library is stale
+        fn.restype, fn.argtypes = res, args
+    if lib.llm_abi_version() != ABI_VERSION:
+        raise ImportError(f"loopback_lm: {path} has ABI {lib.llm_abi_version()}, expected {ABI_VERSION}; rebuild")
+    return lib
+
+
+LIB = _load()
+
+
+def _run(name: str, *args) -> None:
+    code = getattr(LIB, name)(*args)
+    if code:
+        raise RuntimeError(f"{name}: refused or failed to launch (code {code})")
+
+
+def _stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+def native(*tensors) -> bool:
+    first = tensors[0]
+    if not first.is_cuda or first.dtype not in _CODES:
+        return False
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.dtype is not first.dtype \
+                or t.device != first.device:
+            return False
+    return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
+                or torch.jit.is_tracing() or forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
+def _again(fn, inputs, needed, grads):
+    """The gradients of fn at `inputs`, as torch forms them with a graph (a backward that is differentiated)."""
+    with torch.enable_grad():
+        outs = fn(*inputs)
+        wanted = [x for x, need in zip(inputs, needed) if need]
+        got = iter(torch.autograd.grad(outs, wanted, grads, create_graph=True, allow_unused=True))
+    return [next(got) if need else None for need in needed]
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# RMSNorm
+# ---------------------------------------------------------------------------------------------------------------
+def _norm_torch(eps):
+    return lambda h, w: (h, F.rms_norm(h, (h.shape[-1],), w, eps))
+
+
+class _AddRmsNorm(torch.autograd.Function):
+    """(h, y) = (x + add, rms_norm(x + add) w); add may be None (h is then x itself, as an alias). h carries the
+    residual stream on, so the gradient that comes back along it joins the norm's in one kernel."""
+
+    @staticmethod
+    def forward(ctx, x, add, w, eps):
+        d = x.shape[-1]
+        rows = x.numel() // d
+        h = x.view_as(x) if add is None else torch.empty_like(x)
+        y = torch.empty_like(x)
+        rstd = torch.empty(rows, device=x.device, dtype=torch.float32)
+        _run("llm_rms_norm_fwd", x.data_ptr(), None if add is None else add.data_ptr(), w.data_ptr(),
+             None if add is None else h.data_ptr(), y.data_ptr(), rstd.data_ptr(), rows, d, eps, _CODES[x.dtype],
+             _stream(x))
+        ctx.eps, ctx.added = eps, add is not None
+        ctx.save_for_backward(x if add is None else h, w, rstd)
+        ctx.set_materialize_grads(False)
+        return h, y
+
+    @staticmethod
+    def backward(ctx, dh, dy):
+        h, w, rstd = ctx.saved_tensors
+        if dy is None:
+            return dh, dh if ctx.added else None, None, None
+        if torch.is_grad_enabled():
+            dh = torch.zeros_like(dy) if dh is None else dh
+            dx, dw = _again(_norm_torch(ctx.eps), [h, w], [True, ctx.needs_input_grad[2]], (dh, dy))
+            return dx, dx if ctx.added else None, dw, None
+        d = h.shape[-1]
+        rows = h.numel() // d
+        dy = _dense(dy, h)
+        dres = None if dh is None else _dense(dh, h)
+        dx = torch.empty_like(h)
+        parts = LIB.llm_rms_norm_parts(rows)
+        part = torch.empty((parts, d), device=h.device, dtype=torch.float32)
+        dw = torch.empty_like(w)
+        _run("llm_rms_norm_bwd", dy.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(),
+             None if dres is None else dres.data_ptr(), dx.data_ptr(), part.data_ptr(), rows, d, _CODES[h.dtype],
+             _stream(h))
+        _run("llm_sum_rows", part.data_ptr(), parts, d, dw.data_ptr(), _CODES[w.dtype], _stream(h))
+        return dx, dx if ctx.added else None, dw, None
+
+
+def _dense(g, like):
+    """A gradient as the kernels take it: contiguous rows, 16-byte aligned, the saved tensor's dtype."""
+    g = g.to(like.dtype).contiguous()
+    return g if g.data_ptr() % 16 == 0 else g.clone()
+
+
+def _rows_ok(*tensors) -> bool:
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def norm_native(x, w, add=None) -> bool:
+    """Whether add_rms_norm takes the call: rows of a multiple of 8 elements up to NORM_MAX_WIDTH, contiguous."""
+    ts = (x, w) if add is None else (x, w, add)
+    d = x.shape[-1] if x.dim() else 0
+    return (native(*ts) and 8 <= d <= NORM_MAX_WIDTH and d % 8 == 0 and w.shape == (d,)
+            and (add is None or add.shape == x.shape) and _rows_ok(*ts))
+
+
+def add_rms_norm(x, add, w, eps):
+    return _AddRmsNorm.apply(x, add, w, float(eps))
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# SwiGLU
+# ---------------------------------------------------------------------------------------------------------------
+def _swiglu_torch(gu):
+    g, u = gu.chunk(2, dim=-1)
+    return F.silu(g) * u
+
+
+class _SwiGLU(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, gu):
+        n = gu.shape[-1] // 2
+        rows = gu.numel() // (2 * n)
+        act = torch.empty((*gu.shape[:-1], n), device=gu.device, dtype=gu.dtype)
+        _run("llm_swiglu_fwd", gu.data_ptr(), act.data_ptr(), rows, n, _CODES[gu.dtype], _stream(gu))
+        ctx.save_for_backward(gu)
+        return act
+
+    @staticmethod
+    def backward(ctx, da):
+        gu, = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _again(_swiglu_torch, [gu], [True], (da,))[0]
+        n = gu.shape[-1] // 2
+        da = _dense(da, gu)
+        dgu = torch.empty_like(gu)
+        _run("llm_swiglu_bwd", gu.data_ptr(), da.data_ptr(), dgu.data_ptr(), gu.numel() // (2 * n), n,
+             _CODES[gu.dtype], _stream(gu))
+        return dgu
+
+
+def swiglu(gu: torch.Tensor) -> torch.Tensor:
+    """silu(g) * u of rows [g | u]."""
+    if native(gu) and gu.shape[-1] % 16 == 0 and gu.numel() > 0 and _rows_ok(gu):
+        return _SwiGLU.apply(gu)
+    return _swiglu_torch(gu)
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# next-token cross entropy
+# ---------------------------------------------------------------------------------------------------------------
+def _loss_torch(ids):
+    def fn(logits):
+        labels = torch.cat((ids[:, 1:], torch.full_like(ids[:, :1], -100)), dim=1)
+        return F.cross_entropy(logits.reshape(-1, logits.shape[-1]).float(), labels.reshape(-1), ignore_index=-100)
+    return fn
+
+
+class _NextTokenLoss(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, logits, ids):
+        b, t, vocab = logits.shape
+        lse = torch.empty((b * t, 2), device=logits.device, dtype=torch.float32)
+        scratch = torch.empty(b * t, device=logits.device, dtype=torch.float32)
+        loss = torch.empty((), device=logits.device, dtype=torch.float32)
+        _run("llm_next_token_loss_fwd", logits.data_ptr(), ids.data_ptr(), lse.data_ptr(), scratch.data_ptr(),
+             loss.data_ptr(), b, t, vocab, _CODES[logits.dtype], _stream(logits))
+        ctx.save_for_backward(logits, ids, lse)
+        return loss
+
+    @staticmethod
+    def backward(ctx, g):
+        logits, ids, lse = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _again(_loss_torch(ids), [logits], [True], (g,))[0], None
+        b, t, vocab = logits.shape
+        dlogits = torch.empty_like(logits)
+        _run("llm_next_token_loss_bwd", logits.data_ptr(), ids.data_ptr(), lse.data_ptr(), g.data_ptr(),
+             dlogits.data_ptr(), b, t, vocab, _CODES[logits.dtype], _stream(logits))
+        return dlogits, None
+
+
+def next_token_loss(logits: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
+    """Mean cross entropy of logits (b, t, vocab) against ids shifted by one, the last position ignored."""
+    if (native(logits) and type(ids) is torch.Tensor and ids.device == logits.device and ids.dtype is torch.int64
+            and ids.is_contiguous() and logits.is_contiguous() and logits.shape[:-1] == ids.shape
+            and 0 < ids.numel() < 2 ** 31):
+        return _NextTokenLoss.apply(logits, ids)
+    return _loss_torch(ids)(logits)

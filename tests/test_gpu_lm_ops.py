@@ -1,0 +1,138 @@
+"""The language model's row kernels (lm_ops) against torch in fp64 on the same 16-bit inputs: every result is an fp32
+value rounded once, so each element lies within half a unit in the last place (2^-8 of a bf16 value, 2^-11 of an fp16 one)
+plus fp32 round-off (1e-5 of the result's RMS). Sizes: one vector, a lane's and a wave's edges, the widest row; one
+row, remainders, more rows than workgroups take at once; vocabularies below, at and past a vector and a workgroup's
+2048 logits. Then what must stay torch's: second derivatives, hooks on the norms, forward mode, fp32."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from gpu_helpers import DEV
+
+pytestmark = pytest.mark.gpu
+HALF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}   # significands of 8 and 11 bits: half a step of the last
+
+
+def close(got, ref, dtype):
+    ref = ref.double()
+    rms = ref.pow(2).mean().sqrt() if ref.numel() else 0.0
+    tiny = 2.0 ** -25 if dtype is torch.float16 else 0.0   # half of fp16's smallest subnormal
+    bad = (got.double() - ref).abs() > HALF.get(dtype, 0.0) * ref.abs() + 1e-5 * rms + tiny
+    assert not bad.any(), ((got.double() - ref).abs().max().item(), rms)
+
+
+def rnd(shape, dtype, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("rows,d", [(1, 8), (5, 16), (3, 512), (7, 520), (2049, 768), (5, 1032), (9, 2048)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("add", [False, True])
+def test_add_rms_norm(rows, d, dtype, add):
+    from loopback_amd import lm_ops as ops
+    print(f"case norm {rows}x{d} {dtype} add={add}", flush=True)
+    x, w = rnd((rows, d), dtype, 1).requires_grad_(), rnd((d,), dtype, 2).requires_grad_()
+    a = rnd((rows, d), dtype, 3).requires_grad_() if add else None
+    dh, dy = rnd((rows, d), dtype, 4), rnd((rows, d), dtype, 5)
+    assert ops.norm_native(x, w, a)
+    h, y = ops.add_rms_norm(x, a, w, 1e-6)
+    torch.autograd.backward((h, y), (dh, dy))
+    torch.cuda.synchronize()
+    hr = (x + a if add else x).detach()
+    assert torch.equal(h, hr)
+    h64, w64 = hr.double().requires_grad_(), w.detach().double().requires_grad_()
+    y64 = F.rms_norm(h64, (d,), w64, 1e-6)
+    torch.autograd.backward((h64, y64), (dh.double(), dy.double()))
+    close(y, y64.detach(), dtype)
+    close(x.grad, h64.grad, dtype)
+    close(w.grad, w64.grad, dtype)
+    if add:
+        assert torch.equal(a.grad, x.grad)
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 264), (2049, 2048)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu(rows, n, dtype):
+    from loopback_amd import lm_ops as ops
+    print(f"case swiglu {rows}x{n} {dtype}", flush=True)
+    gu = (3 * rnd((rows, 2 * n), dtype, 6)).requires_grad_()
+    da = rnd((rows, n), dtype, 7)
+    act = ops.swiglu(gu)
+    act.backward(da)
+    torch.cuda.synchronize()
+    g64 = gu.detach().double().requires_grad_()
+    a64 = F.silu(g64[:, :n]) * g64[:, n:]
+    a64.backward(da.double())
+    close(act, a64.detach(), dtype)
+    close(gu.grad, g64.grad, dtype)
+
+
+@pytest.mark.parametrize("b,t,vocab", [(1, 2, 1), (2, 3, 7), (1, 9, 8), (3, 5, 33), (2, 17, 2048), (2, 4, 2057),
+                                       (3, 300, 32000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_next_token_loss(b, t, vocab, dtype):
+    from loopback_amd import lm_ops as ops
+    print(f"case loss {b}x{t}x{vocab} {dtype}", flush=True)
+    ids = torch.randint(0, vocab, (b, t), generator=torch.Generator().manual_seed(8)).to(DEV)
+    x = (4 * rnd((b, t, vocab), dtype, 9)).requires_grad_()
+    loss = ops.next_token_loss(x, ids)
+    (2.0 * loss).backward()
+    torch.cuda.synchronize()
+    x64 = x.detach().double().requires_grad_()
+    l64 = F.cross_entropy(x64[:, :-1].reshape(-1, vocab), ids[:, 1:].reshape(-1))
+    (2.0 * l64).backward()
+    assert abs(loss.item() - l64.item()) <= 2e-6 * max(1.0, abs(l64.item()))
+    close(x.grad, x64.grad, dtype)
+
+
+def test_loss_edge_rows():
+    """Rows with -inf logits (masked vocabulary), the type's lowest value and large spreads; one position per
+    sequence (nothing counted: NaN, as torch's mean of nothing, and a zero gradient)."""
+    from loopback_amd import lm_ops as ops
+    x = rnd((1, 6, 4100), torch.bfloat16, 10)
+    x[0, 0, 5:] = float("-inf")
+    x[0, 1] = torch.finfo(torch.bfloat16).min
+    x[0, 2, 7] = 3e38
+    x[0, 3, :4096] = float("-inf")
+    ids = torch.tensor([[0, 3, 9, 7, 4099, 1]], device=DEV)
+    x.requires_grad_()
+    loss = ops.next_token_loss(x, ids)
+    loss.backward()
+    ref = x.detach().float().requires_grad_()
+    lr = F.cross_entropy(ref[0, :-1], ids[0, 1:])
+    lr.backward()
+    assert torch.allclose(loss, lr, rtol=1e-6)
+    close(x.grad, ref.grad, torch.bfloat16)
+    one = rnd((2, 1, 64), torch.bfloat16, 11).requires_grad_()
+    loss = ops.next_token_loss(one, torch.zeros(2, 1, dtype=torch.int64, device=DEV))
+    loss.backward()
+    assert loss.isnan() and not one.grad.any()
+
+
+def test_what_stays_torch():
+    """Second derivatives are torch's; a hooked norm is called as a module; forward-mode, vmap and fp32 calls take
+    torch's operations."""
+    from loopback_amd import lm, lm_ops as ops
+    x, w = rnd((5, 64), torch.bfloat16, 12).requires_grad_(), rnd((64,), torch.bfloat16, 13).requires_grad_()
+    gu = rnd((5, 64), torch.bfloat16, 14).requires_grad_()
+
+    def second(fn, *inputs):
+        out = fn(*inputs)
+        g = torch.autograd.grad(out, inputs, torch.ones_like(out), create_graph=True)
+        return torch.autograd.grad(sum(t.float().pow(2).sum() for t in g), inputs)
+
+    pairs = [(second(lambda a, b: ops.add_rms_norm(a, None, b, 1e-6)[1], x, w),
+              second(lambda a, b: F.rms_norm(a, (64,), b, 1e-6), x, w)),
+             (second(ops.swiglu, gu), second(ops._swiglu_torch, gu))]
+    for got, ref in pairs:
+        for a, b in zip(got, ref):
+            assert (a - b).float().norm() <= 2e-2 * b.float().norm()
+    block = lm.Block(lm.LMConfig(hidden_size=64, num_heads=4)).to(DEV, torch.bfloat16)
+    seen = []
+    y = block(x[None])
+    block.mlp_norm.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    assert torch.allclose(block(x[None]).float(), y.float(), atol=2e-2) and seen == [torch.Size([1, 5, 64])]
+    y, dy = torch.func.jvp(ops.swiglu, (gu.detach(),), (torch.ones_like(gu),))
+    assert torch.equal(y, ops._swiglu_torch(gu.detach())) and dy.shape == y.shape
+    assert torch.func.vmap(ops.swiglu)(gu.detach()[None]).shape == (1, 5, 32)
+    assert not ops.native(x.detach().float())
