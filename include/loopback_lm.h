@@ -55,6 +55,24 @@ int llm_next_token_loss_fwd(const void* logits, const int64_t* ids, float* lse, 
 int llm_next_token_loss_bwd(const void* logits, const int64_t* ids, const float* lse, const float* dloss, void* dlogits,
                             int64_t b, int64_t t, int64_t vocab, int dtype, void* stream);
 
+/* ---- causal rotary attention, head width 64, bf16 --------------------------------------------------------------
+ * qkv [b, t, 3, heads, 64] (16-byte aligned); cos and sin [t, 64] fp32, both halves of a row alike. */
+
+/* q and k rotated (pairs j, j + 32; x1 cos - x2 sin, x2 cos + x1 sin in fp32, one rounding) into qk [b, t, 2, heads,
+ * 64]. */
+int llm_rotary(const void* qkv, const float* cosT, const float* sinT, void* qk, int64_t b, int64_t t, int64_t heads,
+               void* stream);
+
+/* out [b, t, heads, 64] = softmax(q k^T / 8, causal) v from qk and qkv's v; lse2 [b heads, t], the base-2 logarithm of
+ * each query's sum of exponentials, for the backward. */
+int llm_attn_fwd(const void* qk, const void* qkv, void* out, float* lse2, int64_t b, int64_t t, int64_t heads,
+                 void* stream);
+
+/* dqkv [b, t, 3, heads, 64], the gradient of qkv through the rotation and the attention; delta: scratch [b heads, t]. */
+int llm_attn_bwd(const void* qk, const void* qkv, const void* out, const void* dout, const float* lse2,
+                 const float* cosT, const float* sinT, float* delta, void* dqkv, int64_t b, int64_t t, int64_t heads,
+                 void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -337,6 +337,430 @@ __global__ __launch_bounds__(WG) void k_next_token_bwd(const T* __restrict__ log
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// causal rotary attention, head width 64, bf16 (fp32 scores, softmax and accumulators; the probabilities and score
+// gradients enter the matrix cores in bf16, as in every flash attention)
+//
+// Operands go through v_mfma_f32_32x32x16_bf16: lane l holds row (A) or column (B) l mod 32 at k = 8 (l / 32) .. + 8; of
+// the 32 x 32 result it holds column l mod 32 and, in register r, row 4 (l / 32) + r mod 4 + 8 (r / 4). The scores are
+// formed transposed where the next product sums over their rows, so a product's result is the next one's B operand as
+// it lies in the registers (its k order permuted: slot j of lane half h of a 16-row step is row 4 h + j, + 4 past j = 3),
+// and a row's softmax is in-lane but for one exchange of lane halves. The matching A operands, columns of a tile kept by
+// rows, come from LDS with ds_read_b64_tr_b16: of the 16 lanes that read 4 rows x 16 columns together, lane i gets
+// column i of the 4 rows. Tiles of 64 rows sit in LDS in rows of 144 bytes (16 of padding: the 16-byte operand reads of
+// 16 rows then cover the 64 banks once), two buffers each, the next tile's rows in registers while one is worked on.
+//
+// Per 64 x 32 tile a wave issues 512 matrix-core cycles forward (512 per product pair backward) and ~1000 vector cycles
+// (per score an exponential, 16 cycles, and 4-7 operations of 4): the vector units bound it, so two or three waves
+// share a SIMD and the maximum is moved, and the sums rescaled, only when it grows by more than 2^8.
+// 8 x 2048 tokens, 12 heads: the rotation 17-19 us, forward 113-125 us (455 TFLOP/s of the causal half), dq 138-153,
+// dk and dv 224-247; the flash attention of torch took 172, 288 and 480-500 us, and the rotation, its gradient and the
+// copies between layouts another ~700 in some twenty elementwise launches.
+// ---------------------------------------------------------------------------------------------------------------
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int AT_M = 128, AT_N = 64, AT_LD = 72;   // rows per workgroup (32 per wave), rows per LDS tile, its row length
+constexpr float AT_LAZY = 8.f;                      // the maximum moves when it grows by 2^8 or more
+constexpr float AT_SCALE = 0.125f, LOG2E = 1.4426950408889634f;   // 1 / sqrt(64)
+
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 zero16() {
+  f32x16 z;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.f;
+  return z;
+}
+__device__ __forceinline__ bf16x8 frag(uint4 u) { return __builtin_bit_cast(bf16x8, u); }
+// registers 8 s .. 8 s + 7 of a result as the B operand of the next product's 16-row step s
+__device__ __forceinline__ bf16x8 operand(const f32x16& x, int s) {
+  return frag(make_uint4(pack2(x[8 * s], x[8 * s + 1]), pack2(x[8 * s + 2], x[8 * s + 3]),
+                         pack2(x[8 * s + 4], x[8 * s + 5]), pack2(x[8 * s + 6], x[8 * s + 7])));
+}
+// A operand, rows as they lie: rows r0 + l mod 32, columns 16 ks + 8 (l / 32) .. + 8
+__device__ __forceinline__ bf16x8 rows_frag(const bf16_t* tile, int r0, int ks, int lane) {
+  return frag(*reinterpret_cast<const uint4*>(tile + (r0 + (lane & 31)) * AT_LD + 16 * ks + 8 * (lane >> 5)));
+}
+// A operand, columns of the tile: columns c0 + l mod 32, rows r0 + {4 h + 0..3, 8 + 4 h + 0..3}, the order of operand()
+__device__ __forceinline__ bf16x8 cols_frag(const bf16_t* tile, int r0, int c0, int lane) {
+  typedef __attribute__((address_space(3))) s16x4* lds4;
+  const int j = lane & 15;
+  const bf16_t* p = tile + (r0 + 4 * (lane >> 5) + (j >> 2)) * AT_LD + c0 + (lane & 16) + 4 * (j & 3);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(const_cast<bf16_t*>(p)));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(const_cast<bf16_t*>(p + 8 * AT_LD)));
+  const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
+  return frag(make_uint4(ua.x, ua.y, ub.x, ub.y));
+}
+__device__ __forceinline__ float other_half(float x, bool sum) {   // x joined with the other lane half's
+  const unsigned u = __float_as_uint(x);
+  const auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float a = __uint_as_float((unsigned)sw[0]), b = __uint_as_float((unsigned)sw[1]);
+  return sum ? a + b : fmaxf(a, b);
+}
+
+// 64 rows of 64 elements, row stride `stride` elements, rows past the last repeated: 512 16-byte pieces, two per lane
+struct TileRegs { uint4 u[2]; };
+__device__ __forceinline__ TileRegs tile_load(const bf16_t* base, int64_t stride, int row0, int t) {
+  TileRegs r;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    r.u[i] = *reinterpret_cast<const uint4*>(base + (int64_t)min(row0 + (c >> 3), t - 1) * stride + 8 * (c & 7));
+  }
+  return r;
+}
+__device__ __forceinline__ void tile_store(bf16_t* tile, const TileRegs& r) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    *reinterpret_cast<uint4*>(tile + (c >> 3) * AT_LD + 8 * (c & 7)) = r.u[i];
+  }
+}
+
+// Which (batch, head) and block of rows a workgroup takes: the blocks of one head on one XCD (workgroups go to XCDs in
+// turn), so its rows are read from that XCD's L2; false past the last head.
+struct AttnWork { int bh, block; };
+__device__ __forceinline__ bool attn_work(int bhs, int blocks, AttnWork& w) {
+  const int i = (int)blockIdx.x >> 3;
+  w.bh = ((int)blockIdx.x & 7) + 8 * (i / blocks);
+  w.block = i % blocks;
+  return w.bh < bhs;
+}
+
+// q and k of [b, t, 3, heads, 64] rotated (pairs j, j + 32; cos, sin [t, 64] fp32 with both halves alike) into
+// [b, t, 2, heads, 64]: products, then the sum, each rounded in fp32, and one rounding to bf16, as the torch form
+__global__ __launch_bounds__(WG) void k_rotary(const bf16_t* __restrict__ qkv, const float* __restrict__ cosT,
+                                               const float* __restrict__ sinT, bf16_t* __restrict__ qk, int64_t n,
+                                               int t, int heads) {
+#pragma clang fp contract(off)
+  const int per = 2 * heads * 4;   // work items of a token: (q or k, head, 8 of the 32 pairs)
+  for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
+    const int64_t tok = i / per;
+    const int r = (int)(i - tok * per), j = 8 * (r & 3), head = r >> 2;   // head counts q's, then k's
+    const bf16_t* x = qkv + (tok * 3 * heads + head) * 64 + j;
+    const int64_t pos = (tok % t) * 64 + j;
+    float a[8], b[8], c[8], s[8], o[8];
+    IO<bf16_t>::load(x, a);
+    IO<bf16_t>::load(x + 32, b);
+    load_f32x8(cosT + pos, c);
+    load_f32x8(sinT + pos, s);
+    bf16_t* y = qk + (tok * 2 * heads + head) * 64 + j;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = a[k] * c[k] + -b[k] * s[k];
+    IO<bf16_t>::store(y, o);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = b[k] * c[k] + a[k] * s[k];
+    IO<bf16_t>::store(y + 32, o);
+  }
+}
+
+// out [b, t, heads, 64] and lse2 [b heads, t] (the base-2 logarithm of each query's sum of exponentials of c times its
+// scores, c = log2(e) / 8). A workgroup takes 128 queries, the last blocks (the most keys) first.
+__global__ __launch_bounds__(256) void k_attn_fwd(const bf16_t* __restrict__ qk, const bf16_t* __restrict__ qkv,
+                                                  bf16_t* __restrict__ out, float* __restrict__ lse2, int bhs, int t,
+                                                  int heads, float c) {
+  __shared__ __align__(16) bf16_t s_k[2][AT_N * AT_LD], s_v[2][AT_N * AT_LD];
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int blocks = (t + AT_M - 1) / AT_M;
+  AttnWork wk;
+  if (!attn_work(bhs, blocks, wk)) return;
+  const int q0 = (blocks - 1 - wk.block) * AT_M, b = wk.bh / heads, head = wk.bh - b * heads;
+  const int64_t sqk = 2 * (int64_t)heads * 64, sv = 3 * (int64_t)heads * 64, so = (int64_t)heads * 64;
+  const bf16_t* qp = qk + (int64_t)b * t * sqk + head * 64;
+  const bf16_t* kp = qp + heads * 64;
+  const bf16_t* vp = qkv + (int64_t)b * t * sv + (2 * heads + head) * 64;
+  const int w0 = q0 + 32 * wave, query = w0 + (lane & 31), qrow = min(query, t - 1);
+  bf16x8 qf[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    qf[ks] = frag(*reinterpret_cast<const uint4*>(qp + qrow * sqk + 16 * ks + 8 * half));
+  f32x16 o[2] = {zero16(), zero16()};
+  float m = -INFINITY, l = 0.f;
+  const int ntiles = (min(q0 + AT_M, t) + AT_N - 1) / AT_N;
+  TileRegs kr = tile_load(kp, sqk, 0, t), vr = tile_load(vp, sv, 0, t);
+  tile_store(s_k[0], kr);
+  tile_store(s_v[0], vr);
+  __syncthreads();
+  for (int j = 0; j < ntiles; ++j) {
+    const int k0 = j * AT_N, cur = j & 1;
+    if (j + 1 < ntiles) {
+      kr = tile_load(kp, sqk, k0 + AT_N, t);
+      vr = tile_load(vp, sv, k0 + AT_N, t);
+    }
+    if (k0 <= w0 + 31 && w0 < t) {   // this wave has queries past the tile's first key
+      f32x16 s[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        s[i] = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) s[i] = mfma(rows_frag(s_k[cur], 32 * i, ks, lane), qf[ks], s[i]);
+      }
+      if (k0 + AT_N - 1 > w0) {        // keys past the query
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (k0 + 32 * i + 4 * half + (r & 3) + 8 * (r >> 2) > query) s[i][r] = -INFINITY;
+      }
+      float mx = s[0][0];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[i][r]);
+      mx = other_half(mx, false) * c;
+      if (__any(mx > m + AT_LAZY)) {
+        const float mn = fmaxf(m, mx), a = m == mn ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
+        l *= a;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[i][r] *= a;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          s[i][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], c, -m));
+          l += s[i][r];
+        }
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const bf16x8 p = operand(s[i], st);
+#pragma unroll
+          for (int d = 0; d < 2; ++d) o[d] = mfma(cols_frag(s_v[cur], 32 * i + 16 * st, 32 * d, lane), p, o[d]);
+        }
+      }
+    }
+    if (j + 1 < ntiles) {
+      tile_store(s_k[cur ^ 1], kr);
+      tile_store(s_v[cur ^ 1], vr);
+      __syncthreads();
+    }
+  }
+  l = other_half(l, true);
+  if (query < t) {
+    const float inv = 1.f / l;
+    bf16_t* op = out + ((int64_t)b * t + query) * so + head * 64 + 4 * half;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2*>(op + 32 * d + 8 * g) =
+            make_uint2(pack2(o[d][4 * g] * inv, o[d][4 * g + 1] * inv), pack2(o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv));
+    if (half == 0) lse2[(int64_t)wk.bh * t + query] = m + __builtin_amdgcn_logf(l);
+  }
+}
+
+// The gradient of a rotated row, dims j (x) and j + 32 (y) in the registers of a transposed result, turned back and
+// stored in bf16 (scaled by `scale`); row: the 64 elements to write, pos: the token's position.
+__device__ __forceinline__ void store_unrotated(bf16_t* row, const f32x16& x, const f32x16& y, const float* cosT,
+                                                const float* sinT, int pos, int half, float scale) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int j = 8 * g + 4 * half;
+    const float4 c = *reinterpret_cast<const float4*>(cosT + (int64_t)pos * 64 + j);
+    const float4 s = *reinterpret_cast<const float4*>(sinT + (int64_t)pos * 64 + j);
+    const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {s.x, s.y, s.z, s.w};
+    float a[4], b[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float u = x[4 * g + k] * scale, v = y[4 * g + k] * scale;
+      a[k] = u * cc[k] + v * ss[k];
+      b[k] = v * cc[k] - u * ss[k];
+    }
+    *reinterpret_cast<uint2*>(row + j) = make_uint2(pack2(a[0], a[1]), pack2(a[2], a[3]));
+    *reinterpret_cast<uint2*>(row + 32 + j) = make_uint2(pack2(b[0], b[1]), pack2(b[2], b[3]));
+  }
+}
+
+// dq into dqkv's first third, and delta [b heads, t] = sum of dout out for the kernel below. As the forward: 128
+// queries per workgroup, the scores and their gradients transposed (columns = queries).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_bwd_q(
+    const bf16_t* __restrict__ qk, const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ out,
+    const bf16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ cosT,
+    const float* __restrict__ sinT, float* __restrict__ delta, bf16_t* __restrict__ dqkv, int bhs, int t, int heads,
+    float c, float scale) {
+  __shared__ __align__(16) bf16_t s_k[2][AT_N * AT_LD], s_v[2][AT_N * AT_LD];
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int blocks = (t + AT_M - 1) / AT_M;
+  AttnWork wk;
+  if (!attn_work(bhs, blocks, wk)) return;
+  const int q0 = (blocks - 1 - wk.block) * AT_M, b = wk.bh / heads, head = wk.bh - b * heads;
+  const int64_t sqk = 2 * (int64_t)heads * 64, sv = 3 * (int64_t)heads * 64, so = (int64_t)heads * 64;
+  const bf16_t* qp = qk + (int64_t)b * t * sqk + head * 64;
+  const bf16_t* kp = qp + heads * 64;
+  const bf16_t* vp = qkv + (int64_t)b * t * sv + (2 * heads + head) * 64;
+  const int w0 = q0 + 32 * wave, query = w0 + (lane & 31), qrow = min(query, t - 1);
+  const int64_t orow = ((int64_t)b * t + qrow) * so + head * 64 + 8 * half;
+  bf16x8 qf[4], gf[4];
+  float dl = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    qf[ks] = frag(*reinterpret_cast<const uint4*>(qp + qrow * sqk + 16 * ks + 8 * half));
+    float g[8], y[8];
+    const uint4 gu = *reinterpret_cast<const uint4*>(dout + orow + 16 * ks);
+    gf[ks] = frag(gu);
+    IO<bf16_t>::unpack(IO<bf16_t>::Raw{gu}, g);
+    IO<bf16_t>::load(out + orow + 16 * ks, y);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) dl = __builtin_fmaf(g[k], y[k], dl);
+  }
+  dl = other_half(dl, true);
+  const float ls = lse2[(int64_t)wk.bh * t + qrow];
+  if (query < t && half == 0) delta[(int64_t)wk.bh * t + query] = dl;
+  f32x16 dq[2] = {zero16(), zero16()};
+  const int ntiles = (min(q0 + AT_M, t) + AT_N - 1) / AT_N;
+  TileRegs kr = tile_load(kp, sqk, 0, t), vr = tile_load(vp, sv, 0, t);
+  tile_store(s_k[0], kr);
+  tile_store(s_v[0], vr);
+  __syncthreads();
+  for (int j = 0; j < ntiles; ++j) {
+    const int k0 = j * AT_N, cur = j & 1;
+    if (j + 1 < ntiles) {
+      kr = tile_load(kp, sqk, k0 + AT_N, t);
+      vr = tile_load(vp, sv, k0 + AT_N, t);
+    }
+    if (k0 <= w0 + 31 && w0 < t) {
+      const bool edge = k0 + AT_N - 1 > w0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        f32x16 s = zero16(), dp = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          s = mfma(rows_frag(s_k[cur], 32 * i, ks, lane), qf[ks], s);
+          dp = mfma(rows_frag(s_v[cur], 32 * i, ks, lane), gf[ks], dp);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ls));
+          s[r] = p * (dp[r] - dl);
+          if (edge && k0 + 32 * i + 4 * half + (r & 3) + 8 * (r >> 2) > query) s[r] = 0.f;
+        }
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const bf16x8 ds = operand(s, st);
+#pragma unroll
+          for (int d = 0; d < 2; ++d) dq[d] = mfma(cols_frag(s_k[cur], 32 * i + 16 * st, 32 * d, lane), ds, dq[d]);
+        }
+      }
+    }
+    if (j + 1 < ntiles) {
+      tile_store(s_k[cur ^ 1], kr);
+      tile_store(s_v[cur ^ 1], vr);
+      __syncthreads();
+    }
+  }
+  if (query < t)
+    store_unrotated(dqkv + ((int64_t)b * t + query) * sv + head * 64, dq[0], dq[1], cosT, sinT, query, half, scale);
+}
+
+// dk and dv into dqkv's other thirds: 128 keys per workgroup, the first blocks (the most queries) first; the scores as
+// they are (columns = keys, rows = queries), each query's lse2 and delta from LDS.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_bwd_kv(
+    const bf16_t* __restrict__ qk, const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ dout,
+    const float* __restrict__ lse2, const float* __restrict__ delta, const float* __restrict__ cosT,
+    const float* __restrict__ sinT, bf16_t* __restrict__ dqkv, int bhs, int t, int heads, float c, float scale) {
+  __shared__ __align__(16) bf16_t s_q[2][AT_N * AT_LD], s_g[2][AT_N * AT_LD];
+  __shared__ __align__(16) float s_ls[2][AT_N], s_dl[2][AT_N];
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int blocks = (t + AT_M - 1) / AT_M;
+  AttnWork wk;
+  if (!attn_work(bhs, blocks, wk)) return;
+  const int k0 = wk.block * AT_M, b = wk.bh / heads, head = wk.bh - b * heads;
+  const int64_t sqk = 2 * (int64_t)heads * 64, sv = 3 * (int64_t)heads * 64, so = (int64_t)heads * 64;
+  const bf16_t* qp = qk + (int64_t)b * t * sqk + head * 64;
+  const bf16_t* gp = dout + (int64_t)b * t * so + head * 64;
+  const int w0 = k0 + 32 * wave, key = w0 + (lane & 31), krow = min(key, t - 1);
+  const bf16_t* kp = qp + heads * 64 + krow * sqk + 8 * half;
+  const bf16_t* vp = qkv + ((int64_t)b * t + krow) * sv + (2 * heads + head) * 64 + 8 * half;
+  const float* lp = lse2 + (int64_t)wk.bh * t;
+  const float* dp_ = delta + (int64_t)wk.bh * t;
+  bf16x8 kf[4], vf[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    kf[ks] = frag(*reinterpret_cast<const uint4*>(kp + 16 * ks));
+    vf[ks] = frag(*reinterpret_cast<const uint4*>(vp + 16 * ks));
+  }
+  f32x16 dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
+  const int first = k0 / AT_N, ntiles = (t + AT_N - 1) / AT_N;
+  const int tid = (int)threadIdx.x, sr = min(tid, 2 * AT_N - 1);   // lanes 0..63 carry lse2, 64..127 delta
+  auto load_scalar = [&](int row0) { return (sr < AT_N ? lp : dp_)[min(row0 + (sr & (AT_N - 1)), t - 1)]; };
+  auto put = [&](int buf, const TileRegs& qr, const TileRegs& gr, float sc) {
+    tile_store(s_q[buf], qr);
+    tile_store(s_g[buf], gr);
+    if (tid < AT_N) s_ls[buf][tid] = sc;
+    else if (tid < 2 * AT_N) s_dl[buf][tid - AT_N] = sc;
+  };
+  TileRegs qr = tile_load(qp, sqk, first * AT_N, t), gr = tile_load(gp, so, first * AT_N, t);
+  float sc = load_scalar(first * AT_N);
+  put(first & 1, qr, gr, sc);
+  __syncthreads();
+  for (int j = first; j < ntiles; ++j) {
+    const int q0 = j * AT_N, cur = j & 1;
+    if (j + 1 < ntiles) {
+      qr = tile_load(qp, sqk, q0 + AT_N, t);
+      gr = tile_load(gp, so, q0 + AT_N, t);
+      sc = load_scalar(q0 + AT_N);
+    }
+    if (q0 + AT_N - 1 >= w0 && w0 < t) {   // the tile has queries at or past this wave's first key
+      const bool edge = q0 < w0 + 31 || q0 + AT_N > t;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        f32x16 s = zero16(), dp = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          s = mfma(rows_frag(s_q[cur], 32 * i, ks, lane), kf[ks], s);
+          dp = mfma(rows_frag(s_g[cur], 32 * i, ks, lane), vf[ks], dp);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int r0 = 32 * i + 8 * g + 4 * half;
+          const float4 l4 = *reinterpret_cast<const float4*>(&s_ls[cur][r0]);
+          const float4 d4 = *reinterpret_cast<const float4*>(&s_dl[cur][r0]);
+          const float ll[4] = {l4.x, l4.y, l4.z, l4.w}, dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int r = 4 * g + k;
+            const bool off = edge && (key > q0 + r0 + k || q0 + r0 + k >= t);
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ll[k]));
+            s[r] = off ? 0.f : p;
+            dp[r] = off ? 0.f : p * (dp[r] - dd[k]);
+          }
+        }
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const bf16x8 pf = operand(s, st), df = operand(dp, st);
+#pragma unroll
+          for (int d = 0; d < 2; ++d) {
+            dv[d] = mfma(cols_frag(s_g[cur], 32 * i + 16 * st, 32 * d, lane), pf, dv[d]);
+            dk[d] = mfma(cols_frag(s_q[cur], 32 * i + 16 * st, 32 * d, lane), df, dk[d]);
+          }
+        }
+      }
+    }
+    if (j + 1 < ntiles) {
+      put(cur ^ 1, qr, gr, sc);
+      __syncthreads();
+    }
+  }
+  if (key < t) {
+    bf16_t* row = dqkv + ((int64_t)b * t + key) * sv + head * 64;
+    store_unrotated(row + heads * 64, dk[0], dk[1], cosT, sinT, key, half, scale);
+    bf16_t* vo = row + 2 * heads * 64 + 4 * half;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2*>(vo + 32 * d + 8 * g) =
+            make_uint2(pack2(dv[d][4 * g], dv[d][4 * g + 1]), pack2(dv[d][4 * g + 2], dv[d][4 * g + 3]));
+  }
+}
+
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool al2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }
 inline bool dtype_ok(int dt) { return dt == LDR_BF16 || dt == LDR_F16; }
@@ -463,6 +887,62 @@ int llm_next_token_loss_bwd(const void* logits, const int64_t* ids, const float*
                                              static_cast<hipStream_t>(stream), static_cast<const T*>(logits), ids, lse,
                                              dloss, static_cast<T*>(dlogits), t, vocab,
                                              count > 0 ? (float)(1.0 / count) : 0.f))
+  return launched();
+}
+
+int llm_rotary(const void* qkv, const float* cosT, const float* sinT, void* qk, int64_t b, int64_t t, int64_t heads,
+               void* stream) {
+  if (b < 0 || t < 0 || heads < 1 || b * t * heads > 0x7fffffff) return LDR_E_ARG;
+  if (b * t == 0) return LDR_OK;
+  if (!qkv || !cosT || !sinT || !qk) return LDR_E_ARG;
+  if (!al16(qkv) || !al16(cosT) || !al16(sinT) || !al16(qk)) return LDR_E_ALIGN;
+  const int64_t n = b * t * heads * 8;
+  hipLaunchKernelGGL(k_rotary, dim3(grid_of((n + WG - 1) / WG, 8192)), dim3(WG), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const bf16_t*>(qkv), cosT, sinT, static_cast<bf16_t*>(qk), n, (int)t, (int)heads);
+  return launched();
+}
+
+static int attn_grid(int64_t b, int64_t t, int64_t heads, unsigned* grid) {
+  if (b < 0 || t < 0 || heads < 1 || b * heads > 0x7fffff || t > 0x7fffff) return LDR_E_ARG;
+  const int64_t g = 8 * ((b * heads + 7) / 8) * ((t + AT_M - 1) / AT_M);
+  if (g > 0x7fffffff) return LDR_E_SHAPE;
+  *grid = (unsigned)g;
+  return LDR_OK;
+}
+
+int llm_attn_fwd(const void* qk, const void* qkv, void* out, float* lse2, int64_t b, int64_t t, int64_t heads,
+                 void* stream) {
+  unsigned grid = 0;
+  const int e = attn_grid(b, t, heads, &grid);
+  if (e) return e;
+  if (grid == 0) return LDR_OK;
+  if (!qk || !qkv || !out || !lse2) return LDR_E_ARG;
+  if (!al16(qk) || !al16(qkv) || !al16(out)) return LDR_E_ALIGN;
+  hipLaunchKernelGGL(k_attn_fwd, dim3(grid), dim3(256), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const bf16_t*>(qk), static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(out), lse2,
+                     (int)(b * heads), (int)t, (int)heads, AT_SCALE * LOG2E);
+  return launched();
+}
+
+int llm_attn_bwd(const void* qk, const void* qkv, const void* out, const void* dout, const float* lse2,
+                 const float* cosT, const float* sinT, float* delta, void* dqkv, int64_t b, int64_t t, int64_t heads,
+                 void* stream) {
+  unsigned grid = 0;
+  int e = attn_grid(b, t, heads, &grid);
+  if (e) return e;
+  if (grid == 0) return LDR_OK;
+  if (!qk || !qkv || !out || !dout || !lse2 || !cosT || !sinT || !delta || !dqkv) return LDR_E_ARG;
+  if (!al16(qk) || !al16(qkv) || !al16(out) || !al16(dout) || !al16(cosT) || !al16(sinT) || !al16(dqkv))
+    return LDR_E_ALIGN;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(k_attn_bwd_q, dim3(grid), dim3(256), 0, st, static_cast<const bf16_t*>(qk),
+                     static_cast<const bf16_t*>(qkv), static_cast<const bf16_t*>(out),
+                     static_cast<const bf16_t*>(dout), lse2, cosT, sinT, delta, static_cast<bf16_t*>(dqkv),
+                     (int)(b * heads), (int)t, (int)heads, AT_SCALE * LOG2E, AT_SCALE);
+  if ((e = launched())) return e;
+  hipLaunchKernelGGL(k_attn_bwd_kv, dim3(grid), dim3(256), 0, st, static_cast<const bf16_t*>(qk),
+                     static_cast<const bf16_t*>(qkv), static_cast<const bf16_t*>(dout), lse2, delta, cosT, sinT,
+                     static_cast<bf16_t*>(dqkv), (int)(b * heads), (int)t, (int)heads, AT_SCALE * LOG2E, AT_SCALE);
   return launched();
 }
 

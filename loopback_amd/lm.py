@@ -11,7 +11,8 @@ Plain Loop). Init: every Linear and the embedding N(0, initializer_range), RMSNo
 
 MI355X choices (not the reference's parameterization): q, k, v come from one fused projection and the MLP's gate and
 up from another (one GEMM each instead of three / two); in 16 bits the norms, SwiGLU and the loss run in this
-package's own kernels (lm_ops), the residual's add and its gradient inside the norms; attention is torch's SDPA restricted to its flash and
+package's own kernels (lm_ops), the residual's add and its gradient inside the norms, and so does bf16 attention at
+head width 64 with its rotation; other attention is torch's SDPA restricted to its flash and
 memory-efficient kernels in 16-bit (never the math path's batched products in bf16).
 
     python -m loopback_amd.lm --steps 10 --warmup 3            # config 5: the Loopback LM step, tokens/s
@@ -120,6 +121,14 @@ def attention_kernels(dtype):
     return sdpa_kernel(kinds)
 
 
+def _hooked(m: nn.Module) -> bool:
+    """Whether calling m runs more than its forward (hooks of its own, or of every module)."""
+    g = nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
@@ -129,16 +138,24 @@ class Attention(nn.Module):
         self.rotary = Rotary(self.dh, cfg.rope_theta)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        B, T, D = x.shape
-        qkv = self.qkv(x).view(B, T, 3, self.h, self.dh)
+        qkv = self.qkv(x)
+        if ops.attention_native(qkv, self.dh) and type(self.rotary) is Rotary and not _hooked(self.rotary):
+            cos, sin = self.rotary.tables(x.shape[1], x.device, qkv.dtype)
+            return self.o(ops.rotary_attention(qkv, cos, sin, self.h, self.attend))
+        return self.o(self.attend(qkv))
+
+    def attend(self, qkv: torch.Tensor) -> torch.Tensor:
+        """The rotation and attention in torch operations: (B, T, 3 D) -> (B, T, D)."""
+        B, T, _ = qkv.shape
+        qkv = qkv.view(B, T, 3, self.h, self.dh)
         q, k = self.rotary(qkv[:, :, :2]).permute(2, 0, 3, 1, 4).unbind(0)   # (B, H, T, dh) views
         v = qkv[:, :, 2].transpose(1, 2)
-        if x.is_cuda:
-            with attention_kernels(x.dtype):
+        if qkv.is_cuda:
+            with attention_kernels(qkv.dtype):
                 a = F.scaled_dot_product_attention(q, k, v.contiguous(), is_causal=True)
         else:
             a = F.scaled_dot_product_attention(q, k, v, is_causal=True)
-        return self.o(a.transpose(1, 2).reshape(B, T, D))
+        return a.transpose(1, 2).reshape(B, T, self.h * self.dh)
 
 
 class SwiGLU(nn.Module):
@@ -158,14 +175,6 @@ class RMSNorm(nn.RMSNorm):
         if ops.norm_native(x, self.weight):
             return ops.add_rms_norm(x, None, self.weight, self.eps)[1]
         return super().forward(x)
-
-
-def _hooked(m: nn.Module) -> bool:
-    """Whether calling m runs more than its forward (hooks of its own, or of every module)."""
-    g = nn.modules.module
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
-                or g._global_backward_pre_hooks)
 
 
 def add_norm(norm: nn.Module, x: torch.Tensor, add: torch.Tensor | None = None):

@@ -1,6 +1,6 @@
 """The language model's row operations on the HIP kernels of libloopback_lm.so (include/loopback_lm.h): RMSNorm with the
-residual's add before it and the residual's gradient folded into its backward, SwiGLU, and the next-token cross
-entropy on 16-bit logits.
+residual's add before it and the residual's gradient folded into its backward, SwiGLU, the next-token cross entropy on
+16-bit logits, and causal rotary attention in bf16 at head width 64.
 
 `native(...)` says whether the kernels take a call: plain 16-bit GPU tensors of one dtype on one device, no transform
 or tracer that has to see torch operations (torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else --
@@ -34,6 +34,9 @@ SIGNATURES = {
     "llm_swiglu_bwd": (_i32, [_p, _p, _p, _i64, _i64, _i32, _p]),
     "llm_next_token_loss_fwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
     "llm_next_token_loss_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
+    "llm_rotary": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
+    "llm_attn_fwd": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
+    "llm_attn_bwd": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
 }
 
 
@@ -236,3 +239,48 @@ def next_token_loss(logits: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
             and 0 < ids.numel() < 2 ** 31):
         return _NextTokenLoss.apply(logits, ids)
     return _loss_torch(ids)(logits)
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# causal rotary attention
+# ---------------------------------------------------------------------------------------------------------------
+class _RotaryAttention(torch.autograd.Function):
+    """qkv (b, t, 3 heads 64) -> (b, t, heads 64). Saves the rotated q and k, qkv (for v), the output and the queries'
+    sums of exponentials. `again`: the torch form, for a backward that is differentiated."""
+
+    @staticmethod
+    def forward(ctx, qkv, cos, sin, heads, again):
+        b, t, _ = qkv.shape
+        qk = torch.empty((b, t, 2, heads, 64), device=qkv.device, dtype=qkv.dtype)
+        out = torch.empty((b, t, heads * 64), device=qkv.device, dtype=qkv.dtype)
+        lse2 = torch.empty((b * heads, t), device=qkv.device, dtype=torch.float32)
+        st = _stream(qkv)
+        _run("llm_rotary", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), qk.data_ptr(), b, t, heads, st)
+        _run("llm_attn_fwd", qk.data_ptr(), qkv.data_ptr(), out.data_ptr(), lse2.data_ptr(), b, t, heads, st)
+        ctx.heads, ctx.again = heads, again
+        ctx.save_for_backward(qkv, qk, out, lse2, cos, sin)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        qkv, qk, out, lse2, cos, sin = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _again(ctx.again, [qkv], [True], (dout,))[0], None, None, None, None
+        b, t, _ = qkv.shape
+        dout = _dense(dout, out)
+        delta = torch.empty_like(lse2)
+        dqkv = torch.empty_like(qkv)
+        _run("llm_attn_bwd", qk.data_ptr(), qkv.data_ptr(), out.data_ptr(), dout.data_ptr(), lse2.data_ptr(),
+             cos.data_ptr(), sin.data_ptr(), delta.data_ptr(), dqkv.data_ptr(), b, t, ctx.heads, _stream(qkv))
+        return dqkv, None, None, None, None
+
+
+def attention_native(qkv: torch.Tensor, head_dim: int) -> bool:
+    """Whether rotary_attention takes qkv (b, t, 3 heads head_dim): bf16, head width 64, not empty."""
+    return (head_dim == 64 and qkv.dtype is torch.bfloat16 and native(qkv) and qkv.dim() == 3 and qkv.numel() > 0
+            and _rows_ok(qkv))
+
+
+def rotary_attention(qkv, cos, sin, heads, again):
+    """Causal attention over the rotated q and k of qkv; cos and sin (t, 64) fp32, contiguous, both halves alike."""
+    return _RotaryAttention.apply(qkv, cos, sin, heads, again)
