@@ -1,5 +1,5 @@
 """Build libloopback_read.so (the read's kernels and C ABI) and libloopback_lm.so (the language model's) in-tree with
-hipcc for gfx950 (MI355X).
+hipcc for gfx950 (MI355X), and _host.so, the Python module's launch path, with g++ against torch's headers.
 
     python -m loopback_amd.build                          # compile, print the commands
     python -m loopback_amd.build -D LDR_RF_GRID=768 ...   # with launch settings other than the measured defaults
@@ -26,6 +26,8 @@ INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(HERE, "libloopback_read.so")
 LM_SRC = os.path.join(HERE, "csrc", "loopback_lm.hip")
 LM_LIB = os.path.join(HERE, "libloopback_lm.so")
+HOST_SRC = os.path.join(HERE, "csrc", "host.cpp")
+HOST_LIB = os.path.join(HERE, "_host.so")
 # A test fixture: the same source built with the alternative kernel shapes -- the write in the matrix cores' layout
 # for every width and dtype (LDR_WM_ROWS=0, LDR_W32_ROWS=0), the read forward in 256-lane workgroups for every read
 # (LDR_RF_BIG=0) -- so the
@@ -69,12 +71,29 @@ def _start(src: str, lib: str, verbose: bool, defines) -> tuple:
     return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True), tmp, lib
 
 
+def _start_host(verbose: bool) -> tuple:
+    """The host extension: plain C++, linked to the libtorch of the running interpreter."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST_LIB + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           *[f"-I{i}" for i in include_paths()], f"-I{sysconfig.get_paths()['include']}", "-o", tmp, HOST_SRC,
+           f"-L{lib}", "-lc10", "-ltorch_cpu", "-ltorch_python", f"-Wl,-rpath,{lib}"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True), tmp, HOST_LIB
+
+
 def _wait(job) -> str | None:
     """Wait for one compile; install its output, or return its error message."""
     proc, tmp, lib = job
     out, err = proc.communicate()
     if proc.returncode != 0:
-        return f"hipcc failed ({proc.returncode}) for {os.path.basename(lib)}:\n{out}\n{err}"
+        return f"the compiler failed ({proc.returncode}) for {os.path.basename(lib)}:\n{out}\n{err}"
     os.replace(tmp, lib)
     return None
 
@@ -109,14 +128,14 @@ def build(verbose: bool = True, defines=None, fixtures: bool = True) -> str:
     path. Every compile started is waited for before any error is raised. A library's failure raises; a test
     fixture's is reported on stderr and does not fail the library's build (the GPU tests that load the fixture then
     fail on its absence). defines: NAME=VALUE launch settings (see the module docstring)."""
-    jobs = [_start(SRC, LIB, verbose, defines), _start(LM_SRC, LM_LIB, verbose, [])]
+    jobs = [_start(SRC, LIB, verbose, defines), _start(LM_SRC, LM_LIB, verbose, []), _start_host(verbose)]
     if fixtures:
         jobs.append(_start(SRC, TEST_LIB_ALT, verbose, list(defines or []) + ALT_DEFINES))
     errors = [_wait(job) for job in jobs]
-    for e in errors[:2]:
+    for e in errors[:3]:
         if e is not None:
             raise RuntimeError(e)
-    fixture_errors = [e for e in errors[2:] if e is not None]
+    fixture_errors = [e for e in errors[3:] if e is not None]
     if fixtures and not fixture_errors:
         try:
             build_abi_smoke(verbose)

@@ -38,12 +38,15 @@ Layouts:
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import weakref
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib as L
+from . import _host as H      # the launch path (csrc/host.cpp), bound below to the library _lib loaded
 
 __all__ = ["rstd_ref", "rstd", "fused_read_supported", "FusedDattnRead", "DattnGradAccum", "FusedDattnReadAcc",
            "DattnStack", "FusedDattnReadStk", "FusedCombineStk", "_alias"]
@@ -56,11 +59,6 @@ ANY_MAX_SOURCES = L.ANY_MAX_SOURCES
 # ---------------------------------------------------------------------------------------------------------------
 # plumbing
 # ---------------------------------------------------------------------------------------------------------------
-def _p(t: torch.Tensor | None):
-    """A tensor's device address for a pointer argument (an int; None is NULL)."""
-    return None if t is None else t.data_ptr()
-
-
 _raw_stream = torch._C._cuda_getCurrentRawStream   # the device's current hipStream_t, as an int
 
 
@@ -93,7 +91,7 @@ def _aligned(t: torch.Tensor) -> bool:
 def _f32(t: torch.Tensor) -> torch.Tensor:
     """t as a contiguous fp32 tensor for a kernel argument (t itself when it already is one)."""
     if t.dtype is torch.float32 and t.is_contiguous():
-        return t.detach()
+        return t.detach() if t.requires_grad else t
     return t.detach().float().contiguous()
 
 
@@ -145,6 +143,7 @@ def _dev_addrs(addrs, dev: torch.device) -> torch.Tensor:
     return host.to(dev, non_blocking=True)
 
 
+@functools.lru_cache(maxsize=64)
 def _b1_parts(n_tok: int, d: int) -> int:
     """Rows of backward pass 1's query-gradient partials, one per workgroup: as many as fill the GPU (for the scalar
     kernels' widths one per four tokens)."""
@@ -152,9 +151,9 @@ def _b1_parts(n_tok: int, d: int) -> int:
 
 
 class _Src:
-    """The sources of one read: host address arrays (v, r; dr for the scale gradients) for the row-layout entry
-    points when `fast` and for the unaligned-row ones when `rows`, else device address arrays for the any-shape
-    ones."""
+    """The sources of one read: host address tables (v, r; dr for the scale gradients; tuples of tensors or arrays of
+    addresses) for the row-layout entry points when `fast` and for the unaligned-row ones when `rows`, else device
+    address arrays for the any-shape ones."""
     __slots__ = ("fast", "rows", "v", "r", "dr")
 
     def __init__(self, fast: bool, rows: bool, v, r, dr=None):
@@ -162,14 +161,15 @@ class _Src:
 
     @staticmethod
     def of(fast: bool, rows: bool, values, rstds, dev, drs=None):
-        addrs = (lambda ts: L.u64_array(t.data_ptr() for t in ts)) if fast or rows else \
-                (lambda ts: _dev_addrs((t.data_ptr() for t in ts), dev))
         if not fast:
             _refuse_capture()
+        if fast or rows:   # the tensors themselves: the launch takes their addresses
+            return _Src(fast, rows, values, rstds, drs)
+        addrs = lambda ts: _dev_addrs((t.data_ptr() for t in ts), dev)
         return _Src(fast, rows, addrs(values), addrs(rstds), None if drs is None else addrs(drs))
 
     def ptrs(self):
-        """(v, r) as entry-point arguments: host arrays, or the device arrays' addresses."""
+        """(v, r) as entry-point arguments: host tables, or the device arrays' addresses."""
         return (self.v, self.r) if self.fast or self.rows else (self.v.data_ptr(), self.r.data_ptr())
 
     def dr_ptr(self):
@@ -182,15 +182,13 @@ def _read(src: _Src, n: int, q, dots, stored: bool, base, h0, beta: float, cbar,
     and kept in dots: the row-layout kernels when src.fast, else the unaligned-row or any-shape ones. cols: n (cbar, c0 as the read
     takes them) or n - 1 (the previous read's coefficients and prior, scaled by lam, the newest entry implied)."""
     v, r = src.ptrs()
-    tail = (_p(base), _p(h0), float(beta), _p(cbar), cols, _p(c0), cols, float(lam), _inv_sqrt(d), _p(out), _p(tc),
-            _p(prob), _p(next_prior), n_tok, d, dt, st)
+    tail = (base, h0, beta, cbar, cols, c0, cols, lam, _inv_sqrt(d), out, tc, prob, next_prior, n_tok, d, dt, st)
     if not src.fast:
-        _run("read_fwd_rows" if src.rows else "read_fwd_any", v, r, n, None if stored else _p(q), _p(dots), n_tok,
-             *tail)
+        _run("read_fwd_rows" if src.rows else "read_fwd_any", v, r, n, None if stored else q, dots, n_tok, *tail)
     elif stored:
-        _run("read_fwd", v, r, n, _p(dots), n_tok, *tail)
+        _run("read_fwd", v, r, n, dots, n_tok, *tail)
     else:
-        _run("read_fwd_online", v, r, n, _p(q), _p(dots), n_tok, *tail)
+        _run("read_fwd_online", v, r, n, q, dots, n_tok, *tail)
 
 
 # Optional launch observer: a callable name -> context manager, entered around every library call (the bench uses it
@@ -198,14 +196,16 @@ def _read(src: _Src, n: int, q, dots, stored: bool, base, h0, beta: float, cbar,
 _TIMER = None
 
 
-# the entry points, bound once (name without the ldr_ prefix -> ctypes function with its signature)
-_FN = {name[4:]: getattr(_LIB, name) for name in L.SIGNATURES}
+# the entry points, bound once (name without the ldr_ prefix -> the builtin that launches it)
+_FN = {name[4:]: getattr(H, name[4:]) for name in L.SIGNATURES
+       if H.bind(name, ctypes.cast(getattr(_LIB, name), ctypes.c_void_p).value)}
 
 # the kernel family an entry point's launches are reported under, where it is not the entry point's own name
 _FAMILY = {"read_bwd1_rows": "read_bwd1"}
 
 
 def _run(name: str, *args) -> None:
+    """One entry point: pointer arguments are tensors, addresses or None (NULL)."""
     fn = _FN[name]
     if _TIMER is None:
         code = fn(*args)
@@ -235,7 +235,7 @@ class _Rstd(torch.autograd.Function):
         d = xc.shape[-1]
         n_tok = xc.numel() // d
         r = torch.empty(xc.shape[:-1] + (1,), device=xc.device, dtype=torch.float32)
-        _run("rstd_fwd", _p(xc), _p(r), n_tok, d, float(eps), _dtype_code(xc.dtype), _stream(xc.device))
+        _run("rstd_fwd", xc, r, n_tok, d, float(eps), _dtype_code(xc.dtype), _stream(xc.device))
         ctx.save_for_backward(xc, r)
         return r
 
@@ -246,7 +246,7 @@ class _Rstd(torch.autograd.Function):
         n_tok = xc.numel() // d
         gx = torch.empty_like(xc)
         grc = gr.float().contiguous()
-        _run("rstd_bwd", _p(xc), _p(r), _p(grc), _p(gx), n_tok, d, _dtype_code(xc.dtype), _stream(xc.device))
+        _run("rstd_bwd", xc, r, grc, gx, n_tok, d, _dtype_code(xc.dtype), _stream(xc.device))
         return gx, None
 
 
@@ -307,11 +307,8 @@ def _forward_impl(ctx, q, base, cbar, c0, srcs):
     c0c = _f32(c0)
     cbar_c = _f32(cbar)
     base_c = base.detach().contiguous()
-    out = torch.empty_like(base_c)
-    tc = torch.empty((n_tok, n), device=dev, dtype=torch.float32)
     grad = any(ctx.needs_input_grad)      # else no backward: the probabilities are not stored
-    prob = torch.empty((n_tok, n), device=dev, dtype=torch.float32) if grad else None
-    dots = torch.empty((n, n_tok), device=dev, dtype=torch.float32)
+    out, tc, prob, _, dots = H.read_buffers(base_c, n_tok, n, grad, False, True)
     src = _Src.of(_fast(d, n, base_c, qc, *values), _rows(d, n), values, rstds, dev)
     _read(src, n, qc, dots, False, base_c, None, 0.0, cbar_c, n, c0c, 1.0, out, tc, prob, None, n_tok, d, dt, st)
     if grad:
@@ -321,35 +318,35 @@ def _forward_impl(ctx, q, base, cbar, c0, srcs):
 
 
 def _bwd1(src: _Src, n, g, gt, prob, dots, tc, cbar_c, c0c, dr_accum, wz, wz_stride, n_tok, d,
-          dtype, dev, cols=None, lam=1.0, g_prop=None, g_h0=None, beta=0.0, dq=None, part=None):
+          dtype, dev, cols=None, lam=1.0, g_prop=None, g_h0=None, beta=0.0, part=None):
     """Pass 1 of the backward plus the dq reduction; returns (dq fp32, dcbar [n_tok, cols]). src: the sources with the
     scale gradients' addresses (src.dr), on the row-layout kernel when src.fast (chosen with g among its rows;
     g_prop and g_h0 are fresh, aligned allocations), else on the any-shape kernel. prob and dots are the
     forward's probabilities [n_tok, n] and raw scores [n, >= n_tok] (row stride dots.stride(0)). cols = n: cbar_c and c0c
     are the read's own; cols = n - 1: they are the previous read's coefficients and prior (scaled by lam, the newest
     entry implied) and dcbar is the gradient of those coefficients. g_prop / g_h0 receive the iteration-end blend's
-    gradients when given. dq: an fp32 row of d to reduce the query gradient into (else a new one). part: a
-    [bwd1_parts, d] view (any row stride) that takes the per-workgroup partials instead, left for the caller to
-    reduce (dq is then None)."""
+    gradients when given. wz: the tensor (or address) of the pass-2 scalars. part: (address, rows, row stride) of the
+    per-workgroup partials, left for the caller to reduce (dq is then None)."""
     st = _stream(dev)
     cols = n if cols is None else cols
     gt_c = None if gt is None else gt.reshape(n_tok, n).float().contiguous()
     dcbar = torch.empty((n_tok, cols), device=dev, dtype=torch.float32)
-    parts = _b1_parts(n_tok, d) if part is None else part.shape[0]
-    dq_part = torch.empty((parts, d), device=dev, dtype=torch.float32) if part is None else part
+    if part is None:
+        parts, stride = _b1_parts(n_tok, d), d
+        dq_part = torch.empty((parts, d), device=dev, dtype=torch.float32)
+    else:
+        dq_part, parts, stride = part
+    if src.fast and not _fast(d, n, g, g_prop, g_h0):   # the caller chose src with g among its rows
+        raise RuntimeError("delta_attnres HIP read: host source tables with rows the row-layout kernels refuse")
     v, r = src.ptrs()
-    head = (v, r, n, _p(g), _p(gt_c), _p(prob), _p(dots), dots.stride(0), _p(tc), _p(cbar_c), cols, _p(c0c), cols,
-            float(lam), _inv_sqrt(d), _p(dcbar), cols, src.dr_ptr(), int(dr_accum), _p(wz), wz_stride, _p(dq_part))
-    tail = (_p(g_prop), _p(g_h0), float(beta), n_tok, d, dtype, st)
-    if src.fast:
-        if not _fast(d, n, g, g_prop, g_h0):   # the caller chose src with g among its rows
-            raise RuntimeError("delta_attnres HIP read: host source tables with rows the row-layout kernels refuse")
-    _run("read_bwd1_rows" if src.fast or src.rows else "read_bwd1_any", *head, parts, dq_part.stride(0), *tail)
+    _run("read_bwd1_rows" if src.fast or src.rows else "read_bwd1_any", v, r, n, g, gt_c, prob, dots, dots.stride(0),
+         tc, cbar_c, cols, c0c, cols, lam, _inv_sqrt(d), dcbar, cols, src.dr_ptr(), int(dr_accum), wz, wz_stride,
+         dq_part, parts, stride, g_prop, g_h0, beta, n_tok, d, dtype, st)
     if part is not None:
         return None, dcbar
-    dq = torch.empty(d, device=dev, dtype=torch.float32) if dq is None else dq
+    dq = torch.empty(d, device=dev, dtype=torch.float32)
     if n_tok > 0:
-        _run("reduce_rows", _p(dq_part), parts, d, _p(dq), st)
+        _run("reduce_rows", dq_part, parts, d, dq, st)
     else:
         dq.zero_()
     return dq, dcbar
@@ -366,25 +363,22 @@ def _backward_impl(ctx, g, gt, dv, accum):
     dev = v0.device
     dt = _dtype_code(v0.dtype)
     g = g.to(v0.dtype).contiguous()
-    dr = torch.empty((n, n_tok), device=dev, dtype=torch.float32)
+    drs = torch.empty((n, *rstds[0].shape), device=dev, dtype=torch.float32).unbind(0)
     wz = torch.empty((n, n_tok, 2), device=dev, dtype=torch.float32)
     fast = _fast(d, n, g, qc, *values, *dv)
-    src = _Src.of(fast, _rows(d, n), values, rstds, dev, drs=[dr[i] for i in range(n)])
+    src = _Src.of(fast, _rows(d, n), values, rstds, dev, drs=drs)
     dq, dcbar = _bwd1(src, n, g, gt, prob, dots, tc, cbar_c, c0c, False, wz, n_tok, n_tok, d, dt, dev)
     for t in dv:
         if t.dtype != v0.dtype or not t.is_contiguous() or t.numel() != v0.numel():
             raise RuntimeError("delta_attnres HIP read: gradient buffers must match the sources")
     if fast:
-        _run("read_bwd2_list", L.u64_array(t.data_ptr() for t in dv), n, int(bool(accum)), _p(g), _p(qc), _p(wz),
-             n_tok, n_tok, d, dt, _stream(dev))
+        _run("read_bwd2_list", dv, n, int(bool(accum)), g, qc, wz, n_tok, n_tok, d, dt, _stream(dev))
     elif src.rows:
-        _run("read_bwd2_list_rows", L.u64_array(t.data_ptr() for t in dv), n, int(bool(accum)), _p(g), _p(qc), _p(wz),
-             n_tok, n_tok, d, dt, _stream(dev))
+        _run("read_bwd2_list_rows", dv, n, int(bool(accum)), g, qc, wz, n_tok, n_tok, d, dt, _stream(dev))
     else:
         dvt = _dev_addrs((t.data_ptr() for t in dv), dev)
-        _run("read_bwd2_list_any", _p(dvt), n, int(bool(accum)), _p(g), _p(qc), _p(wz), n_tok, n_tok, d, dt,
-             _stream(dev))
-    return dq.to(ctx.q_dtype), g, dcbar.view(*ctx.base_shape[:-1], n), [dr[i].view_as(rstds[i]) for i in range(n)]
+        _run("read_bwd2_list_any", dvt.data_ptr(), n, int(bool(accum)), g, qc, wz, n_tok, n_tok, d, dt, _stream(dev))
+    return dq.to(ctx.q_dtype), g, dcbar.view(*ctx.base_shape[:-1], n), drs
 
 
 class FusedDattnRead(torch.autograd.Function):
@@ -449,10 +443,14 @@ def _alias(stack_tensor: torch.Tensor, s: int) -> torch.Tensor:
     """Slice s of a stack as a tensor that shares its storage but is not an autograd view of it (fused_dattn.py:
     629-636): later slices are written in place, and autograd forbids a custom Function to return a view whose base
     is then modified."""
-    sl = stack_tensor[s]
-    out = torch.empty(0, dtype=stack_tensor.dtype, device=stack_tensor.device)
-    out.set_(stack_tensor.untyped_storage(), sl.storage_offset(), sl.shape, sl.stride())
-    return out
+    return H.alias(stack_tensor, s)
+
+
+def _bypass() -> bool:
+    """Whether a call may skip its autograd Function: gradients are off, and nothing that has to see the Function --
+    torch.func transforms, forward-mode AD, a tracer -- is on."""
+    return not (torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch.jit.is_tracing()
+                or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None)
 
 
 def _pair(s: int, i: int) -> int:
@@ -528,12 +526,12 @@ class DattnStack:
             self.DOTS = torch.empty((max(1, nq), n_steps, b * t), dtype=torch.float32, device=device)
             if nq > 0:   # the queries' bf16 parts: the write's matrix-core operand (every update dtype)
                 self.QB = torch.empty(int(L.LIB.ldr_query_parts_elems(nq, d)), dtype=torch.bfloat16, device=device)
-                _run("split_queries", _p(self.Q), nq, d, _p(self.QB), _stream(self.Q.device))
+                _run("split_queries", self.Q, nq, d, self.QB, _stream(self.Q.device))
 
     def write(self, s: int, h: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         """V[s] = h - x, returned as the update tensor (an alias of the stack's slice, with the autograd edge to
         h and x). The write also stores the update's scale R[s], which rstd(s, ...) then returns."""
-        v, r = _WriteDelta.apply(self, s, h, x)
+        v, r = _write(self, s, h, x) if _bypass() else _WriteDelta.apply(self, s, h, x)
         self.wout[s] = (weakref.ref(v), r)
         return v
 
@@ -573,6 +571,16 @@ class DattnStack:
             return False
         return True
 
+    def wz(self, step: int) -> int:
+        """The address of read `step`'s pairs in WZ (its sources' rows follow one another)."""
+        return self.WZ.data_ptr() + _pair(step, 0) * self.WZ.stride(0) * 4
+
+    def keep(self, step: int, g: torch.Tensor, q: torch.Tensor) -> None:
+        """Keep read `step`'s output gradient and query for the updates' gradients: the tensors, their addresses for the
+        kernel tables, and whether the row-layout kernels take them."""
+        gp, qp = g.data_ptr(), q.data_ptr()
+        self.bwd[step] = (g, q, gp, qp, gp % 16 == 0 and qp % 16 == 0)
+
 
 def _slice_table(t: torch.Tensor):
     """Device addresses of t[0], t[1], ... (a stack's slices), as the kernels' per-source tables."""
@@ -608,27 +616,56 @@ def _assemble(stack: DattnStack, s: int, gr):
                               or not added[0].is_contiguous()):
         added = (added[0].to(v.dtype).contiguous().view(v.shape), added[1])
     bwd = stack.bwd
-    fast = stack.fast_d and _fast(stack.d, len(reads), None if added is None else added[0],
-                                  *[bwd[k][0] for k in reads], *[bwd[k][1] for k in reads])
-    tables = None
+    m = len(reads)
+    fast = (stack.fast_d and m <= MAX_SOURCES and (added is None or _aligned(added[0]))
+            and all(bwd[k][4] for k in reads))
+    tables = (None, None, None)
     if reads:
         wz0, wz_row = stack.WZ.data_ptr(), stack.WZ.stride(0) * stack.WZ.element_size()
         tables = ([bwd[k][2] for k in reads], [wz0 + _pair(k, s) * wz_row for k in reads], [bwd[k][3] for k in reads])
-    args = (len(reads), _p(v), _p(stack.R[s]), _p(grc), _p(None if added is None else added[0]),
-            0.0 if added is None else float(added[1]), int(stack.per_read), _p(dv), _p(dv_neg), stack.n_tok, stack.d,
+    args = (m, v, stack.R.data_ptr() + s * stack.n_tok * 4, grc, None if added is None else added[0],
+            0.0 if added is None else added[1], int(stack.per_read), dv, dv_neg, stack.n_tok, stack.d,
             _dtype_code(v.dtype), _stream(v.device))
     if fast:
-        _run("dv_assemble", *([L.u64_array(t) for t in tables] if tables else [None] * 3), *args)
-    elif _rows(stack.d, len(reads)):
+        _run("dv_assemble", *tables, *args)
+    elif _rows(stack.d, m):
         _refuse_capture()
-        _run("dv_assemble_rows", *([L.u64_array(t) for t in tables] if tables else [None] * 3), *args)
+        _run("dv_assemble_rows", *tables, *args)
     else:
-        dev_tabs = [_dev_addrs(t, v.device) for t in tables] if tables else None
-        _run("dv_assemble_any", *([t.data_ptr() for t in dev_tabs] if dev_tabs else [None] * 3), *args)
+        dev_tabs = [_dev_addrs(t, v.device) for t in tables] if reads else None
+        _run("dv_assemble_any", *([t.data_ptr() for t in dev_tabs] if dev_tabs else tables), *args)
     stack.assembled.add(s)
     for k in [k for k in bwd if all(j in stack.assembled for j in range(k + 1))]:
         del bwd[k]                        # every update read by read k has its gradient: drop g_k
     return dv, dv_neg, added
+
+
+def _write(stack: DattnStack, s: int, h: torch.Tensor, x: torch.Tensor):
+    """The write of update s: (the update, its scale), aliases of the stack's slices."""
+    stack.wh[s] = weakref.ref(h)
+    out = _alias(stack.V, s)
+    r = _alias(stack.R, s)
+    V = stack.V
+    whole = (h.is_cuda and x.is_cuda and h.is_contiguous() and x.is_contiguous() and h.dtype == V.dtype == x.dtype
+             and h.numel() == x.numel() == stack.n_tok * stack.d and h.shape[-1] == stack.d)
+    if whole and stack.fast_d and _aligned(h) and _aligned(x):
+        nq, j_lo, dptr, jstride = 0, 0, None, stack.n_steps * stack.n_tok
+        if stack.DOTS is not None:
+            nq = stack.Q.shape[0]
+            j_lo = min(max(0, s - 1), nq)         # read s' >= s uses query s' - 1: queries j_lo .. nq - 1
+            if j_lo < nq:                         # DOTS[j_lo, s]
+                dptr = stack.DOTS.data_ptr() + (j_lo * jstride + s * stack.n_tok) * 4
+        _run("write_dots", h, x, out, r, stack.Q, stack.QB, nq, j_lo, dptr, stack.n_tok, stack.d, jstride, stack.eps,
+             _dtype_code(V.dtype), _stream(V.device))
+        stack.r_done[s] = True
+    elif whole and not stack.fast_d and h.shape == x.shape == V.shape[1:] and h.device == x.device == V.device:
+        _run("write_rows", h, x, out, r, stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype), _stream(V.device))
+        stack.r_done[s] = False           # the update has no scores (the reads form them online)
+    else:
+        torch.sub(h, x, out=out)
+        _run("rstd_fwd", out, r, stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype), _stream(V.device))
+        stack.r_done[s] = False
+    return out, r
 
 
 class _WriteDelta(torch.autograd.Function):
@@ -645,30 +682,7 @@ class _WriteDelta(torch.autograd.Function):
     @staticmethod
     def forward(ctx, stack: DattnStack, s: int, h: torch.Tensor, x: torch.Tensor):
         ctx.stack, ctx.s = stack, s
-        stack.wh[s] = weakref.ref(h)
-        out = _alias(stack.V, s)
-        r = _alias(stack.R, s)
-        V = stack.V
-        whole = (h.is_cuda and x.is_cuda and h.is_contiguous() and x.is_contiguous() and h.dtype == V.dtype == x.dtype
-                 and h.numel() == x.numel() == stack.n_tok * stack.d and h.shape[-1] == stack.d)
-        if whole and stack.fast_d and _aligned(h) and _aligned(x):
-            nq, j_lo, dptr, jstride = 0, 0, None, stack.n_steps * stack.n_tok
-            if stack.DOTS is not None:
-                nq = stack.Q.shape[0]
-                j_lo = min(max(0, s - 1), nq)         # read s' >= s uses query s' - 1: queries j_lo .. nq - 1
-                if j_lo < nq:
-                    dptr = stack.DOTS[j_lo, s]
-            _run("write_dots", _p(h), _p(x), _p(out), _p(r), _p(stack.Q), _p(stack.QB), nq, j_lo, _p(dptr),
-                 stack.n_tok, stack.d, jstride, stack.eps, _dtype_code(V.dtype), _stream(V.device))
-            stack.r_done[s] = True
-        elif whole and not stack.fast_d and h.shape == x.shape == V.shape[1:] and h.device == x.device == V.device:
-            _run("write_rows", _p(h), _p(x), _p(out), _p(r), stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype),
-                 _stream(V.device))
-            stack.r_done[s] = False           # the update has no scores (the reads form them online)
-        else:
-            torch.sub(h, x, out=out)
-            _run("rstd_fwd", _p(out), _p(r), stack.n_tok, stack.d, stack.eps, _dtype_code(V.dtype), _stream(V.device))
-            stack.r_done[s] = False           # the update has no scores (the reads form them online)
+        out, r = _write(stack, s, h, x)
         ctx.set_materialize_grads(False)
         return out, r
 
@@ -708,8 +722,7 @@ class _RstdStk(torch.autograd.Function):
             xc = x.contiguous()
             if xc.numel() != stack.n_tok * stack.d or xc.dtype != stack.V.dtype:
                 raise RuntimeError("delta_attnres stacked read: the scale's input must be the stack's update")
-            _run("rstd_fwd", _p(xc), _p(r), stack.n_tok, stack.d, float(eps), _dtype_code(xc.dtype),
-                 _stream(xc.device))
+            _run("rstd_fwd", xc, r, stack.n_tok, stack.d, float(eps), _dtype_code(xc.dtype), _stream(xc.device))
         ctx.stack, ctx.s, ctx.x = stack, s, x
         return r
 
@@ -750,14 +763,13 @@ class FusedDattnReadStk(torch.autograd.Function):
         cbar_c = _f32(cbar)
         if cbar_c.numel() != n_tok * n or c0c.numel() != n:
             raise RuntimeError("delta_attnres stacked read: cbar must be (b, t, n) and c0 (n,)")
-        out = torch.empty_like(base)
-        tc = torch.empty((n_tok, n), device=dev, dtype=torch.float32)
         grad = any(ctx.needs_input_grad)
-        prob = torch.empty((n_tok, n), device=dev, dtype=torch.float32) if grad else None
         src = stack.src(n, base, qc)
         stored = stack.DOTS is not None and step >= 1 and all(stack.r_done[:n]) and step - 1 < stack.Q.shape[0]
+        out, tc, prob, _, dots = H.read_buffers(base, n_tok, n, grad, False, not stored)
         # the stored scores of query step - 1 [source, token], else formed (and kept for the backward) as it reads
-        dots = stack.DOTS[step - 1] if stored else torch.empty((n, n_tok), device=dev, dtype=torch.float32)
+        if stored:
+            dots = stack.DOTS[step - 1]
         _read(src, n, qc, dots, stored, base, None, 0.0, cbar_c, n, c0c, 1.0, out, tc, prob, None, n_tok, d, dt, st)
         if grad:
             ctx.save_for_backward(qc, cbar_c, c0c, prob, dots, tc)
@@ -778,11 +790,10 @@ class FusedDattnReadStk(torch.autograd.Function):
         d, n_tok, dev = stack.d, stack.n_tok, stack.V.device
         stack.grads()
         g = g.to(stack.V.dtype).contiguous()
-        wz = stack.WZ[_pair(step, 0):_pair(step, 0) + n]
-        dq, dcbar = _bwd1(stack.src(n, g), n, g, gt, prob, dots, tc, cbar_c, c0c, True, wz, n_tok, n_tok, d,
-                          _dtype_code(stack.V.dtype), dev)
-        # for the updates' gradients, formed once per update (the tensors, and their addresses for the kernel tables)
-        stack.bwd[step] = (g, qc, g.data_ptr(), qc.data_ptr())
+        dq, dcbar = _bwd1(stack.src(n, g), n, g, gt, prob, dots, tc, cbar_c, c0c, True, stack.wz(step), n_tok, n_tok,
+                          d, _dtype_code(stack.V.dtype), dev)
+        # for the updates' gradients, formed once per update
+        stack.keep(step, g, qc)
         final = [i == step or (step == 1 and i == 0) for i in range(n)]   # the last read of scale i, in backward order
         gbase = g
         if ctx.linked and ctx.needs_input_grad[3]:
@@ -799,6 +810,44 @@ class FusedDattnReadStk(torch.autograd.Function):
 # ---------------------------------------------------------------------------------------------------------------
 # extension (no counterpart in the reference module): the caller's glue fused into the stacked read
 # ---------------------------------------------------------------------------------------------------------------
+def _combine(stack: DattnStack, step: int, query, proposal, h0, coeffs, prior, beta: float, at_boundary: bool, n: int,
+             grad: bool):
+    """FusedCombineStk's forward: (out, tc, next prior, lam, and what its backward keeps)."""
+    d, n_tok = stack.d, stack.n_tok
+    if (proposal.dtype != stack.V.dtype or not proposal.is_contiguous() or proposal.shape[:-1] != stack.V.shape[1:3]
+            or proposal.shape[-1] != d):
+        raise RuntimeError("delta_attnres fused combine: proposal must be contiguous, the stack's dtype and shape")
+    if at_boundary and (h0 is None or h0.dtype != proposal.dtype or h0.shape != proposal.shape
+                        or not h0.is_contiguous()):
+        raise RuntimeError("delta_attnres fused combine: h0 must match the proposal at an iteration end")
+    if not 2 <= n <= stack.n_steps or n != step + 1:
+        raise RuntimeError(f"delta_attnres fused combine: {n} sources at step {step} of a stack of {stack.n_steps}")
+    if query.dim() != 2 or query.shape[-1] != d or not 1 <= step <= query.shape[0]:
+        raise RuntimeError(f"delta_attnres fused combine: query must be (n_steps - 1, {d}) with a row for step {step}")
+    lam = 1.0 - float(beta) if at_boundary else 1.0
+    qc = _f32(query[step - 1])
+    coeffs_c = _f32(coeffs)
+    prior_c = _f32(prior)
+    if coeffs_c.numel() != n_tok * (n - 1) or prior_c.numel() != n - 1:
+        raise RuntimeError("delta_attnres fused combine: coeffs must be (b, t, n-1) and prior (n-1,)")
+    h0b = h0 if at_boundary else None
+    src = stack.src(n, proposal, h0b, qc)
+    stored = stack.DOTS is not None and all(stack.r_done[:n]) and step - 1 < stack.Q.shape[0]
+    out, tc, prob, next_prior, dots = H.read_buffers(proposal, n_tok, n, grad, True, not stored)
+    if stored:
+        dots = stack.DOTS[step - 1]
+    _read(src, n, qc, dots, stored, proposal, h0b, beta, coeffs_c, n - 1, prior_c, lam, out, tc, prob, next_prior,
+          n_tok, d, _dtype_code(stack.V.dtype), _stream(stack.V.device))
+    return out, tc.view(*proposal.shape[:-1], n), next_prior, lam, (qc, coeffs_c, prior_c, prob, dots, tc)
+
+
+def combine(stack: DattnStack, step: int, query, proposal, h0, coeffs, prior, beta: float, at_boundary: bool, *scales):
+    """FusedCombineStk.apply, or its forward alone when there is nothing to record."""
+    if _bypass():
+        return _combine(stack, step, query, proposal, h0, coeffs, prior, beta, at_boundary, len(scales), False)[:3]
+    return FusedCombineStk.apply(stack, step, query, proposal, h0, coeffs, prior, beta, at_boundary, *scales)
+
+
 class FusedCombineStk(torch.autograd.Function):
     """One read of `LoopDeltaAttnRes.combine` (modeling_looped_transformer.py:148-169) for step >= 1 on the stacked
     layout, with the caller's glue inside the kernels: the iteration-end blend base = proposal + beta (h0 - proposal)
@@ -819,38 +868,11 @@ class FusedCombineStk(torch.autograd.Function):
     def forward(ctx, stack: DattnStack, step: int, query, proposal, h0, coeffs, prior, beta: float, at_boundary: bool,
                 *scales):
         n = len(scales)
-        d, n_tok, dev = stack.d, stack.n_tok, stack.V.device
-        if (proposal.dtype != stack.V.dtype or not proposal.is_contiguous() or proposal.shape[:-1] != stack.V.shape[1:3]
-                or proposal.shape[-1] != d):
-            raise RuntimeError("delta_attnres fused combine: proposal must be contiguous, the stack's dtype and shape")
-        if at_boundary and (h0 is None or h0.dtype != proposal.dtype or h0.shape != proposal.shape
-                            or not h0.is_contiguous()):
-            raise RuntimeError("delta_attnres fused combine: h0 must match the proposal at an iteration end")
-        if not 2 <= n <= stack.n_steps or n != step + 1:
-            raise RuntimeError(f"delta_attnres fused combine: {n} sources at step {step} of a stack of {stack.n_steps}")
-        if query.dim() != 2 or query.shape[-1] != d or not 1 <= step <= query.shape[0]:
-            raise RuntimeError(f"delta_attnres fused combine: query must be (n_steps - 1, {d}) with a row for step {step}")
-        dt = _dtype_code(stack.V.dtype)
-        st = _stream(dev)
-        lam = 1.0 - float(beta) if at_boundary else 1.0
-        qc = _f32(query[step - 1])
-        coeffs_c = _f32(coeffs)
-        prior_c = _f32(prior)
-        if coeffs_c.numel() != n_tok * (n - 1) or prior_c.numel() != n - 1:
-            raise RuntimeError("delta_attnres fused combine: coeffs must be (b, t, n-1) and prior (n-1,)")
-        out = torch.empty_like(proposal)
-        tc = torch.empty((n_tok, n), device=dev, dtype=torch.float32)
         grad = any(ctx.needs_input_grad)      # else no backward: the probabilities are not stored
-        prob = torch.empty((n_tok, n), device=dev, dtype=torch.float32) if grad else None
-        next_prior = torch.empty(n, device=dev, dtype=torch.float32)
-        h0b = h0 if at_boundary else None
-        src = stack.src(n, proposal, h0b, qc)
-        stored = stack.DOTS is not None and all(stack.r_done[:n]) and step - 1 < stack.Q.shape[0]
-        dots = stack.DOTS[step - 1] if stored else torch.empty((n, n_tok), device=dev, dtype=torch.float32)
-        _read(src, n, qc, dots, stored, proposal, h0b, beta, coeffs_c, n - 1, prior_c, lam, out, tc, prob, next_prior,
-              n_tok, d, dt, st)
+        out, tc, next_prior, lam, kept = _combine(stack, step, query, proposal, h0, coeffs, prior, beta, at_boundary, n,
+                                                  grad)
         if grad:
-            ctx.save_for_backward(qc, coeffs_c, prior_c, prob, dots, tc)
+            ctx.save_for_backward(*kept)
         ctx.stack, ctx.step, ctx.n, ctx.shape = stack, int(step), n, proposal.shape
         ctx.q_shape, ctx.q_dtype = query.shape, query.dtype
         ctx.beta, ctx.at_boundary, ctx.lam = float(beta), bool(at_boundary), lam
@@ -869,7 +891,7 @@ class FusedCombineStk(torch.autograd.Function):
             ctx.h0_sum = True
         ctx.mark_non_differentiable(next_prior)
         ctx.set_materialize_grads(False)
-        return out, tc.view(*proposal.shape[:-1], n), next_prior
+        return out, tc, next_prior
 
     @staticmethod
     def backward(ctx, g: torch.Tensor | None, gt: torch.Tensor | None, gnp):
@@ -888,12 +910,12 @@ class FusedCombineStk(torch.autograd.Function):
         need_prop, need_h0 = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
         g_prop = torch.empty_like(g) if ctx.at_boundary and not ctx.linked and need_prop else None
         g_h0 = torch.empty_like(g) if ctx.at_boundary and not ctx.h0_sum and need_h0 else None
-        wz = stack.WZ[_pair(step, 0):_pair(step, 0) + n]
-        _, dcoeffs = _bwd1(stack.src(n, g), n, g, gt, prob, dots, tc, coeffs_c, prior_c, True, wz, n_tok, n_tok, d,
-                           _dtype_code(stack.V.dtype), dev, cols=n - 1, lam=ctx.lam, g_prop=g_prop, g_h0=g_h0,
-                           beta=ctx.beta, part=stack.dq_parts[:, step - 1, :])
+        part = (stack.dq_parts.data_ptr() + (step - 1) * d * 4, parts, nq * d)   # dq_parts[:, step - 1, :]
+        _, dcoeffs = _bwd1(stack.src(n, g), n, g, gt, prob, dots, tc, coeffs_c, prior_c, True, stack.wz(step), n_tok,
+                           n_tok, d, _dtype_code(stack.V.dtype), dev, cols=n - 1, lam=ctx.lam, g_prop=g_prop,
+                           g_h0=g_h0, beta=ctx.beta, part=part)
         stack.dq_rows.add(step - 1)
-        stack.bwd[step] = (g, qc, g.data_ptr(), qc.data_ptr())
+        stack.keep(step, g, qc)
         final = [i == step or (step == 1 and i == 0) for i in range(n)]
         dquery = None
         if step == 1:   # read 1's backward is the pass's last: every read's partials, summed in one launch
@@ -901,7 +923,7 @@ class FusedCombineStk(torch.autograd.Function):
                 stack.dq_parts[:, j, :].zero_()
             dq = torch.empty((nq, d), device=dev, dtype=torch.float32)
             if n_tok > 0:
-                _run("reduce_rows", _p(stack.dq_parts), parts, nq * d, _p(dq), _stream(dev))
+                _run("reduce_rows", stack.dq_parts, parts, nq * d, dq, _stream(dev))
             else:
                 dq.zero_()
             dquery = dq.to(ctx.q_dtype)
@@ -917,13 +939,13 @@ class FusedCombineStk(torch.autograd.Function):
                 # rounding per read: from the last iteration end to the first, as autograd adds the blends' shares
                 gs = [stack.h0_g[k] for k in sorted(stack.h0_g, reverse=stack.per_read)]
                 dh0 = torch.empty_like(g)
-                tail = (len(gs), ctx.beta, int(stack.per_read), _p(dh0), n_tok, d, _dtype_code(stack.V.dtype),
+                tail = (len(gs), ctx.beta, int(stack.per_read), dh0, n_tok, d, _dtype_code(stack.V.dtype),
                         _stream(dev))
                 if stack.fast_d and _fast(d, len(gs), dh0, *gs):
-                    _run("blend_sum", L.u64_array(x.data_ptr() for x in gs), *tail)
+                    _run("blend_sum", gs, *tail)
                 elif _rows(d, len(gs)):
                     _refuse_capture()
-                    _run("blend_sum_rows", L.u64_array(x.data_ptr() for x in gs), *tail)
+                    _run("blend_sum_rows", gs, *tail)
                 else:
                     gt_ = _dev_addrs((x.data_ptr() for x in gs), dev)
                     _run("blend_sum_any", gt_.data_ptr(), *tail)

@@ -215,3 +215,33 @@ def test_unaligned_row_argument_checks_before_launch(lib):
     parts = lib.bwd1_rows_parts
     assert parts(0, 2048) == 0 and parts(16, 8193) == 0 and parts(16, 7) == 0
     assert [parts(t, 2048) for t in (1, 65, 1024, 2048, 4096, 16384)] == [1, 17, 256, 256, 512, 512]
+
+
+def test_host_launch_path(lib):
+    """The launch path's builtins cover every entry point that launches, convert arguments as the C ABI takes them (the
+    library's own refusals come back), refuse the rest with a Python error, and alias() is a tensor of its own."""
+    import torch
+    from loopback_amd import _host as H
+    from loopback_amd import fused_dattn as FD
+    assert set(FD._FN) == {n[4:] for n in lib.SIGNATURES if n not in (
+        "ldr_abi_version", "ldr_strerror", "ldr_row_layout", "ldr_read_bwd1_parts", "ldr_query_parts_elems",
+        "ldr_read_bwd1_rows_parts")}
+    assert not H.bind("ldr_abi_version", 1)
+    x = torch.empty(8)
+    assert H.rstd_fwd(None, None, 16, 64, 1e-6, 1, None) == -1 and H.rstd_fwd(x, x, 16, 0, 1e-6, 1, 0) == -1
+    assert H.blend_sum([4096, 4100], 2, 0.5, 0, 4096, 16, 64, 1, None) == -3
+    assert H.blend_sum(lib.u64_array([4096, 4100]), 2, 0.5, 0, 4096, 16, 64, 1, None) == -3
+    for bad in (lambda: H.rstd_fwd(x), lambda: H.rstd_fwd("x", x, 16, 64, 1e-6, 1, None),
+                lambda: H.rstd_fwd(x, x, 1.5, 64, 1e-6, 1, None), lambda: H.alias(x), lambda: H.alias(1, 0)):
+        with pytest.raises(TypeError):
+            bad()
+    with pytest.raises(ValueError):
+        H.blend_sum([4096] * 65, 65, 0.5, 0, 4096, 16, 64, 1, None)
+    t = torch.arange(24.0).view(3, 4, 2)
+    a = FD._alias(t, -1)
+    assert torch.equal(a, t[2]) and a._base is None and a.data_ptr() == t[2].data_ptr()
+    v = a._version
+    t.zero_()
+    assert a._version == v and not a.any()
+    with pytest.raises(IndexError):
+        FD._alias(t, 3)
