@@ -353,9 +353,13 @@ __global__ __launch_bounds__(WG) void k_next_token_bwd(const T* __restrict__ log
 // Per 64 x 32 tile a wave issues 512 matrix-core cycles forward (512 per product pair backward) and ~1000 vector cycles
 // (per score an exponential, 16 cycles, and 4-7 operations of 4): the vector units bound it, so two or three waves
 // share a SIMD and the maximum is moved, and the sums rescaled, only when it grows by more than 2^8.
-// 8 x 2048 tokens, 12 heads: the rotation 17-19 us, forward 113-125 us (455 TFLOP/s of the causal half), dq 138-153,
-// dk and dv 224-247; the flash attention of torch took 172, 288 and 480-500 us, and the rotation, its gradient and the
-// copies between layouts another ~700 in some twenty elementwise launches.
+// 8 x 2048 tokens, 12 heads: the rotation 16 us, forward 75-80 us (640-690 TFLOP/s of the causal half), both backward
+// kernels 273-280; the flash attention of torch took 172 and 780 us, and the rotation, its gradient and the copies
+// between layouts another ~700 in some twenty elementwise launches. What took these kernels there from 113 and 362 us:
+// the masks under a wave-uniform branch and before the exponential (they had been a branch per score in the dk, dv
+// kernel), two waves per SIMD asked for (the accumulators then stay in vector registers, 128 moves less per tile),
+// addresses moved on instead of formed per tile, and the order of the work (attn_work). Three waves per SIMD in the
+// dk, dv kernel spill 116 bytes and cost a third; one row half at a time in the backward kernels is level.
 // ---------------------------------------------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -402,17 +406,35 @@ __device__ __forceinline__ float other_half(float x, bool sum) {   // x joined w
   return sum ? a + b : fmaxf(a, b);
 }
 
-// 64 rows of 64 elements, row stride `stride` elements, rows past the last repeated: 512 16-byte pieces, two per lane
+// 64 rows of 64 elements, row stride `stride` elements: 512 16-byte pieces, two per lane. The cursor's addresses move on
+// by a tile per load; rows past the last repeat it.
 struct TileRegs { uint4 u[2]; };
-__device__ __forceinline__ TileRegs tile_load(const bf16_t* base, int64_t stride, int row0, int t) {
-  TileRegs r;
+struct Cursor {
+  const bf16_t* p[2];
+  int64_t stride;
+  int row0, t;
+  __device__ __forceinline__ Cursor(const bf16_t* base, int64_t stride_, int row0_, int t_)
+      : stride(stride_), row0(row0_), t(t_) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = (int)threadIdx.x + 256 * i;
-    r.u[i] = *reinterpret_cast<const uint4*>(base + (int64_t)min(row0 + (c >> 3), t - 1) * stride + 8 * (c & 7));
+    for (int i = 0; i < 2; ++i) p[i] = base + (int64_t)(row0 + row(i)) * stride + 8 * ((int)threadIdx.x & 7);
   }
-  return r;
-}
+  static __device__ __forceinline__ int row(int i) { return ((int)threadIdx.x >> 3) + 32 * i; }
+  __device__ __forceinline__ TileRegs next() {
+    TileRegs r;
+    if (row0 + AT_N <= t) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) r.u[i] = *reinterpret_cast<const uint4*>(p[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        r.u[i] = *reinterpret_cast<const uint4*>(p[i] - (int64_t)max(row0 + row(i) - (t - 1), 0) * stride);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) p[i] += AT_N * stride;
+    row0 += AT_N;
+    return r;
+  }
+};
 __device__ __forceinline__ void tile_store(bf16_t* tile, const TileRegs& r) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -422,12 +444,14 @@ __device__ __forceinline__ void tile_store(bf16_t* tile, const TileRegs& r) {
 }
 
 // Which (batch, head) and block of rows a workgroup takes: the blocks of one head on one XCD (workgroups go to XCDs in
-// turn), so its rows are read from that XCD's L2; false past the last head.
+// turn), so its rows are read from that XCD's L2, and in each XCD the most work of every head first: a head's blocks in
+// one run instead put three long ones on one CU and three short ones on another (2 x 4096 tokens, 12 heads: forward 118
+// -> 82 us, backward 304 -> 244; 8 x 2048: 103 -> 76 and 307 -> 273). False past the last head.
 struct AttnWork { int bh, block; };
 __device__ __forceinline__ bool attn_work(int bhs, int blocks, AttnWork& w) {
-  const int i = (int)blockIdx.x >> 3;
-  w.bh = ((int)blockIdx.x & 7) + 8 * (i / blocks);
-  w.block = i % blocks;
+  const int i = (int)blockIdx.x >> 3, heads = (bhs + 7) >> 3;   // heads of an XCD
+  w.bh = ((int)blockIdx.x & 7) + 8 * (i % heads);
+  w.block = i / heads;
   return w.bh < bhs;
 }
 
@@ -460,11 +484,12 @@ __global__ __launch_bounds__(WG) void k_rotary(const bf16_t* __restrict__ qkv, c
 
 // out [b, t, heads, 64] and lse2 [b heads, t] (the base-2 logarithm of each query's sum of exponentials of c times its
 // scores, c = log2(e) / 8). A workgroup takes 128 queries, the last blocks (the most keys) first.
-__global__ __launch_bounds__(256) void k_attn_fwd(const bf16_t* __restrict__ qk, const bf16_t* __restrict__ qkv,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_fwd(const bf16_t* __restrict__ qk, const bf16_t* __restrict__ qkv,
                                                   bf16_t* __restrict__ out, float* __restrict__ lse2, int bhs, int t,
                                                   int heads, float c) {
   __shared__ __align__(16) bf16_t s_k[2][AT_N * AT_LD], s_v[2][AT_N * AT_LD];
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int lane = (int)threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int blocks = (t + AT_M - 1) / AT_M;
   AttnWork wk;
   if (!attn_work(bhs, blocks, wk)) return;
@@ -481,15 +506,16 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16_t* __restrict__ qk,
   f32x16 o[2] = {zero16(), zero16()};
   float m = -INFINITY, l = 0.f;
   const int ntiles = (min(q0 + AT_M, t) + AT_N - 1) / AT_N;
-  TileRegs kr = tile_load(kp, sqk, 0, t), vr = tile_load(vp, sv, 0, t);
+  Cursor kc(kp, sqk, 0, t), vc(vp, sv, 0, t);
+  TileRegs kr = kc.next(), vr = vc.next();
   tile_store(s_k[0], kr);
   tile_store(s_v[0], vr);
   __syncthreads();
   for (int j = 0; j < ntiles; ++j) {
     const int k0 = j * AT_N, cur = j & 1;
     if (j + 1 < ntiles) {
-      kr = tile_load(kp, sqk, k0 + AT_N, t);
-      vr = tile_load(vp, sv, k0 + AT_N, t);
+      kr = kc.next();
+      vr = vc.next();
     }
     if (k0 <= w0 + 31 && w0 < t) {   // this wave has queries past the tile's first key
       f32x16 s[2];
@@ -521,12 +547,13 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16_t* __restrict__ qk,
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[i][r] *= a;
       }
+      float ls[4] = {0.f, 0.f, 0.f, 0.f};   // four sums: no chain of 32 dependent adds
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           s[i][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][r], c, -m));
-          l += s[i][r];
+          ls[r & 3] += s[i][r];
         }
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
@@ -535,6 +562,7 @@ __global__ __launch_bounds__(256) void k_attn_fwd(const bf16_t* __restrict__ qk,
           for (int d = 0; d < 2; ++d) o[d] = mfma(cols_frag(s_v[cur], 32 * i + 16 * st, 32 * d, lane), p, o[d]);
         }
       }
+      l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
     }
     if (j + 1 < ntiles) {
       tile_store(s_k[cur ^ 1], kr);
@@ -586,7 +614,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const float* __restrict__ sinT, float* __restrict__ delta, bf16_t* __restrict__ dqkv, int bhs, int t, int heads,
     float c, float scale) {
   __shared__ __align__(16) bf16_t s_k[2][AT_N * AT_LD], s_v[2][AT_N * AT_LD];
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int lane = (int)threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int blocks = (t + AT_M - 1) / AT_M;
   AttnWork wk;
   if (!attn_work(bhs, blocks, wk)) return;
@@ -615,15 +644,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (query < t && half == 0) delta[(int64_t)wk.bh * t + query] = dl;
   f32x16 dq[2] = {zero16(), zero16()};
   const int ntiles = (min(q0 + AT_M, t) + AT_N - 1) / AT_N;
-  TileRegs kr = tile_load(kp, sqk, 0, t), vr = tile_load(vp, sv, 0, t);
+  Cursor kc(kp, sqk, 0, t), vc(vp, sv, 0, t);
+  TileRegs kr = kc.next(), vr = vc.next();
   tile_store(s_k[0], kr);
   tile_store(s_v[0], vr);
   __syncthreads();
   for (int j = 0; j < ntiles; ++j) {
     const int k0 = j * AT_N, cur = j & 1;
     if (j + 1 < ntiles) {
-      kr = tile_load(kp, sqk, k0 + AT_N, t);
-      vr = tile_load(vp, sv, k0 + AT_N, t);
+      kr = kc.next();
+      vr = vc.next();
     }
     if (k0 <= w0 + 31 && w0 < t) {
       const bool edge = k0 + AT_N - 1 > w0;
@@ -635,12 +665,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
           s = mfma(rows_frag(s_k[cur], 32 * i, ks, lane), qf[ks], s);
           dp = mfma(rows_frag(s_v[cur], 32 * i, ks, lane), gf[ks], dp);
         }
+        if (edge) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ls));
-          s[r] = p * (dp[r] - dl);
-          if (edge && k0 + 32 * i + 4 * half + (r & 3) + 8 * (r >> 2) > query) s[r] = 0.f;
+          for (int r = 0; r < 16; ++r)
+            if (k0 + 32 * i + 4 * half + (r & 3) + 8 * (r >> 2) > query) s[r] = -INFINITY;
         }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ls)) * (dp[r] - dl);
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
           const bf16x8 ds = operand(s, st);
@@ -667,7 +698,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const float* __restrict__ sinT, bf16_t* __restrict__ dqkv, int bhs, int t, int heads, float c, float scale) {
   __shared__ __align__(16) bf16_t s_q[2][AT_N * AT_LD], s_g[2][AT_N * AT_LD];
   __shared__ __align__(16) float s_ls[2][AT_N], s_dl[2][AT_N];
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, half = lane >> 5;
+  const int lane = (int)threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int blocks = (t + AT_M - 1) / AT_M;
   AttnWork wk;
   if (!attn_work(bhs, blocks, wk)) return;
@@ -696,15 +728,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     if (tid < AT_N) s_ls[buf][tid] = sc;
     else if (tid < 2 * AT_N) s_dl[buf][tid - AT_N] = sc;
   };
-  TileRegs qr = tile_load(qp, sqk, first * AT_N, t), gr = tile_load(gp, so, first * AT_N, t);
+  Cursor qc(qp, sqk, first * AT_N, t), gc(gp, so, first * AT_N, t);
+  TileRegs qr = qc.next(), gr = gc.next();
   float sc = load_scalar(first * AT_N);
   put(first & 1, qr, gr, sc);
   __syncthreads();
   for (int j = first; j < ntiles; ++j) {
     const int q0 = j * AT_N, cur = j & 1;
     if (j + 1 < ntiles) {
-      qr = tile_load(qp, sqk, q0 + AT_N, t);
-      gr = tile_load(gp, so, q0 + AT_N, t);
+      qr = qc.next();
+      gr = gc.next();
       sc = load_scalar(q0 + AT_N);
     }
     if (q0 + AT_N - 1 >= w0 && w0 < t) {   // the tile has queries at or past this wave's first key
@@ -717,6 +750,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
           s = mfma(rows_frag(s_q[cur], 32 * i, ks, lane), kf[ks], s);
           dp = mfma(rows_frag(s_g[cur], 32 * i, ks, lane), vf[ks], dp);
         }
+        if (edge) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int query = q0 + 32 * i + 4 * half + (r & 3) + 8 * (r >> 2);
+            if (key > query || query >= t) s[r] = -INFINITY;
+          }
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int r0 = 32 * i + 8 * g + 4 * half;
@@ -726,10 +766,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             const int r = 4 * g + k;
-            const bool off = edge && (key > q0 + r0 + k || q0 + r0 + k >= t);
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ll[k]));
-            s[r] = off ? 0.f : p;
-            dp[r] = off ? 0.f : p * (dp[r] - dd[k]);
+            s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -ll[k]));
+            dp[r] = s[r] * (dp[r] - dd[k]);
           }
         }
 #pragma unroll
