@@ -73,6 +73,11 @@ int llm_attn_bwd(const void* qk, const void* qkv, const void* out, const void* d
                  const float* cosT, const float* sinT, float* delta, void* dqkv, int64_t b, int64_t t, int64_t heads,
                  void* stream);
 
+/* dw [n, k] = round(sum over m tokens of dy [m, n] x [m, k]), the weight gradient of a bias-free linear layer in bf16 (fp32
+ * sums; n and k multiples of 8, 16-byte aligned). part: scratch, llm_wgrad_splits(m, n, k) x n x k floats. */
+int64_t llm_wgrad_splits(int64_t m, int64_t n, int64_t k);
+int llm_wgrad(const void* dy, const void* x, float* part, void* dw, int64_t m, int64_t n, int64_t k, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

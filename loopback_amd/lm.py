@@ -129,12 +129,19 @@ def _hooked(m: nn.Module) -> bool:
                 or g._global_backward_pre_hooks)
 
 
+class Linear(nn.Linear):
+    """nn.Linear without a bias, its weight's gradient on the HIP kernel where that is faster (lm_ops.linear)."""
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return ops.linear(x, self.weight) if self.bias is None else super().forward(x)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
         self.h, self.dh = cfg.num_heads, cfg.hidden_size // cfg.num_heads
-        self.qkv = nn.Linear(cfg.hidden_size, 3 * cfg.hidden_size, bias=False)
-        self.o = nn.Linear(cfg.hidden_size, cfg.hidden_size, bias=False)
+        self.qkv = Linear(cfg.hidden_size, 3 * cfg.hidden_size, bias=False)
+        self.o = Linear(cfg.hidden_size, cfg.hidden_size, bias=False)
         self.rotary = Rotary(self.dh, cfg.rope_theta)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -161,8 +168,8 @@ class Attention(nn.Module):
 class SwiGLU(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
-        self.gate_up = nn.Linear(cfg.hidden_size, 2 * cfg.intermediate, bias=False)
-        self.down = nn.Linear(cfg.intermediate, cfg.hidden_size, bias=False)
+        self.gate_up = Linear(cfg.hidden_size, 2 * cfg.intermediate, bias=False)
+        self.down = Linear(cfg.intermediate, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.down(ops.swiglu(self.gate_up(x)))

@@ -1,6 +1,6 @@
 """The language model's row operations on the HIP kernels of libloopback_lm.so (include/loopback_lm.h): RMSNorm with the
 residual's add before it and the residual's gradient folded into its backward, SwiGLU, the next-token cross entropy on
-16-bit logits, and causal rotary attention in bf16 at head width 64.
+16-bit logits, causal rotary attention in bf16 at head width 64, and the weight gradients of the linear layers.
 
 `native(...)` says whether the kernels take a call: plain 16-bit GPU tensors of one dtype on one device, no transform
 or tracer that has to see torch operations (torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else --
@@ -36,6 +36,8 @@ SIGNATURES = {
     "llm_next_token_loss_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
     "llm_rotary": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "llm_attn_fwd": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
+    "llm_wgrad_splits": (_i64, [_i64, _i64, _i64]),
+    "llm_wgrad": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "llm_attn_bwd": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
 }
 
@@ -284,3 +286,47 @@ def attention_native(qkv: torch.Tensor, head_dim: int) -> bool:
 def rotary_attention(qkv, cos, sin, heads, again):
     """Causal attention over the rotated q and k of qkv; cos and sin (t, 64) fp32, contiguous, both halves alike."""
     return _RotaryAttention.apply(qkv, cos, sin, heads, again)
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# bias-free linear layers, their weight gradient by llm_wgrad
+# ---------------------------------------------------------------------------------------------------------------
+# Where the split reduction is the faster one (16384 tokens, weights 256 x 256 to 4096 x 768: 1.2 to 3.2 times the library;
+# 8192 tokens: 1.2; 4096 tokens and fewer: 0.6 to 1.1, the library's), and enough runs of tokens fill the GPU (with two
+# runs, 5632 x 1024: 0.84).
+WGRAD_MIN_TOKENS, WGRAD_MIN_SPLITS = 8192, 4
+
+
+def wgrad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """dy^T x of (tokens, n) and (tokens, k) rows, bf16."""
+    (m, n), k = dy.shape, x.shape[1]
+    part = torch.empty((LIB.llm_wgrad_splits(m, n, k), n, k), device=x.device, dtype=torch.float32)
+    dw = torch.empty((n, k), device=x.device, dtype=x.dtype)
+    _run("llm_wgrad", dy.data_ptr(), x.data_ptr(), part.data_ptr(), dw.data_ptr(), m, n, k, _stream(x))
+    return dw
+
+
+class _Linear(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return F.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return tuple(_again(F.linear, [x, w], ctx.needs_input_grad, (dy,)))
+        dy = _dense(dy, x).view(-1, w.shape[0])
+        dx = (dy @ w).view(x.shape) if ctx.needs_input_grad[0] else None
+        return dx, wgrad(dy, x.view(-1, w.shape[1])) if ctx.needs_input_grad[1] else None
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w), with the weight's gradient by llm_wgrad where that is the faster one."""
+    if (torch.is_grad_enabled() and w.requires_grad and x.dtype is torch.bfloat16 and x.dim() > 1 and w.dim() == 2
+            and x.shape[-1] == w.shape[1] and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1] and w.shape[0] % 8 == 0
+            and w.shape[1] % 8 == 0 and native(x, w) and _rows_ok(x, w)
+            and LIB.llm_wgrad_splits(x.numel() // w.shape[1], *w.shape) >= WGRAD_MIN_SPLITS):
+        return _Linear.apply(x, w)
+    return F.linear(x, w)

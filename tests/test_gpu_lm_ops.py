@@ -109,6 +109,40 @@ def test_loss_edge_rows():
     assert loss.isnan() and not one.grad.any()
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (63, 264, 40), (65, 256, 256), (700, 40, 520), (1600, 512, 264),
+                                   (8200, 776, 768)])
+def test_wgrad(m, n, k):
+    """dy^T x: one and several runs of tokens, remainders of a step, a tile and a run. Half a step of the result, and of
+    fp32 sums over m products 1e-5 of the RMS per 16384 tokens (a fraction of it here)."""
+    from loopback_amd import lm_ops as ops
+    print(f"case wgrad {m}x{n}x{k} in {ops.LIB.llm_wgrad_splits(m, n, k)} runs", flush=True)
+    dy, x = rnd((m, n), torch.bfloat16, m), rnd((m, k), torch.bfloat16, n)
+    close(ops.wgrad(dy, x), dy.double().t() @ x.double(), torch.bfloat16)
+
+
+def test_linear_module():
+    """The layer's output and input gradient are torch's bits, its weight gradient at most as far from fp64 as torch's;
+    second derivatives are torch's; few tokens stay on torch's product."""
+    from loopback_amd import lm, lm_ops as ops
+    torch.manual_seed(1)
+    lin = lm.Linear(256, 512, bias=False).to(DEV, torch.bfloat16)
+    x, g = rnd((2, 4100, 256), torch.bfloat16, 15).requires_grad_(), rnd((2, 4100, 512), torch.bfloat16, 16)
+    y = lin(x)
+    assert type(y.grad_fn).__name__ == "_LinearBackward"
+    dx, dw = torch.autograd.grad(y, (x, lin.weight), g)
+    yr = F.linear(x, lin.weight)
+    dxr, dwr = torch.autograd.grad(yr, (x, lin.weight), g)
+    exact = g.double().view(-1, 512).t() @ x.detach().double().view(-1, 256)
+    assert torch.equal(y, yr) and torch.equal(dx, dxr)
+    assert (dw.double() - exact).norm() <= 1.01 * (dwr.double() - exact).norm()
+    d1, = torch.autograd.grad(lin(x), x, g, create_graph=True)
+    second, = torch.autograd.grad(d1.float().pow(2).sum(), lin.weight)
+    d1, = torch.autograd.grad(F.linear(x, lin.weight), x, g, create_graph=True)
+    ref, = torch.autograd.grad(d1.float().pow(2).sum(), lin.weight)
+    assert (second - ref).float().norm() <= 1e-2 * ref.float().norm()
+    assert type(lin(x[:, :10]).grad_fn).__name__ != "_LinearBackward"
+
+
 def test_what_stays_torch():
     """Second derivatives are torch's; a hooked norm is called as a module; forward-mode, vmap and fp32 calls take
     torch's operations."""
