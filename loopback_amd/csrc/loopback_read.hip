@@ -474,7 +474,8 @@ __global__ __launch_bounds__(WG) void k_rstd_bwd(const T* __restrict__ x, const 
 // instruction) and backward pass 1 ran one wave on each of n_tok / 64 partial rows. A 12-step training pass of 2049
 // tokens at d = 1001 in bf16: 31.8 -> 2.06 ms (the host's launch rate; 1.04 ms of kernels), per launch backward
 // pass 1 2690 -> 22.6 us (7 sources on average), the read 70-79 -> 23-26, the update gradient 44.6 -> 24.1. A read of
-// 65-72 sources of 4096 x 768 bf16: 746 -> 138 us (3.1 TB/s; two waves per SIMD, a row's online softmax between loads).
+// 65-72 sources of 4096 x 768 bf16: 746 -> 94 us (4.7 TB/s; 138 with two vectors on each of 64 lanes, a quarter of them
+// idle, where three on 32 lanes put two rows in a wave).
 // ---------------------------------------------------------------------------------------------------------------
 // Row geometry at any width d >= 8: vector c of a row covers elements [8c, 8c + 8), the last one [d - 8, d).
 struct URows {
@@ -2841,7 +2842,7 @@ __device__ __forceinline__ void row_softmax(float* a, int n, const URows& R) {
 
 // sources of a row in flight in the read's ring: 64 bytes per lane or more, within two waves' registers
 template <typename T, int VPT> struct URing {
-  static constexpr int PD = std::is_same<T, float>::value ? (VPT == 1 ? 4 : VPT == 2 ? 2 : 1) : (VPT <= 2 ? 4 : 2);
+  static constexpr int PD = std::is_same<T, float>::value ? (VPT == 1 ? 4 : VPT <= 3 ? 2 : 1) : (VPT <= 2 ? 4 : VPT == 3 ? 3 : 2);
 };
 
 // The read (k_read_fwd without stored scores q == NULL, k_read_online with): its formulas and summation orders.
@@ -3535,14 +3536,14 @@ __global__ __launch_bounds__(WG) void k_zero(float* __restrict__ p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) p[i] = 0.f;
 }
 
-// unaligned rows: vectors per lane (1, 2 or 4) and lanes per row for width d, the fewest idle lanes first, then rows
+// unaligned rows: vectors per lane (1 to 4) and lanes per row for width d, the fewest idle lanes first, then rows
 // inside one wave, then fewer vectors per lane; with many sources fewer rows per workgroup (their per-source scalars
 // take 3 n floats of LDS each: at most 48 KiB)
 int rows_layout(int64_t d, int64_t n, int* vpt, int* tpr) {
   if (d < 8 || d > LDR_MAX_WIDTH) return LDR_E_SHAPE;
   const int64_t d8 = (d + 7) >> 3;
   int64_t best = INT64_MAX;
-  for (int v = 1; v <= 4; v <<= 1) {
+  for (int v = 1; v <= 4; ++v) {
     for (int t = 8; t <= WG; t <<= 1) {
       if ((int64_t)v * t < d8 || (WG / t) * n > 4096) continue;
       const int64_t key = ((int64_t)v * t - d8) * 16 + (t > 64 ? 8 : 0) + v;
@@ -3554,13 +3555,6 @@ int rows_layout(int64_t d, int64_t n, int* vpt, int* tpr) {
 
 inline bool rows_width(int64_t d) { return d >= 8 && d <= LDR_MAX_WIDTH; }
 
-#define LDR_VPT124_SWITCH(VPT_RT, ...)                           \
-  switch (VPT_RT) {                                              \
-    case 1: { constexpr int VPT = 1; __VA_ARGS__; } break;       \
-    case 2: { constexpr int VPT = 2; __VA_ARGS__; } break;       \
-    default: { constexpr int VPT = 4; __VA_ARGS__; } break;      \
-  }
-
 template <typename TAB>
 int rows_read(const TAB& src, int64_t n, const float* q, float* dots, int64_t dots_stride, const void* base,
               const void* h0, float beta, const Coef& cf, float inv, void* out, float* tc, float* p,
@@ -3570,7 +3564,7 @@ int rows_read(const TAB& src, int64_t n, const float* q, float* dots, int64_t do
   const size_t lds = sizeof(float) * (size_t)(3 * n * (1 + WG / tpr));
   const unsigned grid = grid_of(cdiv(n_tok, WG / tpr), 2048);   // no tokens: one workgroup writes next_prior
 #define LDR_ROWS_READ(BL)                                                                                            \
-  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_read<T, VPT, BL, TAB>), dim3(grid),        \
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rows_read<T, VPT, BL, TAB>), dim3(grid),        \
       dim3(WG), lds, st, src, (int)n, q, dots, dots_stride, static_cast<const T*>(base), static_cast<const T*>(h0),    \
       beta, cf, inv, static_cast<T*>(out), tc, p, next_prior, n_tok, (int)d, tpr)))
   if (h0) {
@@ -3591,7 +3585,7 @@ int rows_bwd1(const TAB& src, int64_t n, const void* g, const float* gt, const f
   if (e) return e;
   const int64_t planes = 3 * n * (WG / tpr);
   const size_t lds = sizeof(float) * (size_t)(planes > d ? planes : d);
-  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd1<T, VPT, TAB>),
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd1<T, VPT, TAB>),
       dim3((unsigned)dq_parts), dim3(WG), lds, st, src, (int)n, static_cast<const T*>(g), gt, p, dots, dots_stride, tc,
       cf, inv, dcbar, (int)dcbar_cols, dr_accum, wz, wz_stride, dq_part, dq_part_stride, static_cast<T*>(g_prop),
       static_cast<T*>(g_h0), beta, n_tok, (int)d, tpr)))
@@ -3607,7 +3601,7 @@ int rows_dv_assemble(const TAB& tab, int64_t m, const void* v, const float* r, c
   const int rb = dtype == LDR_F32 ? rows_rb<float>(vpt) : rows_rb<bf16_t>(vpt);
   const unsigned grid = grid_of(cdiv(n_tok, (WG / tpr) * rb), 65535);
 #define LDR_ROWS_AS(PR)                                                                                              \
-  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_dv_assemble<T, VPT, PR, TAB>), dim3(grid), \
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rows_dv_assemble<T, VPT, PR, TAB>), dim3(grid), \
       dim3(WG), 0, st, tab, (int)m, static_cast<const T*>(v), r, gr, static_cast<const T*>(add), add_beta,             \
       static_cast<T*>(dv), static_cast<T*>(dv_neg), n_tok, (int)d, tpr)))
   if (per_read) {
@@ -3625,7 +3619,7 @@ int rows_bwd2_list(const TAB& dv, int64_t n, int accum, const void* g, const flo
   int vpt, tpr, e = rows_layout(d, 1, &vpt, &tpr);
   if (e) return e;
   const unsigned grid = grid_of(cdiv(n_tok, WG / tpr), 8192);
-  LDR_DTYPE_SWITCH(dtype, LDR_VPT124_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd2_list<T, VPT, TAB>), dim3(grid),
+  LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rows_bwd2_list<T, VPT, TAB>), dim3(grid),
       dim3(WG), 0, st, dv, (int)n, accum, static_cast<const T*>(g), q, wz, wz_stride, n_tok, (int)d, tpr)))
   return launched();
 }
