@@ -188,8 +188,12 @@ def reference_bytes(cfg, mode):
 
 
 def source_sha256() -> str:
-    with open(os.path.join(ROOT, "loopback_amd", "csrc", "loopback_read.hip"), "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()
+    """Of the read's kernel sources: loopback_read.hip and the header of its memory helpers, one after the other."""
+    h = hashlib.sha256()
+    for name in ("loopback_read.hip", "device_io.h"):
+        with open(os.path.join(ROOT, "loopback_amd", "csrc", name), "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()
 
 
 @contextlib.contextmanager

@@ -245,3 +245,20 @@ def test_host_launch_path(lib):
     assert a._version == v and not a.any()
     with pytest.raises(IndexError):
         FD._alias(t, 3)
+
+
+def test_lm_library(lib):
+    """The LM library exports what include/loopback_lm.h declares, the binding's table is the header's, and calls whose
+    operands the kernels do not take are refused before any launch."""
+    from loopback_amd import lm_ops as ops
+    with open(os.path.join(ROOT, "include", "loopback_lm.h")) as f:
+        names = set(re.findall(r"\b(llm_\w+)\s*\(", re.sub(r"/\*.*?\*/", "", f.read(), flags=re.S)))
+    assert names == set(ops.SIGNATURES) and all(hasattr(ops.LIB, n) for n in names)
+    L, p, null = ops.LIB, 4096, None
+    wg = lambda m, n, k, a=p: L.llm_wgrad(a, p, p, p, m, n, k, null)
+    assert wg(64, 60, 64) == -2 and wg(64, 64, 7) == -2 and wg(0, 64, 64) == -1 and wg(64, 64, 64, 4098) == -3
+    assert [L.llm_wgrad_splits(*s) for s in ((511, 256, 256), (16384, 2304, 768), (8192, 5632, 1024), (16384, 64, 64))] \
+        == [1, 9, 2, 32]
+    at = lambda b, t, h, a=p: L.llm_attn_fwd(a, p, p, p, b, t, h, null)
+    assert at(1, 16, 0) == -1 and at(1, -1, 1) == -1 and at(1, 16, 1, 4098) == -3 and at(0, 16, 1) == 0
+    assert L.llm_rotary(4098, p, p, p, 1, 16, 1, null) == -3 and L.llm_rotary(null, p, p, p, 1, 16, 1, null) == -1
