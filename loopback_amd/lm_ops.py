@@ -277,10 +277,14 @@ class _RotaryAttention(torch.autograd.Function):
         return dqkv, None, None, None, None
 
 
+ATTN_MAX = 0x7fffff   # tokens a sequence, and sequences times heads, as llm_attn_fwd checks them
+
+
 def attention_native(qkv: torch.Tensor, head_dim: int) -> bool:
-    """Whether rotary_attention takes qkv (b, t, 3 heads head_dim): bf16, head width 64, not empty."""
+    """Whether rotary_attention takes qkv (b, t, 3 heads head_dim): bf16, head width 64, not empty, within the
+    kernels' index range."""
     return (head_dim == 64 and qkv.dtype is torch.bfloat16 and native(qkv) and qkv.dim() == 3 and qkv.numel() > 0
-            and _rows_ok(qkv))
+            and qkv.shape[1] <= ATTN_MAX and qkv.shape[0] * qkv.shape[2] <= 192 * ATTN_MAX and _rows_ok(qkv))
 
 
 def rotary_attention(qkv, cos, sin, heads, again):
