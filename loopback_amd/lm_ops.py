@@ -2,10 +2,11 @@
 residual's add before it and the residual's gradient folded into its backward, SwiGLU, the next-token cross entropy on
 16-bit logits, causal rotary attention in bf16 at head width 64, and the weight gradients of the linear layers.
 
-`native(...)` says whether the kernels take a call: plain 16-bit GPU tensors of one dtype on one device, no transform
-or tracer that has to see torch operations (torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else --
-the CPU, fp32, other shapes -- stays on torch in lm.py. A backward that is itself differentiated (create_graph) runs
-the torch form of the operation, so second derivatives are torch's.
+`native(...)` says whether the kernels take a call: plain 16-bit tensors of one dtype on the current GPU (a launch on
+another GPU's default stream would run on the current one), no transform or tracer that has to see torch operations
+(torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else -- the CPU, fp32, other shapes --
+stays on torch in lm.py. A backward that is itself differentiated (create_graph) runs the torch form of the operation,
+so second derivatives are torch's.
 """
 from __future__ import annotations
 
@@ -70,7 +71,7 @@ def _stream(t: torch.Tensor) -> int:
 
 def native(*tensors) -> bool:
     first = tensors[0]
-    if not first.is_cuda or first.dtype not in _CODES:
+    if not first.is_cuda or first.dtype not in _CODES or first.device.index != torch._C._cuda_getDevice():
         return False
     for t in tensors:
         if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.dtype is not first.dtype \

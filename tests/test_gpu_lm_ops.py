@@ -170,3 +170,12 @@ def test_what_stays_torch():
     assert torch.equal(y, ops._swiglu_torch(gu.detach())) and dy.shape == y.shape
     assert torch.func.vmap(ops.swiglu)(gu.detach()[None]).shape == (1, 5, 32)
     assert not ops.native(x.detach().float())
+
+
+def test_only_on_the_current_gpu(monkeypatch):
+    """Tensors of a GPU that is not the current one stay on torch: the default stream is the current GPU's."""
+    from loopback_amd import lm_ops as ops
+    x = rnd((2, 16), torch.bfloat16, 30)
+    assert ops.native(x)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.device.index + 1)
+    assert not ops.native(x)
