@@ -122,11 +122,12 @@ def attention_kernels(dtype):
 
 
 def _hooked(m: nn.Module) -> bool:
-    """Whether calling m runs more than its forward (hooks of its own, or of every module)."""
+    """Whether calling m runs more than its class's forward (hooks of its own, or of every module, or a forward set on
+    the instance, as wrappers that move or cast a module's inputs do)."""
     g = nn.modules.module
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
-                or g._global_backward_pre_hooks)
+    return bool("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or g._global_forward_hooks or g._global_forward_pre_hooks
+                or g._global_backward_hooks or g._global_backward_pre_hooks)
 
 
 class Linear(nn.Linear):

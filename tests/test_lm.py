@@ -366,3 +366,14 @@ def test_lm_training_memory_is_steady(monkeypatch, stack, dots):
         torch.cuda.synchronize()
         seen.append(torch.cuda.memory_allocated())
     assert len(set(seen[1:])) == 1, seen
+
+
+def test_a_forward_set_on_a_norm_is_called():
+    """A norm whose forward a wrapper replaced on the instance is called, not passed by."""
+    from loopback_amd import lm
+    norm = lm.RMSNorm(64)
+    assert not lm._hooked(norm)
+    norm.forward = lambda x: 2 * x
+    assert lm._hooked(norm)
+    x = torch.randn(3, 64)
+    assert torch.equal(lm.add_norm(norm, x)[1], 2 * x)
