@@ -180,7 +180,7 @@ class RMSNorm(nn.RMSNorm):
     """nn.RMSNorm, on the HIP kernel where it takes the rows."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if ops.norm_native(x, self.weight):
+        if ops.norm_native(x, self.weight, None, self.eps):
             return ops.add_rms_norm(x, None, self.weight, self.eps)[1]
         return super().forward(x)
 
@@ -188,7 +188,7 @@ class RMSNorm(nn.RMSNorm):
 def add_norm(norm: nn.Module, x: torch.Tensor, add: torch.Tensor | None = None):
     """(x + add, norm(x + add)); add None: (x, norm(x)). The kernel takes both steps in one pass, and the gradient
     that comes back along the first output joins the norm's in one, unless the norm's call is hooked."""
-    if type(norm) is RMSNorm and not _hooked(norm) and ops.norm_native(x, norm.weight, add):
+    if type(norm) is RMSNorm and not _hooked(norm) and ops.norm_native(x, norm.weight, add, norm.eps):
         return ops.add_rms_norm(x, add, norm.weight, norm.eps)
     h = x if add is None else x + add
     return h, norm(h)

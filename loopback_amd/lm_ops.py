@@ -151,8 +151,11 @@ def _rows_ok(*tensors) -> bool:
     return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
 
 
-def norm_native(x, w, add=None) -> bool:
-    """Whether add_rms_norm takes the call: rows of a multiple of 8 elements up to NORM_MAX_WIDTH, contiguous."""
+def norm_native(x, w, add=None, eps=0.0) -> bool:
+    """Whether add_rms_norm takes the call: rows of a multiple of 8 elements up to NORM_MAX_WIDTH, contiguous; eps given
+    (None, the type's epsilon, is torch's to choose)."""
+    if eps is None:
+        return False
     ts = (x, w) if add is None else (x, w, add)
     d = x.shape[-1] if x.dim() else 0
     return (native(*ts) and 8 <= d <= NORM_MAX_WIDTH and d % 8 == 0 and w.shape == (d,)

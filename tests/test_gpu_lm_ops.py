@@ -179,3 +179,11 @@ def test_only_on_the_current_gpu(monkeypatch):
     assert ops.native(x)
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.device.index + 1)
     assert not ops.native(x)
+
+
+def test_norm_without_eps():
+    """RMSNorm's own default, eps None (the type's epsilon), is torch's operation."""
+    from loopback_amd import lm
+    x, norm = rnd((3, 64), torch.bfloat16, 31), lm.RMSNorm(64).to(DEV, torch.bfloat16)
+    ref = F.rms_norm(x, (64,), norm.weight, None)
+    assert torch.equal(norm(x), ref) and torch.equal(lm.add_norm(norm, x)[1], ref)
