@@ -4,9 +4,9 @@ residual's add before it and the residual's gradient folded into its backward, S
 
 `native(...)` says whether the kernels take a call: plain 16-bit tensors of one dtype on the current GPU (a launch on
 another GPU's default stream would run on the current one), no transform or tracer that has to see torch operations
-(torch.func, forward-mode AD, torch.compile, jit tracing), no autocast. Everything else -- the CPU, fp32, other shapes --
-stays on torch in lm.py. A backward that is itself differentiated (create_graph) runs the torch form of the operation,
-so second derivatives are torch's.
+(torch.func, forward-mode AD, torch.compile, jit tracing, a dispatch mode such as make_fx's), no autocast. Everything
+else -- the CPU, fp32, other shapes -- stays on torch in lm.py. A backward that is itself differentiated (create_graph)
+runs the torch form of the operation, so second derivatives are torch's.
 """
 from __future__ import annotations
 
@@ -79,7 +79,7 @@ def native(*tensors) -> bool:
             return False
     return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
                 or torch.jit.is_tracing() or forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None)
+                or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None)
 
 
 def _again(fn, inputs, needed, grads):

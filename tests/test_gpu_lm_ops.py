@@ -187,3 +187,21 @@ def test_norm_without_eps():
     x, norm = rnd((3, 64), torch.bfloat16, 31), lm.RMSNorm(64).to(DEV, torch.bfloat16)
     ref = F.rms_norm(x, (64,), norm.weight, None)
     assert torch.equal(norm(x), ref) and torch.equal(lm.add_norm(norm, x)[1], ref)
+
+
+def test_dispatch_modes_see_torch_operations():
+    """make_fx records the operations of a norm, SwiGLU and the loss: its graph gives their results on other inputs (to
+    a few roundings of bf16, half a step 2^-9 to 2^-8 each)."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from loopback_amd import lm, lm_ops as ops
+    norm = lm.RMSNorm(64, eps=1e-6).to(DEV, torch.bfloat16).requires_grad_(False)
+    ids = torch.arange(6, device=DEV).view(2, 3)
+
+    def fn(x):
+        y = lm.add_norm(norm, x, x)[1]
+        return ops.swiglu(y), ops.next_token_loss(y, ids)
+
+    graph = make_fx(fn)(rnd((2, 3, 64), torch.bfloat16, 32))
+    x = rnd((2, 3, 64), torch.bfloat16, 33)
+    for got, ref in zip(graph(x), fn(x)):
+        assert (got.float() - ref.float()).norm() <= 2e-2 * ref.float().norm()
