@@ -69,17 +69,28 @@ def _stream(t: torch.Tensor) -> int:
     return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
+def _watched() -> bool:
+    """Whether something is on that has to see torch operations: torch.compile, jit tracing, a torch.func transform,
+    forward-mode AD, a dispatch mode."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def native(*tensors) -> bool:
+    # what watches the call first, then what the arguments are: a tracer's arguments (fake tensors, proxies) are not
+    # asked for a device, and a compiler meets no query of the GPU
+    if _watched():
+        return False
     first = tensors[0]
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
     if not first.is_cuda or first.dtype not in _CODES or first.device.index != torch._C._cuda_getDevice():
         return False
     for t in tensors:
-        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.dtype is not first.dtype \
-                or t.device != first.device:
+        if t.dtype is not first.dtype or t.device != first.device:
             return False
-    return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
-                or torch.jit.is_tracing() or forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None)
+    return not torch.is_autocast_enabled("cuda")
 
 
 def _again(fn, inputs, needed, grads):
@@ -157,8 +168,10 @@ def norm_native(x, w, add=None, eps=0.0) -> bool:
     if eps is None:
         return False
     ts = (x, w) if add is None else (x, w, add)
+    if not native(*ts):
+        return False
     d = x.shape[-1] if x.dim() else 0
-    return (native(*ts) and 8 <= d <= NORM_MAX_WIDTH and d % 8 == 0 and w.shape == (d,)
+    return (8 <= d <= NORM_MAX_WIDTH and d % 8 == 0 and w.shape == (d,)
             and (add is None or add.shape == x.shape) and _rows_ok(*ts))
 
 
