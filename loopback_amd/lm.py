@@ -130,6 +130,9 @@ def _hooked(m: nn.Module) -> bool:
                 or g._global_backward_hooks or g._global_backward_pre_hooks)
 
 
+# The model's layers are torch's own modules (what replaces, quantizes, scripts or traces modules by their type finds
+# them); the two functions below run a plain one on the kernels, and call any other. Linear and RMSNorm are the same as
+# modules, for programs that hold a layer alone.
 class Linear(nn.Linear):
     """nn.Linear without a bias, its weight's gradient on the HIP kernel where that is faster (lm_ops.linear)."""
 
@@ -137,20 +140,27 @@ class Linear(nn.Linear):
         return ops.linear(x, self.weight) if self.bias is None else super().forward(x)
 
 
+def linear(layer: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """layer(x), its weight's gradient on the HIP kernel where that is faster."""
+    if type(layer) is nn.Linear and layer.bias is None and ops.linear_native(x, layer.weight) and not _hooked(layer):
+        return ops.linear(x, layer.weight)
+    return layer(x)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
         self.h, self.dh = cfg.num_heads, cfg.hidden_size // cfg.num_heads
-        self.qkv = Linear(cfg.hidden_size, 3 * cfg.hidden_size, bias=False)
-        self.o = Linear(cfg.hidden_size, cfg.hidden_size, bias=False)
+        self.qkv = nn.Linear(cfg.hidden_size, 3 * cfg.hidden_size, bias=False)
+        self.o = nn.Linear(cfg.hidden_size, cfg.hidden_size, bias=False)
         self.rotary = Rotary(self.dh, cfg.rope_theta)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        qkv = self.qkv(x)
+        qkv = linear(self.qkv, x)
         if ops.attention_native(qkv, self.dh) and type(self.rotary) is Rotary and not _hooked(self.rotary):
             cos, sin = self.rotary.tables(x.shape[1], x.device, qkv.dtype)
-            return self.o(ops.rotary_attention(qkv, cos, sin, self.h, self.attend))
-        return self.o(self.attend(qkv))
+            return linear(self.o, ops.rotary_attention(qkv, cos, sin, self.h, self.attend))
+        return linear(self.o, self.attend(qkv))
 
     def attend(self, qkv: torch.Tensor) -> torch.Tensor:
         """The rotation and attention in torch operations: (B, T, 3 D) -> (B, T, D)."""
@@ -169,11 +179,16 @@ class Attention(nn.Module):
 class SwiGLU(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
-        self.gate_up = Linear(cfg.hidden_size, 2 * cfg.intermediate, bias=False)
-        self.down = Linear(cfg.intermediate, cfg.hidden_size, bias=False)
+        self.gate_up = nn.Linear(cfg.hidden_size, 2 * cfg.intermediate, bias=False)
+        self.down = nn.Linear(cfg.intermediate, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down(ops.swiglu(self.gate_up(x)))
+        if torch.jit.is_scripting():   # a scripted layer is torch operations
+            g, u = self.gate_up(x).chunk(2, dim=-1)
+            y = self.down(F.silu(g) * u)
+        else:
+            y = linear(self.down, ops.swiglu(linear(self.gate_up, x)))
+        return y
 
 
 class RMSNorm(nn.RMSNorm):
@@ -188,7 +203,7 @@ class RMSNorm(nn.RMSNorm):
 def add_norm(norm: nn.Module, x: torch.Tensor, add: torch.Tensor | None = None):
     """(x + add, norm(x + add)); add None: (x, norm(x)). The kernel takes both steps in one pass, and the gradient
     that comes back along the first output joins the norm's in one, unless the norm's call is hooked."""
-    if type(norm) is RMSNorm and not _hooked(norm) and ops.norm_native(x, norm.weight, add, norm.eps):
+    if type(norm) in (nn.RMSNorm, RMSNorm) and ops.norm_native(x, norm.weight, add, norm.eps) and not _hooked(norm):
         return ops.add_rms_norm(x, add, norm.weight, norm.eps)
     h = x if add is None else x + add
     return h, norm(h)
@@ -197,9 +212,9 @@ def add_norm(norm: nn.Module, x: torch.Tensor, add: torch.Tensor | None = None):
 class Block(nn.Module):
     def __init__(self, cfg: LMConfig):
         super().__init__()
-        self.attn_norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.attn_norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.attn = Attention(cfg)
-        self.mlp_norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.mlp_norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.mlp = SwiGLU(cfg)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -219,7 +234,7 @@ class LoopbackLM(nn.Module):
         self.prelude = nn.ModuleList(Block(cfg) for _ in range(cfg.prelude))
         self.middle = nn.ModuleList(Block(cfg) for _ in range(cfg.loop_blocks))   # shared over the R iterations
         self.coda = nn.ModuleList(Block(cfg) for _ in range(cfg.coda))
-        self.norm = RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
+        self.norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
         self.head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
         self.read = (LoopDeltaAttnRes(cfg.hidden_size, cfg.loops, cfg.loop_blocks, beta=cfg.beta, eps=cfg.norm_eps)
                      if cfg.residual == "delta_attnres" else None)
@@ -266,7 +281,7 @@ class LoopbackLM(nn.Module):
                     h, coeffs, prior = self.read.combine(hs, h0, deltas, coeffs, prior, l, blk, keys=keys)
         for blk in self.coda:
             h = blk(h)
-        return self.norm(h)
+        return add_norm(self.norm, h)[1]
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         return ops.next_token_loss(self.head(self.hidden(ids)), ids)

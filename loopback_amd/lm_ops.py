@@ -343,11 +343,14 @@ class _Linear(torch.autograd.Function):
         return dx, wgrad(dy, x.view(-1, w.shape[1])) if ctx.needs_input_grad[1] else None
 
 
+def linear_native(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether linear(x, w) records a weight gradient by llm_wgrad."""
+    return (torch.is_grad_enabled() and x.dtype is torch.bfloat16 and native(x, w) and w.requires_grad and x.dim() > 1
+            and w.dim() == 2 and x.shape[-1] == w.shape[1] and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1]
+            and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and _rows_ok(x, w)
+            and LIB.llm_wgrad_splits(x.numel() // w.shape[1], *w.shape) >= WGRAD_MIN_SPLITS)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w), with the weight's gradient by llm_wgrad where that is the faster one."""
-    if (torch.is_grad_enabled() and w.requires_grad and x.dtype is torch.bfloat16 and x.dim() > 1 and w.dim() == 2
-            and x.shape[-1] == w.shape[1] and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1] and w.shape[0] % 8 == 0
-            and w.shape[1] % 8 == 0 and native(x, w) and _rows_ok(x, w)
-            and LIB.llm_wgrad_splits(x.numel() // w.shape[1], *w.shape) >= WGRAD_MIN_SPLITS):
-        return _Linear.apply(x, w)
-    return F.linear(x, w)
+    return _Linear.apply(x, w) if linear_native(x, w) else F.linear(x, w)

@@ -47,3 +47,47 @@ def test_compiled_block_is_one_graph():
     with torch.no_grad():
         got, ref = torch.compile(block, backend="eager", fullgraph=True)(x), block(x)
     assert (got.float() - ref.float()).norm() <= 2e-2 * ref.float().norm()
+
+
+def test_layers_are_torch_modules():
+    """What finds layers by their type finds the model's: its linear layers and norms are torch's own classes, dynamic
+    quantization replaces them, torch.fx keeps them as leaves (with SwiGLU's operations between), and a SwiGLU and a
+    norm can be scripted. Each gives the eager results."""
+    from torch import nn
+    block = lm.Block(CFG)
+    assert [type(m) for m in block.modules() if isinstance(m, (nn.Linear, nn.RMSNorm))] == \
+        [nn.RMSNorm, nn.Linear, nn.Linear, nn.RMSNorm, nn.Linear, nn.Linear]
+    assert type(lm.LoopbackLM(lm.LMConfig(hidden_size=64, num_heads=2, vocab_size=32)).norm) is nn.RMSNorm
+    x = torch.randn(2, 8, 128)
+
+    class AttentionLeaf(torch.fx.Tracer):
+        def is_leaf_module(self, m, name):
+            return isinstance(m, lm.Attention) or super().is_leaf_module(m, name)
+
+    tracer = AttentionLeaf()
+    graph = tracer.trace(block)
+    assert [n.target for n in graph.nodes if n.op == "call_module"] == \
+        ["attn_norm", "attn", "mlp_norm", "mlp.gate_up", "mlp.down"]
+    ref = block(x)
+    assert torch.equal(torch.fx.GraphModule(tracer.root, graph)(x), ref)
+    assert torch.equal(torch.fx.symbolic_trace(lm.RMSNorm(128, eps=1e-6))(x), lm.RMSNorm(128, eps=1e-6)(x))
+    assert torch.allclose(torch.jit.script(block.mlp)(x), block.mlp(x), atol=1e-6)
+    assert torch.allclose(torch.jit.script(block.mlp_norm)(x), block.mlp_norm(x), atol=1e-6)
+    quantized = torch.ao.quantization.quantize_dynamic(block, {nn.Linear}, dtype=torch.qint8)
+    assert not any(isinstance(m, nn.Linear) for m in quantized.modules())
+    assert (quantized(x) - ref).norm() <= 5e-2 * ref.norm()   # 8-bit weights and activations
+
+
+def test_a_hooked_linear_layer_is_called(monkeypatch):
+    """A linear layer whose call is hooked, or that has a bias, is called as a module where the kernel would take it."""
+    from torch import nn
+    monkeypatch.setattr(lm.ops, "linear_native", lambda x, w: True)
+    x = torch.randn(2, 16)
+    for bias, hooked, calls in ((False, False, 0), (False, True, 1), (True, False, 0)):
+        layer, seen = nn.Linear(16, 8, bias=bias), []
+        taken = []
+        monkeypatch.setattr(lm.ops, "linear", lambda x, w: taken.append(1) or torch.nn.functional.linear(x, w))
+        if hooked:
+            layer.register_forward_hook(lambda m, i, o: seen.append(1))
+        assert torch.equal(lm.linear(layer, x), layer.forward(x))
+        assert len(seen) == calls and bool(taken) == (not hooked and not bias)
