@@ -93,22 +93,19 @@ def native(*tensors) -> bool:
     return not torch.is_autocast_enabled("cuda")
 
 
-def _again(fn, inputs, needed, grads):
+def _again(fn, inputs, needed, grad):
     """The gradients of fn at `inputs`, as torch forms them with a graph (a backward that is differentiated)."""
+    wanted = [x for x, need in zip(inputs, needed) if need]
+    if not wanted:
+        return [None] * len(needed)
     with torch.enable_grad():
-        outs = fn(*inputs)
-        wanted = [x for x, need in zip(inputs, needed) if need]
-        got = iter(torch.autograd.grad(outs, wanted, grads, create_graph=True, allow_unused=True))
+        got = iter(torch.autograd.grad(fn(*inputs), wanted, grad, create_graph=True))
     return [next(got) if need else None for need in needed]
 
 
 # ---------------------------------------------------------------------------------------------------------------
 # RMSNorm
 # ---------------------------------------------------------------------------------------------------------------
-def _norm_torch(eps):
-    return lambda h, w: (h, F.rms_norm(h, (h.shape[-1],), w, eps))
-
-
 class _AddRmsNorm(torch.autograd.Function):
     """(h, y) = (x + add, rms_norm(x + add) w); add may be None (h is then x itself, as an alias). h carries the
     residual stream on, so the gradient that comes back along it joins the norm's in one kernel."""
@@ -126,6 +123,8 @@ class _AddRmsNorm(torch.autograd.Function):
         ctx.eps, ctx.added = eps, add is not None
         ctx.save_for_backward(x if add is None else h, w, rstd)
         ctx.set_materialize_grads(False)
+        if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
+            ctx.mark_non_differentiable(h)   # only the weight is trained: the residual stream needs no gradient
         return h, y
 
     @staticmethod
@@ -133,9 +132,10 @@ class _AddRmsNorm(torch.autograd.Function):
         h, w, rstd = ctx.saved_tensors
         if dy is None:
             return dh, dh if ctx.added else None, None, None
+        needed = [ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]]
         if torch.is_grad_enabled():
-            dh = torch.zeros_like(dy) if dh is None else dh
-            dx, dw = _again(_norm_torch(ctx.eps), [h, w], [True, ctx.needs_input_grad[2]], (dh, dy))
+            dx, dw = _again(lambda h, w: F.rms_norm(h, (h.shape[-1],), w, ctx.eps), [h, w], needed, dy)
+            dx = dx if dx is None or dh is None else dx + dh
             return dx, dx if ctx.added else None, dw, None
         d = h.shape[-1]
         rows = h.numel() // d
@@ -201,7 +201,7 @@ class _SwiGLU(torch.autograd.Function):
     def backward(ctx, da):
         gu, = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return _again(_swiglu_torch, [gu], [True], (da,))[0]
+            return _again(_swiglu_torch, [gu], [True], da)[0]
         n = gu.shape[-1] // 2
         da = _dense(da, gu)
         dgu = torch.empty_like(gu)
@@ -243,7 +243,7 @@ class _NextTokenLoss(torch.autograd.Function):
     def backward(ctx, g):
         logits, ids, lse = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return _again(_loss_torch(ids), [logits], [True], (g,))[0], None
+            return _again(_loss_torch(ids), [logits], [True], g)[0], None
         b, t, vocab = logits.shape
         dlogits = torch.empty_like(logits)
         _run("llm_next_token_loss_bwd", logits.data_ptr(), ids.data_ptr(), lse.data_ptr(), g.data_ptr(),
@@ -284,7 +284,7 @@ class _RotaryAttention(torch.autograd.Function):
     def backward(ctx, dout):
         qkv, qk, out, lse2, cos, sin = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return _again(ctx.again, [qkv], [True], (dout,))[0], None, None, None, None
+            return _again(ctx.again, [qkv], [True], dout)[0], None, None, None, None
         b, t, _ = qkv.shape
         dout = _dense(dout, out)
         delta = torch.empty_like(lse2)
@@ -337,7 +337,7 @@ class _Linear(torch.autograd.Function):
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return tuple(_again(F.linear, [x, w], ctx.needs_input_grad, (dy,)))
+            return tuple(_again(F.linear, [x, w], ctx.needs_input_grad, dy))
         dy = _dense(dy, x).view(-1, w.shape[0])
         dx = (dy @ w).view(x.shape) if ctx.needs_input_grad[0] else None
         return dx, wgrad(dy, x.view(-1, w.shape[1])) if ctx.needs_input_grad[1] else None
