@@ -5,8 +5,8 @@ residual's add before it and the residual's gradient folded into its backward, S
 `native(...)` says whether the kernels take a call: plain 16-bit tensors of one dtype on the current GPU (a launch on
 another GPU's default stream would run on the current one), no transform or tracer that has to see torch operations
 (torch.func, forward-mode AD, torch.compile, jit tracing, a dispatch mode such as make_fx's), no autocast. Everything
-else -- the CPU, fp32, other shapes -- stays on torch in lm.py. A backward that is itself differentiated (create_graph)
-runs the torch form of the operation, so second derivatives are torch's.
+else -- the CPU, fp32, other shapes -- stays on torch in lm.py. A backward that is itself differentiated (create_graph),
+that one of these watches or that gets batched gradients runs the torch form of the operation.
 """
 from __future__ import annotations
 
@@ -93,13 +93,26 @@ def native(*tensors) -> bool:
     return not torch.is_autocast_enabled("cuda")
 
 
+def _launchable(*grads) -> bool:
+    """Whether a backward runs on the kernels: it is not itself differentiated, nothing watches it, and its gradients
+    are plain tensors (not the batched ones of is_grads_batched and jacobian(vectorize=True))."""
+    if torch.is_grad_enabled() or _watched():
+        return False
+    for g in grads:
+        if g is not None and ((type(g) is not torch.Tensor and type(g) is not torch.nn.Parameter)
+                              or torch._C._functorch.is_legacy_batchedtensor(g)):
+            return False
+    return True
+
+
 def _again(fn, inputs, needed, grad):
-    """The gradients of fn at `inputs`, as torch forms them with a graph (a backward that is differentiated)."""
+    """The gradients of fn at `inputs` as torch forms them, with a graph where this backward is differentiated."""
     wanted = [x for x, need in zip(inputs, needed) if need]
     if not wanted:
         return [None] * len(needed)
+    graph = torch.is_grad_enabled()
     with torch.enable_grad():
-        got = iter(torch.autograd.grad(fn(*inputs), wanted, grad, create_graph=True))
+        got = iter(torch.autograd.grad(fn(*inputs), wanted, grad, create_graph=graph))
     return [next(got) if need else None for need in needed]
 
 
@@ -133,7 +146,7 @@ class _AddRmsNorm(torch.autograd.Function):
         if dy is None:
             return dh, dh if ctx.added else None, None, None
         needed = [ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]]
-        if torch.is_grad_enabled():
+        if not _launchable(dh, dy):
             dx, dw = _again(lambda h, w: F.rms_norm(h, (h.shape[-1],), w, ctx.eps), [h, w], needed, dy)
             dx = dx if dx is None or dh is None else dx + dh
             return dx, dx if ctx.added else None, dw, None
@@ -200,7 +213,7 @@ class _SwiGLU(torch.autograd.Function):
     @staticmethod
     def backward(ctx, da):
         gu, = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _launchable(da):
             return _again(_swiglu_torch, [gu], [True], da)[0]
         n = gu.shape[-1] // 2
         da = _dense(da, gu)
@@ -242,7 +255,7 @@ class _NextTokenLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         logits, ids, lse = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _launchable(g):
             return _again(_loss_torch(ids), [logits], [True], g)[0], None
         b, t, vocab = logits.shape
         dlogits = torch.empty_like(logits)
@@ -283,7 +296,7 @@ class _RotaryAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         qkv, qk, out, lse2, cos, sin = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _launchable(dout):
             return _again(ctx.again, [qkv], [True], dout)[0], None, None, None, None
         b, t, _ = qkv.shape
         dout = _dense(dout, out)
@@ -336,7 +349,7 @@ class _Linear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _launchable(dy):
             return tuple(_again(F.linear, [x, w], ctx.needs_input_grad, dy))
         dy = _dense(dy, x).view(-1, w.shape[0])
         dx = (dy @ w).view(x.shape) if ctx.needs_input_grad[0] else None

@@ -40,6 +40,41 @@ def test_norm_second_derivatives(no_launch, need_x, need_w, add):
         assert (p is None) == (q is None) and (p is None or (p - q).float().norm() <= 2e-2 * q.float().norm() + 1e-6)
 
 
+def _operations(monkeypatch):
+    """name -> (the kernel operation, its torch form, the input it is differentiated by)."""
+    monkeypatch.setattr(ops, "wgrad", lambda dy, x: pytest.fail("a weight gradient was launched"))
+    w, u, ids = rnd((64,), 2), rnd((32, 64), 5), torch.arange(6).view(2, 3)
+    cos, sin = lm.Rotary(64, 1e6).tables(3, "cpu", torch.bfloat16)
+    attn = lm.Attention(lm.LMConfig(hidden_size=64, num_heads=1))
+    return {"norm": (lambda x: ops.add_rms_norm(x, None, w, 1e-6)[1], lambda x: F.rms_norm(x, (64,), w, 1e-6),
+                     rnd((5, 64), 1)),
+            "swiglu": (ops._SwiGLU.apply, ops._swiglu_torch, rnd((5, 64), 1)),
+            "loss": (lambda x: ops._NextTokenLoss.apply(x, ids), ops._loss_torch(ids), rnd((2, 3, 64), 1)),
+            "linear": (lambda x: ops._Linear.apply(x, u), lambda x: F.linear(x, u), rnd((5, 64), 1)),
+            "attention": (lambda x: ops.rotary_attention(x, cos, sin, 1, attn.attend), attn.attend, rnd((1, 3, 192), 1))}
+
+
+@pytest.mark.parametrize("name", ["norm", "swiglu", "loss", "linear", "attention"])
+@pytest.mark.parametrize("how", ["batched", "vmap", "mode"])
+def test_watched_backwards(no_launch, monkeypatch, name, how):
+    """Batched gradients, a vmap over the backward, and a dispatch mode around it: torch's operations."""
+    fn, ref_fn, x = _operations(monkeypatch)[name]
+    x.requires_grad_()
+    y, yr = fn(x), ref_fn(x)
+    gs = torch.stack([rnd(y.shape, k, y.dtype) for k in (7, 8)])
+
+    def grads(out):
+        if how == "batched":
+            return torch.autograd.grad(out, x, gs, is_grads_batched=True)[0]
+        if how == "vmap":
+            return torch.func.vmap(lambda g: torch.autograd.grad(out, x, g, retain_graph=True)[0])(gs)
+        from torch.utils.flop_counter import FlopCounterMode
+        with FlopCounterMode(display=False):
+            return torch.autograd.grad(out, x, gs[0])[0]
+
+    assert torch.allclose(grads(y), grads(yr), rtol=1e-2, atol=1e-3)
+
+
 @pytest.mark.gpu
 def test_block_gradients_with_a_graph():
     """A block fed plain activations, its parameters' gradients taken with a graph: those taken without."""
