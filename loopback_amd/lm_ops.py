@@ -105,6 +105,13 @@ def _launchable(*grads) -> bool:
     return True
 
 
+def _saved(ctx):
+    """The saved tensors as the kernels take them: a saved-tensor hook may give one back with other strides or another
+    alignment than it was saved with."""
+    ts = ctx.saved_tensors
+    return ts if _rows_ok(*ts) else [t if _rows_ok(t) else t.clone(memory_format=torch.contiguous_format) for t in ts]
+
+
 def _again(fn, inputs, needed, grad):
     """The gradients of fn at `inputs` as torch forms them, with a graph where this backward is differentiated."""
     wanted = [x for x, need in zip(inputs, needed) if need]
@@ -142,7 +149,7 @@ class _AddRmsNorm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dh, dy):
-        h, w, rstd = ctx.saved_tensors
+        h, w, rstd = _saved(ctx)
         if dy is None:
             return dh, dh if ctx.added else None, None, None
         needed = [ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]]
@@ -212,7 +219,7 @@ class _SwiGLU(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, da):
-        gu, = ctx.saved_tensors
+        gu, = _saved(ctx)
         if not _launchable(da):
             return _again(_swiglu_torch, [gu], [True], da)[0]
         n = gu.shape[-1] // 2
@@ -254,7 +261,7 @@ class _NextTokenLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        logits, ids, lse = ctx.saved_tensors
+        logits, ids, lse = _saved(ctx)
         if not _launchable(g):
             return _again(_loss_torch(ids), [logits], [True], g)[0], None
         b, t, vocab = logits.shape
@@ -295,7 +302,7 @@ class _RotaryAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        qkv, qk, out, lse2, cos, sin = ctx.saved_tensors
+        qkv, qk, out, lse2, cos, sin = _saved(ctx)
         if not _launchable(dout):
             return _again(ctx.again, [qkv], [True], dout)[0], None, None, None, None
         b, t, _ = qkv.shape
@@ -348,7 +355,7 @@ class _Linear(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        x, w = ctx.saved_tensors
+        x, w = _saved(ctx)
         if not _launchable(dy):
             return tuple(_again(F.linear, [x, w], ctx.needs_input_grad, dy))
         dy = _dense(dy, x).view(-1, w.shape[0])

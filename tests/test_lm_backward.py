@@ -75,6 +75,41 @@ def test_watched_backwards(no_launch, monkeypatch, name, how):
     assert torch.allclose(grads(y), grads(yr), rtol=1e-2, atol=1e-3)
 
 
+def test_saved_tensors_with_other_strides():
+    """What a saved-tensor hook gives back strided or unaligned reaches the kernels as contiguous aligned rows."""
+    ctx = type("ctx", (), {})()
+    x = rnd((4, 8), 1)
+    ctx.saved_tensors = (x, x.t().contiguous().t(), torch.cat((x.new_zeros(1), x.flatten()))[1:].view(4, 8),
+                         torch.ones(1)[0], x[:0])
+    for got, t in zip(ops._saved(ctx), ctx.saved_tensors):
+        assert torch.equal(got, t) and got.is_contiguous() and got.data_ptr() % 16 == 0
+    assert ops._saved(ctx)[0] is x
+    ctx.saved_tensors = (x,)
+    assert ops._saved(ctx) is ctx.saved_tensors
+
+
+@pytest.mark.gpu
+def test_gradients_through_saved_tensor_hooks():
+    """Hooks that transpose what is saved and give back transposed views: the gradients' bits without them."""
+    w, ids = rnd((192,), 2).cuda().requires_grad_(), torch.arange(80).view(2, 40).cuda()
+    cos, sin = lm.Rotary(64, 1e6).tables(40, torch.device("cuda", 0), torch.bfloat16)
+    x = rnd((2, 40, 192), 1).cuda().requires_grad_()
+
+    def grads():
+        h, n = ops.add_rms_norm(x, None, w, 1e-6)
+        a = ops.rotary_attention(n, cos, sin, 1, None)
+        y = ops.add_rms_norm(ops.swiglu(h + n), a.repeat(1, 1, 3)[..., :96].contiguous(), w[:96].detach(), 1e-6)[1]
+        return ops.next_token_loss(y, ids)
+
+    print("case saved-tensor hooks", flush=True)
+    ref = torch.autograd.grad(grads(), (x, w))
+    turn = lambda t: t.transpose(0, -1).contiguous() if t.dim() > 1 else t
+    with torch.autograd.graph.saved_tensors_hooks(turn, lambda t: t.transpose(0, -1) if t.dim() > 1 else t):
+        loss = grads()
+    for p, q in zip(torch.autograd.grad(loss, (x, w)), ref):
+        assert torch.equal(p, q)
+
+
 @pytest.mark.gpu
 def test_block_gradients_with_a_graph():
     """A block fed plain activations, its parameters' gradients taken with a graph: those taken without."""
