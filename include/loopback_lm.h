@@ -32,7 +32,8 @@ int llm_rms_norm_fwd(const void* x, const void* add, const void* w, void* h_out,
 int64_t llm_rms_norm_parts(int64_t rows);
 
 /* dx = round(r (dy w - h r mean(dy w h r)) + dres) (dres, another gradient of h, may be NULL) and the partial weight
- * gradients dw_part [llm_rms_norm_parts(rows), d], whose column sums are sum_rows dy h r. */
+ * gradients dw_part [llm_rms_norm_parts(rows), d], whose column sums are sum_rows dy h r. Either result may be NULL (not
+ * wanted), not both. */
 int llm_rms_norm_bwd(const void* dy, const void* h, const void* w, const float* rstd, const void* dres, void* dx,
                      float* dw_part, int64_t rows, int64_t d, int dtype, void* stream);
 

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(WG) void k_rms_norm_fwd(const T* __restrict__ x, co
 }
 
 // A workgroup's waves take rows in turn and keep the weight gradient's columns in registers; the four waves' sums meet
-// in LDS, one partial row per workgroup.
+// in LDS, one partial row per workgroup. dx or dw_part NULL: not asked for, not written.
 constexpr int NORM_GRID = 512;
 
 template <typename T, int VPT>
@@ -114,6 +114,7 @@ __global__ __launch_bounds__(WG) void k_rms_norm_bwd(const T* __restrict__ dy, c
         dw[v][k] = __builtin_fmaf(a[k], b[k] * r, dw[v][k]);
       }
     }
+    if (!dx) continue;
     c = lanes_reduce(c, 64, AddOp()) * r * r / (float)d;
 #pragma unroll
     for (int v = 0; v < VPT; ++v) {
@@ -133,6 +134,7 @@ __global__ __launch_bounds__(WG) void k_rms_norm_bwd(const T* __restrict__ dy, c
       }
     }
   }
+  if (!dw_part) return;
   for (int k = 0; k < WAVES; ++k) {
     if (wave == k) {
 #pragma unroll
@@ -970,7 +972,7 @@ int llm_rms_norm_bwd(const void* dy, const void* h, const void* w, const float* 
   if (d < 8 || (d & 7) || d > LLM_NORM_MAX_WIDTH) return LDR_E_SHAPE;
   if (rows < 0 || !w) return LDR_E_ARG;
   if (rows == 0) return LDR_OK;
-  if (!dy || !h || !rstd || !dx || !dw_part) return LDR_E_ARG;
+  if (!dy || !h || !rstd || (!dx && !dw_part)) return LDR_E_ARG;
   if (!al16(dy) || !al16(h) || !al16(w) || !al16(dx) || !al16(dres)) return LDR_E_ALIGN;
   const int vpt = (int)((d / 8 + 63) / 64);
   LLM_DTYPE_SWITCH(dtype, LLM_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rms_norm_bwd<T, VPT>),

@@ -161,14 +161,17 @@ class _AddRmsNorm(torch.autograd.Function):
         rows = h.numel() // d
         dy = _dense(dy, h)
         dres = None if dh is None else _dense(dh, h)
-        dx = torch.empty_like(h)
-        parts = LIB.llm_rms_norm_parts(rows)
-        part = torch.empty((parts, d), device=h.device, dtype=torch.float32)
-        dw = torch.empty_like(w)
-        _run("llm_rms_norm_bwd", dy.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(),
-             None if dres is None else dres.data_ptr(), dx.data_ptr(), part.data_ptr(), rows, d, _CODES[h.dtype],
-             _stream(h))
-        _run("llm_sum_rows", part.data_ptr(), parts, d, dw.data_ptr(), _CODES[w.dtype], _stream(h))
+        dx = torch.empty_like(h) if needed[0] else None
+        dw = part = None
+        if needed[1]:
+            parts = LIB.llm_rms_norm_parts(rows)
+            part = torch.empty((parts, d), device=h.device, dtype=torch.float32)
+            dw = torch.empty_like(w)
+        ptr = lambda t: None if t is None else t.data_ptr()
+        _run("llm_rms_norm_bwd", dy.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(), ptr(dres), ptr(dx),
+             ptr(part), rows, d, _CODES[h.dtype], _stream(h))
+        if needed[1]:
+            _run("llm_sum_rows", part.data_ptr(), parts, d, dw.data_ptr(), _CODES[w.dtype], _stream(h))
         return dx, dx if ctx.added else None, dw, None
 
 

@@ -40,6 +40,37 @@ def test_norm_second_derivatives(no_launch, need_x, need_w, add):
         assert (p is None) == (q is None) and (p is None or (p - q).float().norm() <= 2e-2 * q.float().norm() + 1e-6)
 
 
+def test_norm_backward_forms_what_is_needed(monkeypatch):
+    """A frozen gain gets no partial sums and no reduction, an input that needs no gradient none."""
+    launches = []
+    monkeypatch.setattr(ops, "_run", lambda name, *args: launches.append((name, args)))
+    monkeypatch.setattr(ops, "_stream", lambda t: 0)
+    for need_x, need_w in ((True, False), (False, True), (True, True)):
+        x, w = rnd((5, 64), 1).requires_grad_(need_x), rnd((64,), 2).requires_grad_(need_w)
+        y = ops.add_rms_norm(x, None, w, 1e-6)[1]
+        launches.clear()
+        y.backward(rnd((5, 64), 3))
+        assert [n for n, _ in launches] == ["llm_rms_norm_bwd"] + ["llm_sum_rows"] * need_w
+        assert (launches[0][1][5] is not None) == need_x and (launches[0][1][6] is not None) == need_w
+    assert ops.LIB.llm_rms_norm_bwd(4096, 4096, 4096, 4096, None, None, None, 1, 64, 1, None) == -1   # neither
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,d", [(5, 64), (2049, 768), (9, 2048)])
+def test_norm_gradients_one_at_a_time(rows, d):
+    """Each gradient alone has the bits it has beside the other."""
+    print(f"case norm gradients alone {rows}x{d}", flush=True)
+    x, w, g = (rnd(s, k).cuda() for s, k in (((rows, d), 1), ((d,), 2), ((rows, d), 3)))
+    got = {}
+    for need in ((True, True), (True, False), (False, True)):
+        a, b = x.clone().requires_grad_(need[0]), w.clone().requires_grad_(need[1])
+        ops.add_rms_norm(a, None, b, 1e-6)[1].backward(g)
+        got[need] = a.grad, b.grad
+    both = got[True, True]
+    assert torch.equal(got[True, False][0], both[0]) and got[True, False][1] is None
+    assert torch.equal(got[False, True][1], both[1]) and got[False, True][0] is None
+
+
 def _operations(monkeypatch):
     """name -> (the kernel operation, its torch form, the input it is differentiated by)."""
     monkeypatch.setattr(ops, "wgrad", lambda dy, x: pytest.fail("a weight gradient was launched"))
