@@ -2845,8 +2845,26 @@ template <typename T, int VPT> struct URing {
   static constexpr int PD = std::is_same<T, float>::value ? (VPT == 1 ? 4 : VPT <= 3 ? 2 : 1) : (VPT <= 2 ? 4 : VPT == 3 ? 3 : 2);
 };
 
+// s += w x in fp32; COMP: with what the sum loses to rounding kept in c (Kahan's summation: the sum is s - c)
+template <bool COMP> __device__ __forceinline__ void add_comp(float& s, float& c, float w, float x) {
+  if (COMP) {
+    const float y = __builtin_fmaf(w, x, -c), t = s + y;
+    c = (t - s) - y;
+    s = t;
+  } else {
+    s += w * x;
+  }
+}
+
 // The read (k_read_fwd without stored scores q == NULL, k_read_online with): its formulas and summation orders.
-// Dynamic LDS: c0, lc, p0 [n], then per row of the workgroup its logits, fixed weights and scales [n].
+// Dynamic LDS: c0, lc, p0 [n], then per row of the workgroup its logits, fixed weights and scales [n], and the query for
+// wide fp32 rows.
+// Forming the softmax as the sources stream splits a source's weight into a fixed part and a share of the softmax, whose
+// sums are larger than the correction they add up to: plain fp32 sums left an fp32 result 1.0 (2 sources) to 1.9 times (64)
+// as far from 64 bits as one weight per source. fp32 sums are compensated, the base added last (an infinite base would
+// turn the compensation into NaN): 0.75 to 0.98 times. 12 sources of 16384 x 1001 197 -> 205 us, 70 of 4096 x 768
+// 202 -> 220, 16 of 8192 x 2049 271 -> 315, 8 of 4096 x 8191 276 -> 369 (two passes over the sources: 498, 852, 703,
+// 1046). Results in 16 bits are the same distance away either way (their own rounding), and keep plain sums.
 template <typename T, int VPT, bool BLEND, typename TAB>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_rows_read(TAB src, int n, const float* __restrict__ q,
                                                   float* __restrict__ dots, int64_t dots_stride,
@@ -2854,10 +2872,12 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
                                                   Coef cf, float inv, T* __restrict__ out, float* __restrict__ tc,
                                                   float* __restrict__ prob, float* __restrict__ next_prior,
                                                   int64_t n_tok, int d, int tpr) {
-  extern __shared__ float dyn[];
+  extern __shared__ __align__(16) float dyn[];
   __shared__ float s_M, red[4];
   __shared__ int s_qnz;
   using Raw = typename IO<T>::Raw;
+  constexpr bool COMP = std::is_same<T, float>::value;
+  constexpr bool QLDS = COMP && VPT >= 3;   // the query in LDS: the sums leave no registers for it
   constexpr int PD = URing<T, VPT>::PD;
   const URows R(d, tpr);
   const int tid = (int)threadIdx.x;
@@ -2879,17 +2899,24 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
     for (int i = 0; i < n; ++i) m += s_c0[i];
     s_M = m;
   }
-  float qv[VPT][8];
+  float qv[QLDS ? 1 : VPT][8];
+  // QLDS: vector v's halves at [v][half][lane of the row], alike for every row (written by the first)
+  float4* s_q = reinterpret_cast<float4*>(dyn + ((3 * n * (1 + R.rpw) + 3) & ~3)) + R.lr;
   typename UIO<T>::Mask mk[VPT];
   bool nz = false;
 #pragma unroll
   for (int v = 0; v < VPT; ++v) {
     mk[v] = UIO<T>::mask(R.skip(v));
+    float (&o)[8] = qv[QLDS ? 0 : v];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const float x = q ? q[R.off(v) + k] : 0.f;
-      qv[v][k] = k >= R.skip(v) ? x : 0.f;
-      nz |= qv[v][k] != 0.f;
+      o[k] = k >= R.skip(v) ? x : 0.f;
+      nz |= o[k] != 0.f;
+    }
+    if (QLDS && R.rs == 0) {
+      s_q[(2 * v) * tpr] = make_float4(o[0], o[1], o[2], o[3]);
+      s_q[(2 * v + 1) * tpr] = make_float4(o[4], o[5], o[6], o[7]);
     }
   }
   if (nz) s_qnz = 1;   // every writer stores the same value
@@ -2911,9 +2938,30 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
 #pragma unroll
     for (int j = 0; j < PD; ++j)
       if (j < n) load_src(j, buf[j]);
-    float acc[VPT][8];
+    auto load_base = [&](float (&o)[VPT][8]) {
 #pragma unroll
-    for (int v = 0; v < VPT; ++v) IO<T>::unpack(UIO<T>::raw(base + roff + R.off(v)), acc[v]);
+      for (int v = 0; v < VPT; ++v) IO<T>::unpack(UIO<T>::raw(base + roff + R.off(v)), o[v]);
+      if (BLEND) {   // iteration end: base = proposal + beta (h0 - proposal), each step rounded as the caller's ops
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) {
+          float hv[8];
+          IO<T>::unpack(UIO<T>::raw(h0 + roff + R.off(v)), hv);
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            o[v][k] = IO<T>::round(o[v][k] + IO<T>::round(beta * IO<T>::round(hv[k] - o[v][k])));
+        }
+      }
+    };
+    float acc[VPT][8];
+    if (COMP) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[v][k] = 0.f;
+    } else {
+      load_base(acc);
+    }
     for (int i = R.lr; i < n; i += tpr) {   // the row's per-source scalars, spread over its lanes
       const float cb = coef_cbar(cf, tk, i), rv = src.r(i)[tk];
       if (online) {
@@ -2938,23 +2986,12 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
       }
       R.sync();
     }
-    if (BLEND) {   // iteration end: base = proposal + beta (h0 - proposal), each step rounded as the caller's ops
-#pragma clang fp contract(off)
-#pragma unroll
-      for (int v = 0; v < VPT; ++v) {
-        float hv[8];
-        IO<T>::unpack(UIO<T>::raw(h0 + roff + R.off(v)), hv);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          acc[v][k] = IO<T>::round(acc[v][k] + IO<T>::round(beta * IO<T>::round(hv[k] - acc[v][k])));
-      }
-    }
-    float P[VPT][8];
+    float P[VPT][8], cp[VPT][8], ca[VPT][8];   // cp, ca: what P and acc lost to rounding (COMP)
 #pragma unroll
     for (int v = 0; v < VPT; ++v)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) P[v][k] = 0.f;
-    float S = 0.f, mref = -INFINITY;
+      for (int k = 0; k < 8; ++k) P[v][k] = cp[v][k] = ca[v][k] = 0.f;
+    float S = 0.f, cs = 0.f, mref = -INFINITY;
     auto one = [&](int i, Raw (&rw)[VPT]) {   // source i, then its slot refilled with source i + PD
       float e[VPT][8];
 #pragma unroll
@@ -2963,9 +3000,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
       if (online) {
         float pd[1] = {0.f};
 #pragma unroll
-        for (int v = 0; v < VPT; ++v)
+        for (int v = 0; v < VPT; ++v) {
+          if (QLDS) IO<float>::unpack(IO<float>::Raw{s_q[(2 * v) * tpr], s_q[(2 * v + 1) * tpr]}, qv[0]);
 #pragma unroll
-          for (int k = 0; k < 8; ++k) pd[0] += qv[v][k] * e[v][k];
+          for (int k = 0; k < 8; ++k) pd[0] += qv[QLDS ? 0 : v][k] * e[v][k];
+        }
         row_sum<1>(pd, tpr, red);
         const float l = pd[0] * rsc[i] * inv + s_lc[i];
         if (R.lr == 0) {
@@ -2976,25 +3015,29 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
           if (l > mref + RF_LAZY) {   // the reference maximum moves: the running sums rescaled (k_read_online)
             const float a = expf(mref - l);
             S *= a;
+            if (COMP) cs *= a;
 #pragma unroll
             for (int v = 0; v < VPT; ++v)
 #pragma unroll
-              for (int k = 0; k < 8; ++k) P[v][k] *= a;
+              for (int k = 0; k < 8; ++k) {
+                P[v][k] *= a;
+                if (COMP) cp[v][k] *= a;
+              }
             mref = l;
           }
           const float ex = expf(l - mref);
-          S += ex;
+          add_comp<COMP>(S, cs, ex, 1.f);
 #pragma unroll
           for (int v = 0; v < VPT; ++v)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) P[v][k] += ex * e[v][k];
+            for (int k = 0; k < 8; ++k) add_comp<COMP>(P[v][k], cp[v][k], ex, e[v][k]);
         }
       }
       const float w = wt[i];
 #pragma unroll
       for (int v = 0; v < VPT; ++v)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc[v][k] += w * e[v][k];
+        for (int k = 0; k < 8; ++k) add_comp<COMP>(acc[v][k], ca[v][k], w, e[v][k]);
     };
     int i0 = 0;
     for (; i0 + PD <= n; i0 += PD) {
@@ -3005,11 +3048,21 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2))) void k_
     for (int j = 0; j < PD; ++j)
       if (i0 + j < n) one(i0 + j, buf[j]);
     if (online && !qz) {
-      const float f = M / S;
+      const float f = M / (COMP ? S - cs : S);
 #pragma unroll
       for (int v = 0; v < VPT; ++v)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc[v][k] += f * P[v][k];
+        for (int k = 0; k < 8; ++k)
+          acc[v][k] += COMP ? __builtin_fmaf(f, P[v][k], -__builtin_fmaf(f, cp[v][k], ca[v][k])) : f * P[v][k];
+    }
+    if (COMP) {   // the base joins the sums last
+      const bool fixed = !online || qz;
+      float bv[VPT][8];
+      load_base(bv);
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[v][k] = bv[v][k] + (fixed ? acc[v][k] - ca[v][k] : acc[v][k]);
     }
     if (valid) {
 #pragma unroll
@@ -3561,7 +3614,13 @@ int rows_read(const TAB& src, int64_t n, const float* q, float* dots, int64_t do
               float* next_prior, int64_t n_tok, int64_t d, int dtype, hipStream_t st) {
   int vpt, tpr, e = rows_layout(d, n, &vpt, &tpr);
   if (e) return e;
-  const size_t lds = sizeof(float) * (size_t)(3 * n * (1 + WG / tpr));
+  const auto bytes = [&]() -> int64_t {   // the rows' scalars; for wide fp32 rows the query too
+    const int64_t planes = 12 * n * (1 + WG / tpr);
+    return dtype == LDR_F32 && vpt >= 3 ? ((planes + 15) & ~(int64_t)15) + 32 * vpt * tpr : planes;
+  };
+  if (bytes() > 65536) e = rows_layout(d, 2 * n, &vpt, &tpr);   // half the rows per workgroup
+  if (e) return e;
+  const size_t lds = (size_t)bytes();
   const unsigned grid = grid_of(cdiv(n_tok, WG / tpr), 2048);   // no tokens: one workgroup writes next_prior
 #define LDR_ROWS_READ(BL)                                                                                            \
   LDR_DTYPE_SWITCH(dtype, LDR_VPT_SWITCH(vpt, hipLaunchKernelGGL((k_rows_read<T, VPT, BL, TAB>), dim3(grid),        \

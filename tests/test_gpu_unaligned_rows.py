@@ -47,3 +47,38 @@ def test_write_stores_the_scale_of_rstd(dtype, d):
         r = FD.rstd(v, stack.eps)
     torch.cuda.synchronize()
     assert torch.equal(v, h - x) and torch.equal(stack.R[0], r.view_as(stack.R[0]))
+
+
+def read_errors(d, n, t=300):
+    """The 2-norm errors from 64 bits of an fp32 read and of a model of it in fp32 torch operations that adds one
+    weight per source, each addition rounded once."""
+    from loopback_amd import fused_dattn as FD
+    g = torch.Generator().manual_seed(d + n)
+    base, q = torch.randn(1, t, d, generator=g), 0.3 * torch.randn(d, generator=g)
+    vs = [torch.randn(1, t, d, generator=g) for _ in range(n)]
+    c0 = torch.rand(n, generator=g) * 0.9 + 0.1
+    cbar = c0 + 0.2 * torch.randn(1, t, n, generator=g)
+    rs = [FD.rstd_ref(v, 1e-6) for v in vs]
+    dev = lambda ts: [x.to(DEV) for x in ts]
+    with torch.no_grad():
+        out, _ = FD.FusedDattnRead.apply(*dev((q, base, cbar, c0, *vs, *rs)))
+
+    def weights(dt):
+        z = torch.stack([(v.to(dt) @ q.to(dt)) * r.to(dt)[..., 0] for v, r in zip(vs, rs)], -1) / d ** 0.5
+        lc, c = c0.to(dt).log(), c0.to(dt)
+        return c + c.sum() * (torch.softmax(z + lc, -1) - torch.softmax(lc, -1)) - cbar.to(dt)
+
+    exact, model, w64, w32 = base.double(), base, weights(torch.float64), weights(torch.float32)
+    for i, v in enumerate(vs):
+        exact = exact + w64[..., i:i + 1] * v.double()
+        model = (model.double() + w32[..., i:i + 1].double() * v.double()).float()
+    return (out.cpu().double() - exact).norm().item(), (model.double() - exact).norm().item()
+
+
+@pytest.mark.parametrize("d,n", [(333, 2), (1001, 8), (1001, 24), (768, 72), (2049, 64), (4099, 12)])
+def test_read_error_of_one_weight_per_source(d, n):
+    """fp32 reads whose softmax is formed as the sources stream (their fixed and softmax shares summed apart) are no
+    further from 64 bits than one weight per source in fp32 (0.5 to 0.9 of it; without compensated sums 1.0 to 1.8)."""
+    got, model = read_errors(d, n)
+    print(f"case read error d{d} n{n}: {got:.3e}, one weight per source {model:.3e}, ratio {got / model:.3f}", flush=True)
+    assert got <= model
