@@ -39,6 +39,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import operator
 import os
 import weakref
 
@@ -528,9 +529,18 @@ class DattnStack:
                 self.QB = torch.empty(int(L.LIB.ldr_query_parts_elems(nq, d)), dtype=torch.bfloat16, device=device)
                 _run("split_queries", self.Q, nq, d, self.QB, _stream(self.Q.device))
 
+    def step(self, s) -> int:
+        """A step's index as an int: any integer type, a negative one from the end, as indexing V takes them (the
+        kernels get addresses computed from it)."""
+        s = operator.index(s)
+        if not -self.n_steps <= s < self.n_steps:
+            raise IndexError(f"delta_attnres stack: step {s} of {self.n_steps}")
+        return s + self.n_steps if s < 0 else s
+
     def write(self, s: int, h: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         """V[s] = h - x, returned as the update tensor (an alias of the stack's slice, with the autograd edge to
         h and x). The write also stores the update's scale R[s], which rstd(s, ...) then returns."""
+        s = self.step(s)
         v, r = _write(self, s, h, x) if _bypass() else _WriteDelta.apply(self, s, h, x)
         self.wout[s] = (weakref.ref(v), r)
         return v
@@ -538,6 +548,7 @@ class DattnStack:
     def rstd(self, s: int, delta: torch.Tensor, eps: float) -> torch.Tensor:
         """R[s] = the RMS scale of V[s], returned as an alias of the stack (differentiable through `delta`): the
         scale the write of `delta` stored with it, or computed here for another update or eps."""
+        s = self.step(s)
         w = self.wout.pop(s, None)
         if w is not None and w[0]() is delta and float(eps) == self.eps:
             return w[1]

@@ -229,3 +229,34 @@ def test_missing_library_fails_at_import():
                           capture_output=True, text=True, timeout=300)
     assert proc.returncode != 0
     assert "ImportError" in proc.stderr and "no fallback" in proc.stderr, proc.stderr[-2000:]
+
+
+def test_a_steps_index_is_normalized(monkeypatch):
+    """A stack's step may be any integer, a negative one counting from the end, as indexing takes them: the write's
+    score row is DOTS[query, step] whatever the step's type, and never outside the table."""
+    import numpy as np
+
+    class OnGpu(torch.Tensor):   # a CPU tensor that passes for a GPU one; nothing is launched
+        is_cuda = True
+
+    calls = []
+    monkeypatch.setattr(FD, "_run", lambda name, *args: calls.append((name, args)))
+    monkeypatch.setattr(FD, "_require_gpu", lambda t, what: None)
+    monkeypatch.setattr(FD, "_stream", lambda dev: 0)
+    n, tok, d = 4, 6, 16
+    stack = FD.DattnStack(n, (1, tok, d), torch.float32, "cpu", query=torch.zeros(n - 1, d))
+    h, x = (torch.randn(1, tok, d).as_subclass(OnGpu) for _ in range(2))
+    with torch.no_grad():
+        for s, want in ((0, 0), (n - 1, n - 1), (-1, n - 1), (-n, 0), (np.int64(2), 2), (torch.tensor(1), 1)):
+            calls.clear()
+            v = stack.write(s, h, x)
+            (name, args), = calls
+            j = max(0, want - 1)
+            assert name == "write_dots" and type(args[8]) is int and args[8] == stack.DOTS[j, want].data_ptr()
+            assert args[7] == j and v.data_ptr() == stack.V[want].data_ptr() and stack.r_done[want]
+            assert stack.rstd(want, v, stack.eps).data_ptr() == stack.R[want].data_ptr()
+    for s in (n, -n - 1):
+        with pytest.raises(IndexError):
+            stack.write(s, h, x)
+    with pytest.raises(TypeError):
+        stack.write(1.0, h, x)
