@@ -82,3 +82,17 @@ def test_read_error_of_one_weight_per_source(d, n):
     got, model = read_errors(d, n)
     print(f"case read error d{d} n{n}: {got:.3e}, one weight per source {model:.3e}, ratio {got / model:.3f}", flush=True)
     assert got <= model
+
+
+def test_infinite_base_element():
+    """An infinite element of the base stays infinite, and alone (the compensated sums do not see it)."""
+    from loopback_amd import fused_dattn as FD
+    g = torch.Generator().manual_seed(3)
+    base, q, cbar = torch.randn(1, 5, 333, generator=g), torch.randn(333, generator=g), torch.rand(1, 5, 6, generator=g)
+    base[0, 2, 331] = float("inf")
+    vs = [torch.randn(1, 5, 333, generator=g).to(DEV) for _ in range(6)]
+    rs = [FD.rstd(v, 1e-6) for v in vs]
+    with torch.no_grad():
+        out, _ = FD.FusedDattnRead.apply(q.to(DEV), base.to(DEV), cbar.to(DEV), torch.ones(6, device=DEV), *vs, *rs)
+    out = out.cpu()
+    assert out[0, 2, 331] == float("inf") and out.isfinite().sum() == out.numel() - 1
