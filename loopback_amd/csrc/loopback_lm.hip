@@ -181,6 +181,9 @@ __global__ __launch_bounds__(WG) void k_sum_rows(const float* __restrict__ part,
 // SwiGLU, bound by its rows (3 of n in and out forward, 5 backward). 16384 x 2048 bf16: forward 34-38 us (5.6 TB/s),
 // backward 52 us (6.5 TB/s); torch's silu, product, their gradients and the concatenation of the halves took ~290 us
 // ---------------------------------------------------------------------------------------------------------------
+// (the fast exponential: its error, some 2^-24 |x|, is far below the results' own rounding -- from 64 bits at N(0, 1) to
+// N(0, 256): forward 1.66e-3 to 1.65e-3 in bf16 and 2.1e-4 in fp16, to the sixth digit what the accurate one gives;
+// torch's two operations 1.67e-3 to 2.4e-3 and 2.1e-4 to 2.9e-4)
 __device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + __expf(-x)); }
 
 template <typename T>
@@ -223,6 +226,10 @@ __global__ __launch_bounds__(WG) void k_swiglu_bwd(const T* __restrict__ gu, con
 // vocabulary size), the last vocab mod 8 one per lane. A vocabulary of 32000 is 16 vectors per lane: the row's online
 // maximum and sum stay in registers, so a pass reads each logit once: 16384 x 32000 bf16 188 us forward (5.6 TB/s) and
 // 387 us backward (5.4 TB/s), against ~5.5 ms for an fp32 copy, torch's log-softmax and its gradient, and the casts.
+// Exponentials of differences from the maximum by the fast form: where its error (some 2^-24 of the difference) is large
+// the term is small. The loss lies as far from 64 bits as torch's fp32 form (1.8e-8 to 9e-8 of it over logits of
+// N(0, 0.25) to N(0, 400), vocabularies 4096 to 32000), its gradient to six digits where the accurate exponential puts
+// it; that one took 298 us forward.
 // ---------------------------------------------------------------------------------------------------------------
 // sum of exp(x - m) over a workgroup's lanes, each holding (m, s); every lane ends with the totals
 __device__ __forceinline__ void join_lse(float& m, float& s, float (&red)[2 * WAVES]) {

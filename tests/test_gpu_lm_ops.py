@@ -205,3 +205,27 @@ def test_dispatch_modes_see_torch_operations():
     x = rnd((2, 3, 64), torch.bfloat16, 33)
     for got, ref in zip(graph(x), fn(x)):
         assert (got.float() - ref.float()).norm() <= 2e-2 * ref.float().norm()
+
+
+@pytest.mark.parametrize("scale,vocab", [(0.5, 32000), (4.0, 32000), (20.0, 4096), (1.0, 33)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fast_exponential_costs_no_accuracy(scale, vocab, dtype):
+    """The loss, its gradient and SwiGLU with its gradient are no further from 64 bits than torch's fp32 forms: the loss
+    to an fp32 rounding (2^-24 of it), gradients to a ten-thousandth of the distance their 16-bit rounding leaves."""
+    from loopback_amd import lm_ops as ops
+    print(f"case fast exponential {scale} {vocab} {dtype}", flush=True)
+    ids = torch.randint(0, vocab, (2, 128), generator=torch.Generator().manual_seed(40)).to(DEV)
+    x, gu = scale * rnd((2, 128, vocab), dtype, 41), scale * rnd((256, 1024), dtype, 42)
+    da, err = rnd((256, 512), dtype, 43), lambda a, b: ((a.double() - b).norm() / b.norm()).item()
+
+    def run(loss, swiglu, cast):
+        a, b = cast(x.detach()).requires_grad_(), cast(gu.detach()).requires_grad_()
+        lo, act = loss(a), swiglu(b)
+        return [lo.detach(), torch.autograd.grad(lo, a)[0], act.detach(), torch.autograd.grad(act, b, cast(da))[0]]
+
+    exact = run(lambda a: F.cross_entropy(a[:, :-1].reshape(-1, vocab), ids[:, 1:].reshape(-1)), ops._swiglu_torch,
+                torch.Tensor.double)
+    got = run(lambda a: ops._NextTokenLoss.apply(a, ids), ops._SwiGLU.apply, lambda t: t)
+    ref = run(ops._loss_torch(ids), ops._swiglu_torch, lambda t: t)
+    for i, (a, b, e) in enumerate(zip(got, ref, exact)):
+        assert err(a, e) <= err(b, e) * (1 + 1e-4) + (2.0 ** -24 if i == 0 else 0.0), i
