@@ -129,8 +129,9 @@ def _rows(d: int, n: int) -> bool:
 
 
 def _refuse_capture() -> None:
-    """Shapes outside the row layout are not captured in a HIP graph: a replay of the any-shape path would copy its
-    address arrays from a host buffer torch may since have reused."""
+    """Address tables for shapes outside the row layout are not made under HIP graph capture: a replay would copy the
+    any-shape path's device arrays from a host buffer torch may since have reused. The unaligned-row path, whose
+    addresses go by value, is refused with it, so that what can be captured does not depend on the source count."""
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("delta_attnres HIP read: shapes the row-layout kernels do not take (d not a multiple of 8 "
                            "or above 8192, more than 64 sources, unaligned rows) cannot be captured in a HIP graph")
@@ -473,7 +474,7 @@ class DattnStack:
     matrix-core product loads them."""
     __slots__ = ("V", "R", "dV", "dR", "n_steps", "n_tok", "d", "eps", "Q", "QT", "QB", "DOTS", "r_done", "WZ", "bwd",
                  "assembled", "neg", "dq_parts", "dq_rows", "wh", "gadd", "h0_ref", "h0_steps", "h0_g", "vptr",
-                 "rptr", "drptr", "wout", "fast_d", "src_fast", "src_any", "per_read")
+                 "rptr", "drptr", "wout", "fast_d", "src_fast", "src_rows", "src_any", "per_read")
 
     def __init__(self, n_steps: int, shape, dtype, device, query=None, eps: float = 1e-6):
         b, t, d = shape
@@ -487,7 +488,7 @@ class DattnStack:
         # rows the row-layout kernels take (the slices of V are then 16-byte aligned); other widths, and reads of
         # more than MAX_SOURCES sources, run on the any-shape kernels
         self.fast_d = d % 8 == 0 and d <= L.MAX_WIDTH
-        self.src_fast = self.src_any = None
+        self.src_fast = self.src_rows = self.src_any = None
         # the updates' gradients: one fp32 sum rounded once (default), or rounded per read as the list layout's
         # per-read gradients are when autograd adds them (LOOP_DATTN_GRAD_ROUNDING=per_read: bitwise the list layout)
         self.per_read = grad_rounding() == "per_read"
@@ -563,14 +564,14 @@ class DattnStack:
             if self.src_fast is None or (self.src_fast.dr is None and self.drptr is not None):
                 self.src_fast = _Src(True, False, self.vptr, self.rptr, self.drptr)
             return self.src_fast
-        _refuse_capture()
-        if _rows(self.d, n):
-            return _Src(False, True, self.vptr, self.rptr, self.drptr)
         if self.src_any is None or (self.src_any.dr is None and self.dR is not None):
-            dev = self.V.device
-            self.src_any = _Src(False, False, _dev_addrs(self.vptr, dev), _dev_addrs(self.rptr, dev),
-                                None if self.dR is None else _dev_addrs(self.drptr, dev))
-        return self.src_any
+            _refuse_capture()             # reads over tables made before the capture are captured
+            self.src_any = self.src_rows = _Src(False, True, self.vptr, self.rptr, self.drptr)
+            if not _rows(self.d, self.n_steps):
+                dev = self.V.device
+                self.src_any = _Src(False, False, _dev_addrs(self.vptr, dev), _dev_addrs(self.rptr, dev),
+                                    None if self.dR is None else _dev_addrs(self.drptr, dev))
+        return self.src_rows if _rows(self.d, n) else self.src_any
 
     def grads(self):
         """Allocate the backward state on the first backward of the pass; False then, True afterwards."""
@@ -640,7 +641,8 @@ def _assemble(stack: DattnStack, s: int, gr):
     if fast:
         _run("dv_assemble", *tables, *args)
     elif _rows(stack.d, m):
-        _refuse_capture()
+        if reads:
+            _refuse_capture()
         _run("dv_assemble_rows", *tables, *args)
     else:
         dev_tabs = [_dev_addrs(t, v.device) for t in tables] if reads else None

@@ -231,6 +231,32 @@ def test_missing_library_fails_at_import():
     assert "ImportError" in proc.stderr and "no fallback" in proc.stderr, proc.stderr[-2000:]
 
 
+@pytest.mark.parametrize("n_steps", [4, 70])
+def test_capture_takes_tables_made_before_it(monkeypatch, n_steps):
+    """Under graph capture a stack of a width outside the row layout refuses to make its address tables, and reads over
+    tables it already made; a gradient that no read takes part in needs none."""
+    monkeypatch.setattr(FD, "_require_gpu", lambda t, what: None)
+    monkeypatch.setattr(FD, "_stream", lambda dev: 0)
+    monkeypatch.setattr(FD, "_run", lambda name, *args: None)
+    capturing = [True]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(FD, "_dev_addrs", lambda a, dev: FD._refuse_capture() or torch.tensor(list(a)))
+    stack = FD.DattnStack(n_steps, (1, 6, 13), torch.float32, "cpu")
+    with pytest.raises(RuntimeError, match="HIP graph"):
+        stack.src(2)
+    capturing[0] = False
+    first = stack.src(2)
+    capturing[0] = True
+    assert first.rows and stack.src(3) is first and stack.src(n_steps).rows == (n_steps <= 64)
+    stack.grads()                                # the scale gradients' addresses join: the tables are made again
+    with pytest.raises(RuntimeError, match="HIP graph"):
+        stack.src(2)
+    FD._assemble(stack, 1, None)                 # no read of update 1 ran its backward
+    stack.keep(2, torch.zeros(1, 6, 13), torch.zeros(13))
+    with pytest.raises(RuntimeError, match="HIP graph"):
+        FD._assemble(stack, 1, None)
+
+
 def test_a_steps_index_is_normalized(monkeypatch):
     """A stack's step may be any integer, a negative one counting from the end, as indexing takes them: the write's
     score row is DOTS[query, step] whatever the step's type, and never outside the table."""
