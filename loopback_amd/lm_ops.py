@@ -335,10 +335,11 @@ def rotary_attention(qkv, cos, sin, heads, again):
 # ---------------------------------------------------------------------------------------------------------------
 # bias-free linear layers, their weight gradient by llm_wgrad
 # ---------------------------------------------------------------------------------------------------------------
-# Where the split reduction is the faster one (16384 tokens, weights 256 x 256 to 4096 x 768: 1.2 to 3.2 times the library;
-# 8192 tokens: 1.2; 4096 tokens and fewer: 0.6 to 1.1, the library's), and enough runs of tokens fill the GPU (with two
-# runs, 5632 x 1024: 0.84).
-WGRAD_MIN_TOKENS, WGRAD_MIN_SPLITS = 8192, 4
+# Where the split reduction is the faster one, library's time over the kernels': 8192 to 65536 tokens, weights 64 x 64 to
+# 4096 x 768 and up to 2056 x 1032: 1.08 to 5.9 (the smallest too, though their tile is mostly padding: the library runs a
+# few workgroups). A side of 8 or 16: 0.94 to 1.06 up to 16384 tokens. Four runs of tokens (2048 x 2048, 4096 x 1024): 0.95
+# to 1.16; two (5632 x 1024): 0.84. 4096 tokens and fewer: 0.6 to 1.1. The library's then.
+WGRAD_MIN_TOKENS, WGRAD_MIN_SPLITS, WGRAD_MIN_SIDE = 8192, 5, 64
 
 
 def wgrad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
@@ -370,7 +371,7 @@ def linear_native(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether linear(x, w) records a weight gradient by llm_wgrad."""
     return (torch.is_grad_enabled() and x.dtype is torch.bfloat16 and native(x, w) and w.requires_grad and x.dim() > 1
             and w.dim() == 2 and x.shape[-1] == w.shape[1] and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1]
-            and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and _rows_ok(x, w)
+            and min(w.shape) >= WGRAD_MIN_SIDE and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and _rows_ok(x, w)
             and LIB.llm_wgrad_splits(x.numel() // w.shape[1], *w.shape) >= WGRAD_MIN_SPLITS)
 
 

@@ -152,3 +152,18 @@ def test_block_gradients_with_a_graph():
     got = torch.autograd.grad(block(x), params, g, create_graph=True)
     for p, q in zip(got, ref):
         assert (p - q).float().norm() <= 2e-2 * q.float().norm()
+
+
+def test_weight_gradient_rule(monkeypatch):
+    """Which linear layers record the split-token weight gradient: from 64 x 64 weights and 8192 tokens on, with at
+    least five runs of tokens."""
+    monkeypatch.setattr(ops, "native", lambda *ts: True)
+
+    def takes(tokens, n, k):
+        w = torch.empty(n, k, dtype=torch.bfloat16, requires_grad=True)
+        return ops.linear_native(torch.empty(1, dtype=torch.bfloat16).expand(tokens, k), w)
+
+    monkeypatch.setattr(ops, "_rows_ok", lambda *ts: True)
+    assert [takes(*s) for s in ((8192, 64, 64), (8192, 4096, 768), (65536, 72, 2048), (12000, 3072, 1024))] == [True] * 4
+    assert [takes(*s) for s in ((8191, 64, 64), (16384, 56, 512), (16384, 512, 16), (8192, 2048, 2048),
+                                (8192, 4096, 1024), (16384, 5632, 1024), (16384, 68, 64))] == [False] * 7
