@@ -29,7 +29,12 @@ FAMILIES = [("k_read_fwd", "read_fwd"), ("k_read_online", "read_fwd_online"), ("
             # the unaligned-row kernels (their read runs with and without stored scores)
             ("k_write_any", "write_rows"), ("k_rows_read", "read_fwd_rows"), ("k_rows_bwd1", "read_bwd1_rows"),
             ("k_rows_dv_assemble", "dv_assemble_rows"), ("k_rows_bwd2_list", "read_bwd2_list_rows"),
-            ("k_flat_blend_sum", "blend_sum_rows")]
+            ("k_flat_blend_sum", "blend_sum_rows"),
+            # the language model's kernels
+            ("k_rms_norm_fwd", "rms_norm_fwd"), ("k_rms_norm_bwd", "rms_norm_bwd"), ("k_sum_rows", "sum_rows"),
+            ("k_swiglu_fwd", "swiglu_fwd"), ("k_swiglu_bwd", "swiglu_bwd"), ("k_next_token_fwd", "next_token_loss_fwd"),
+            ("k_mean", "next_token_loss_fwd"), ("k_next_token_bwd", "next_token_loss_bwd"), ("k_rotary", "rotary"),
+            ("k_attn_fwd", "attn_fwd"), ("k_attn_bwd", "attn_bwd"), ("k_wgrad", "wgrad")]
 COPY_BYTES = 1 << 30   # bench.py --copy-calibration copies 1 GiB
 
 

@@ -153,3 +153,19 @@ def test_compare_pass_timelines(tmp_path):
     RS.main(["--config", "c3", "--compare", str(kt1), str(kt2), "--name", "cmp", "--out", str(out)])
     text = (out / "cmp.md").read_text()
     assert "| eager | 8 |" in text and "| graph replay | 8 |" in text
+
+
+def test_every_kernel_has_a_family():
+    """Each kernel of the two libraries' sources is counted as this library's (k_zero apart, which no chain or model
+    launches), and torch's are not."""
+    import re
+    names = set()
+    for src in ("loopback_read.hip", "loopback_lm.hip"):
+        with open(os.path.join(os.path.dirname(RS.__file__), "csrc", src)) as f:
+            names |= set(re.findall(r"__global__[^;{]*?\bvoid\s+(k_\w+)\s*\(", f.read(), flags=re.S))
+    assert {"k_read_fwd", "k_bwd1", "k_wgrad_sum", "k_attn_bwd_kv", "k_rms_norm_bwd", "k_next_token_fwd"} <= names
+    missed = {n for n in names if RS.family(f"void (anonymous namespace)::{n}<float, 1>(...)") == "torch / runtime"}
+    assert missed <= {"k_zero", "k_any_read", "k_any_bwd1", "k_any_dv_assemble", "k_any_bwd2_list"}, missed
+    for name in ("at::native::vectorized_elementwise_kernel<8, CUDAFunctor_add>", "Cijk_Ailk_Bljk_BBS_BH", "attn_fwd",
+                 "void at::native::reduce_kernel<512, 1, at::native::MeanOps>"):
+        assert RS.family(name) == "torch / runtime"
