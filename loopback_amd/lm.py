@@ -157,9 +157,11 @@ class Attention(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         qkv = linear(self.qkv, x)
-        if ops.attention_native(qkv, self.dh) and type(self.rotary) is Rotary and not _hooked(self.rotary):
-            cos, sin = self.rotary.tables(x.shape[1], x.device, qkv.dtype)
-            return linear(self.o, ops.rotary_attention(qkv, cos, sin, self.h, self.attend))
+        if (ops.attention_native(qkv, self.dh) and type(self.rotary) is Rotary and not _hooked(self.rotary)
+                and "tables" not in self.rotary.__dict__):
+            cos, sin = self.rotary.tables(qkv.shape[1], qkv.device, qkv.dtype)
+            if ops.tables_native(qkv, cos, sin, self.h):
+                return linear(self.o, ops.rotary_attention(qkv, cos, sin, self.h, self.attend))
         return linear(self.o, self.attend(qkv))
 
     def attend(self, qkv: torch.Tensor) -> torch.Tensor:

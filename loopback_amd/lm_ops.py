@@ -327,6 +327,13 @@ def attention_native(qkv: torch.Tensor, head_dim: int) -> bool:
             and qkv.shape[1] <= ATTN_MAX and qkv.shape[0] * qkv.shape[2] <= 192 * ATTN_MAX and _rows_ok(qkv))
 
 
+def tables_native(qkv, cos, sin, heads: int) -> bool:
+    """Whether the operands have the sizes the kernels index by: qkv's width that of the heads, cos and sin (t, 64)."""
+    return qkv.shape[2] == 192 * heads and all(
+        type(x) is torch.Tensor and x.dtype is torch.float32 and x.device == qkv.device
+        and x.shape == (qkv.shape[1], 64) and _rows_ok(x) for x in (cos, sin))
+
+
 def rotary_attention(qkv, cos, sin, heads, again):
     """Causal attention over the rotated q and k of qkv; cos and sin (t, 64) fp32, contiguous, both halves alike."""
     return _RotaryAttention.apply(qkv, cos, sin, heads, again)

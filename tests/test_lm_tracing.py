@@ -91,3 +91,27 @@ def test_a_hooked_linear_layer_is_called(monkeypatch):
             layer.register_forward_hook(lambda m, i, o: seen.append(1))
         assert torch.equal(lm.linear(layer, x), layer.forward(x))
         assert len(seen) == calls and bool(taken) == (not hooked and not bias)
+
+
+def test_attention_operands_are_checked(monkeypatch):
+    """A projection whose width is not the heads' is refused, as the torch form refuses its view, and tables the kernels
+    do not index (another width, type or order of halves) go to the torch form."""
+    taken = []
+    monkeypatch.setattr(lm.ops, "attention_native", lambda qkv, dh: True)
+    monkeypatch.setattr(lm.ops, "rotary_attention", lambda qkv, cos, sin, h, again: taken.append(1) or again(qkv))
+    x = torch.randn(1, 5, 128)
+    attn = lm.Attention(CFG)
+    y = attn(x)
+    assert taken == [1]
+    attn.qkv = torch.nn.Linear(128, 2 * 128, bias=False)
+    with pytest.raises(RuntimeError, match="shape"):
+        attn(x)
+    attn = lm.Attention(CFG)
+    cos, sin = attn.rotary.tables(5, x.device, x.dtype)
+    attn.rotary.tables = lambda *a: (cos.flip(-1), sin)
+    taken.clear()
+    assert attn(x).shape == y.shape and not taken
+    ok = lambda c, s, heads=2, width=384: lm.ops.tables_native(torch.empty(1, 5, width), c, s, heads)
+    assert ok(cos, sin)
+    assert not any((ok(cos, sin, 3), ok(cos, sin, 2, 256), ok(cos.double(), sin), ok(cos, sin[:4]), ok(cos[:, :32], sin),
+                    ok(cos, sin.t().contiguous().t())))
