@@ -1,7 +1,8 @@
 /*
  * loopback_lm.h -- C ABI of libloopback_lm.so: the MI355X (gfx950) kernels of the language model around the Loopback
  * read (loopback_amd/lm.py) -- RMSNorm, SwiGLU and the next-token cross entropy, forward and backward, each one pass
- * over its rows. The reference leaves these to torch (looped_transformer.py:5-33, 431-615).
+ * over its rows; causal rotary attention in bf16 at head width 64, forward and backward; and the weight gradients of
+ * bias-free linear layers in bf16. The reference leaves these to torch (looped_transformer.py:5-33, 431-615).
  *
  * Conventions: device pointers to contiguous row-major tensors; dtype is LDR_BF16 or LDR_F16 (loopback_read.h) for
  * the rows and weights, every statistic and partial sum is fp32, results are rounded once from fp32; stream is a

@@ -66,7 +66,7 @@ int64_t ldr_read_bwd1_parts(int64_t n_tok, int64_t d);
 /* r[tok] = rsqrt(sum_k x[tok,k]^2 / d + eps).
  * Replaces _rstd_fwd_kernel and its launches (fused_dattn.py:206-215, 240, 705). Any d >= 1 and any alignment, as
  * the reference's masked kernel: rows the vector layout does not take (d not a multiple of 8 or above
- * LDR_MAX_WIDTH, x not 16-byte aligned) run on scalar loads. */
+ * LDR_MAX_WIDTH, x not 16-byte aligned) load their eight-element vectors at element alignment (d < 8: one by one). */
 int ldr_rstd_fwd(const void* x, float* r, int64_t n_tok, int64_t d, float eps, int dtype, void* stream);
 
 /* gx[tok,:] = gr[tok] * (-r[tok]^3) / d * x[tok,:], rounded to dtype.
@@ -149,6 +149,8 @@ int ldr_read_fwd_online(const uint64_t* src_v, const uint64_t* src_r, int64_t n,
  *     [p][read][d] and one ldr_reduce_rows over rows of k d sums them all)
  *   with g_prop and / or g_h0 (each may be NULL): the iteration-end blend's gradients g_h0 = round(beta g),
  *     g_prop = round(g - g_h0), rounded as autograd rounds them
+ * Its workgroups take 32-token tiles; ldr_read_bwd1_rows, given as many partial rows as ldr_read_bwd1_rows_parts says,
+ * runs the same kernel on smaller ones where the tokens are too few to reach every CU.
  * Replaces _dattn_bwd1_stk_kernel (fused_dattn.py:459-493, launched at 777-779) and pass 1 of _dattn_bwd_kernel
  * (111-151); dr is also the dR update of _dattn_bwd2_stk_kernel (532-535). */
 int ldr_read_bwd1(const uint64_t* src_v, const uint64_t* src_r, int64_t n, const void* g, const float* gt,

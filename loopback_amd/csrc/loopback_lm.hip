@@ -1,8 +1,11 @@
-// loopback_lm.hip -- MI355X (gfx950, CDNA4) kernels of the language model around the Loopback read: RMSNorm, SwiGLU
-// and the next-token cross entropy, forward and backward. All are bound by the HBM stream of their rows, and torch's
-// composed forms move those rows several times (an fp32 copy of the logits, the softmax, its gradient and its cast;
-// silu and the product; the norm's gradient, its weight's gradient and the residual's add): each is one pass here,
-// with fp32 statistics and one rounding per result. Every sum has a fixed order: results are deterministic.
+// loopback_lm.hip -- MI355X (gfx950, CDNA4) kernels of the language model around the Loopback read, in three kinds:
+//   * RMSNorm, SwiGLU and the next-token cross entropy, forward and backward, bound by the HBM stream of their rows.
+//     torch's composed forms move those rows several times (an fp32 copy of the logits, the softmax, its gradient and its
+//     cast; silu and the product; the norm's gradient, its weight's gradient and the residual's add): each is one pass
+//     here, with fp32 statistics and one rounding per result;
+//   * causal rotary attention in bf16, forward and backward, on the matrix cores, bound by the vector units (the softmax);
+//   * weight gradients of the linear layers on the matrix cores, the tokens split over the CUs, bound by LDS reads.
+// Every sum has a fixed order: results are deterministic.
 
 #include <hip/hip_runtime.h>
 #include <math.h>

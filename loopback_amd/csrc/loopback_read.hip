@@ -474,7 +474,7 @@ __global__ __launch_bounds__(WG) void k_rstd_bwd(const T* __restrict__ x, const 
 // instruction) and backward pass 1 ran one wave on each of n_tok / 64 partial rows. A 12-step training pass of 2049
 // tokens at d = 1001 in bf16: 31.8 -> 2.06 ms (the host's launch rate; 1.04 ms of kernels), per launch backward
 // pass 1 2690 -> 22.6 us (7 sources on average), the read 70-79 -> 23-26, the update gradient 44.6 -> 24.1. A read of
-// 65-72 sources of 4096 x 768 bf16: 746 -> 94 us (4.7 TB/s; 138 with two vectors on each of 64 lanes, a quarter of them
+// 65-72 sources of 4096 x 768 bf16: 746 -> 94 us (4.7 TB/s; 142 with two vectors on each of 64 lanes, a quarter of them
 // idle, where three on 32 lanes put two rows in a wave).
 // ---------------------------------------------------------------------------------------------------------------
 // Row geometry at any width d >= 8: vector c of a row covers elements [8c, 8c + 8), the last one [d - 8, d).
@@ -3753,7 +3753,7 @@ int ldr_rstd_fwd(const void* x, float* r, int64_t n_tok, int64_t d, float eps, i
   if (n_tok == 0) return LDR_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   int vpt, tpr;
-  if (!al16(x) || row_layout(d, &vpt, &tpr) != LDR_OK) {   // any other row: scalar loads
+  if (!al16(x) || row_layout(d, &vpt, &tpr) != LDR_OK) {   // any other row: eight-element vectors at element alignment
     const unsigned grid = grid_of(cdiv(n_tok, WG / 64), 8192);
     LDR_DTYPE_SWITCH(dtype, hipLaunchKernelGGL((k_rstd_fwd_any<T>), dim3(grid), dim3(WG), 0, st,
                                                 static_cast<const T*>(x), r, n_tok, d, eps))
