@@ -57,23 +57,31 @@ def _load() -> ctypes.CDLL:
 
 
 LIB = _load()
+_FN = {name: getattr(LIB, name) for name in SIGNATURES}
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _run(name: str, *args) -> None:
-    code = getattr(LIB, name)(*args)
+    code = _FN[name](*args)
     if code:
         raise RuntimeError(f"{name}: refused or failed to launch (code {code})")
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    return _raw_stream(t.device.index)
+
+
+_Tensor, _Parameter = torch.Tensor, torch.nn.Parameter   # bound once: these run a few times per layer and pass
+_compiling, _tracing, _grad_on = torch.compiler.is_compiling, torch._C._is_tracing, torch.is_grad_enabled
+_modes, _transform = torch._C._len_torch_dispatch_stack, torch._C._functorch.peek_interpreter_stack
+_batched = torch._C._functorch.is_legacy_batchedtensor
 
 
 def _watched() -> bool:
     """Whether something is on that has to see torch operations: torch.compile, jit tracing, a torch.func transform,
     forward-mode AD, a dispatch mode."""
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None)
+    return (_compiling() or _tracing() or forward_ad._current_level >= 0 or _modes() > 0
+            or _transform() is not None)
 
 
 def native(*tensors) -> bool:
@@ -83,11 +91,11 @@ def native(*tensors) -> bool:
         return False
     first = tensors[0]
     for t in tensors:
-        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+        if type(t) is not _Tensor and type(t) is not _Parameter:
             return False
     if not first.is_cuda or first.dtype not in _CODES or first.device.index != torch._C._cuda_getDevice():
         return False
-    for t in tensors:
+    for t in tensors[1:]:
         if t.dtype is not first.dtype or t.device != first.device:
             return False
     return not torch.is_autocast_enabled("cuda")
@@ -96,11 +104,10 @@ def native(*tensors) -> bool:
 def _launchable(*grads) -> bool:
     """Whether a backward runs on the kernels: it is not itself differentiated, nothing watches it, and its gradients
     are plain tensors (not the batched ones of is_grads_batched and jacobian(vectorize=True))."""
-    if torch.is_grad_enabled() or _watched():
+    if _grad_on() or _watched():
         return False
     for g in grads:
-        if g is not None and ((type(g) is not torch.Tensor and type(g) is not torch.nn.Parameter)
-                              or torch._C._functorch.is_legacy_batchedtensor(g)):
+        if g is not None and ((type(g) is not _Tensor and type(g) is not _Parameter) or _batched(g)):
             return False
     return True
 
@@ -152,7 +159,8 @@ class _AddRmsNorm(torch.autograd.Function):
         h, w, rstd = _saved(ctx)
         if dy is None:
             return dh, dh if ctx.added else None, None, None
-        needed = [ctx.needs_input_grad[0] or ctx.needs_input_grad[1], ctx.needs_input_grad[2]]
+        need = ctx.needs_input_grad
+        needed = need[0] or need[1], need[2]
         if not _launchable(dh, dy):
             dx, dw = _again(lambda h, w: F.rms_norm(h, (h.shape[-1],), w, ctx.eps), [h, w], needed, dy)
             dx = dx if dx is None or dh is None else dx + dh
@@ -167,9 +175,9 @@ class _AddRmsNorm(torch.autograd.Function):
             parts = LIB.llm_rms_norm_parts(rows)
             part = torch.empty((parts, d), device=h.device, dtype=torch.float32)
             dw = torch.empty_like(w)
-        ptr = lambda t: None if t is None else t.data_ptr()
-        _run("llm_rms_norm_bwd", dy.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(), ptr(dres), ptr(dx),
-             ptr(part), rows, d, _CODES[h.dtype], _stream(h))
+        _run("llm_rms_norm_bwd", dy.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(),
+             None if dres is None else dres.data_ptr(), None if dx is None else dx.data_ptr(),
+             None if part is None else part.data_ptr(), rows, d, _CODES[h.dtype], _stream(h))
         if needed[1]:
             _run("llm_sum_rows", part.data_ptr(), parts, d, dw.data_ptr(), _CODES[w.dtype], _stream(h))
         return dx, dx if ctx.added else None, dw, None
@@ -182,7 +190,10 @@ def _dense(g, like):
 
 
 def _rows_ok(*tensors) -> bool:
-    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+    for t in tensors:
+        if not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+    return True
 
 
 def norm_native(x, w, add=None, eps=0.0) -> bool:
@@ -376,9 +387,10 @@ class _Linear(torch.autograd.Function):
 
 def linear_native(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether linear(x, w) records a weight gradient by llm_wgrad."""
-    return (torch.is_grad_enabled() and x.dtype is torch.bfloat16 and native(x, w) and w.requires_grad and x.dim() > 1
-            and w.dim() == 2 and x.shape[-1] == w.shape[1] and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1]
-            and min(w.shape) >= WGRAD_MIN_SIDE and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and _rows_ok(x, w)
+    return (torch.is_grad_enabled() and x.dtype is torch.bfloat16 and not _compiling()
+            and w.requires_grad and x.dim() > 1 and w.dim() == 2 and x.shape[-1] == w.shape[1]
+            and x.numel() >= WGRAD_MIN_TOKENS * w.shape[1] and min(w.shape) >= WGRAD_MIN_SIDE and w.shape[0] % 8 == 0
+            and w.shape[1] % 8 == 0 and native(x, w) and _rows_ok(x, w)
             and LIB.llm_wgrad_splits(x.numel() // w.shape[1], *w.shape) >= WGRAD_MIN_SPLITS)
 
 
