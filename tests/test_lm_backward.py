@@ -106,6 +106,36 @@ def test_watched_backwards(no_launch, monkeypatch, name, how):
     assert torch.allclose(grads(y), grads(yr), rtol=1e-2, atol=1e-3)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["batched", "vmap", "mode", "plain"])
+def test_watched_backwards_on_the_gpu(how):
+    """The same through the engine's GPU thread, the forward by the kernels: torch's gradients, to a few roundings of
+    bf16 (both round each result once, torch some intermediate ones too)."""
+    print(f"case watched backward {how}", flush=True)
+    dev = lambda *ts: [t.cuda() for t in ts]
+    w, u, ids = dev(rnd((64,), 2), rnd((32, 64), 5), torch.arange(6).view(2, 3))
+    for fn, ref_fn, shape in ((lambda x: ops.add_rms_norm(x, None, w, 1e-6)[1], lambda x: F.rms_norm(x, (64,), w, 1e-6), (5, 64)),
+                              (ops._SwiGLU.apply, ops._swiglu_torch, (5, 64)),
+                              (lambda x: ops._NextTokenLoss.apply(x, ids), ops._loss_torch(ids), (2, 3, 64)),
+                              (lambda x: ops._Linear.apply(x, u), lambda x: F.linear(x, u), (5, 64))):
+        x = rnd(shape, 1).cuda().requires_grad_()
+
+        def grads(out):
+            gs = torch.stack([rnd(out.shape, k, out.dtype) for k in (7, 8)]).cuda()
+            if how == "batched":
+                return torch.autograd.grad(out, x, gs, is_grads_batched=True)[0]
+            if how == "vmap":
+                return torch.func.vmap(lambda g: torch.autograd.grad(out, x, g, retain_graph=True)[0])(gs)
+            if how == "plain":
+                return torch.autograd.grad(out, x, gs[0])[0]
+            from torch.utils.flop_counter import FlopCounterMode
+            with FlopCounterMode(display=False):
+                return torch.autograd.grad(out, x, gs[0])[0]
+
+        got, ref = grads(fn(x)), grads(ref_fn(x))
+        assert (got - ref).float().norm() <= 2e-2 * ref.float().norm()
+
+
 def test_saved_tensors_with_other_strides():
     """What a saved-tensor hook gives back strided or unaligned reaches the kernels as contiguous aligned rows."""
     ctx = type("ctx", (), {})()
