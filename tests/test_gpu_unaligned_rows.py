@@ -96,3 +96,12 @@ def test_infinite_base_element():
         out, _ = FD.FusedDattnRead.apply(q.to(DEV), base.to(DEV), cbar.to(DEV), torch.ones(6, device=DEV), *vs, *rs)
     out = out.cpu()
     assert out[0, 2, 331] == float("inf") and out.isfinite().sum() == out.numel() - 1
+
+
+@pytest.mark.parametrize("d,n", [(2000, 900), (2000, 1000), (1500, 1024), (8192, 1024)])
+def test_many_sources_of_wide_fp32_rows(d, n):
+    """The query and a workgroup's per-source scalars in LDS at its bound (62192 bytes), and past it with half the rows
+    per workgroup: the read of one weight per source."""
+    got, model = read_errors(d, n, 5)
+    print(f"case wide rows d{d} n{n}: {got:.3e}, one weight per source {model:.3e}", flush=True)
+    assert got <= model
